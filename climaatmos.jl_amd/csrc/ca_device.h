@@ -67,6 +67,7 @@ struct DevNum {
     double dR_d, dcp_d, dcv_d, dT_0, dp0inv, dkex, dTsr, dTmr, dTmin;
     double dicv_d;  // 1 / cv_d
     double dkex_r;  // kex - 2/7 (|.| <= 1e-6, checked at create)
+    float kex7r;    // 7 (kex - 2/7)
     float nu_v, nu_s, dd;
     float alpha_uh, alpha_w, dt;
     float Cd, Ch, gust;  // surface flux exchange coefficients and wind-speed floor
@@ -153,24 +154,69 @@ __device__ __forceinline__ float ca_pow7(float x) {
     return x4 * x2 * x;
 }
 __device__ __forceinline__ float ca_Tref(const DevNum &n, float Pi) { return n.Tmr + (n.Tsr - n.Tmr) * ca_pow7(Pi); }
-// Phi_r(p_b) - Phi_r(p_a) in a cancellation-free form:
-//   -cp_d [T_min ln(Pi_b / Pi_a) + (T_sfc - T_min) / 7 (Pi_b^7 - Pi_a^7)]
-// with ln(Pi_b / Pi_a) = kex ln(p_b / p_a) and Pi_b^7 - Pi_a^7 = Pi_a^7 expm1(7 ln(Pi_b / Pi_a)).
+// Phi_r(p_b) - Phi_r(p_a) in a cancellation-free form, with x = (p_b - p_a) / p_a:
+//   -cp_d [T_min ln(Pi_b / Pi_a) + (T_sfc - T_min) / 7 (Pi_b^7 - Pi_a^7)],
+//   ln(Pi_b / Pi_a) = kex log1p(x),  Pi_b^7 - Pi_a^7 = Pi_a^7 ((1 + x)^(7 kex) - 1).
+// 7 kex is 2 up to 7 kex_r (|7 kex_r| <= 7e-6, checked at create), so the last
+// factor is x (2 + x) + (1 + x)^2 7 kex_r log1p(x) to below 1e-9 of its size.
+// The neighbours of one element's level differ by a few per cent in pressure:
+// log1p and expm1 take short series for |x| <= 1/4 and a longer form otherwise,
+// chosen per wavefront (a NaN takes the longer form and stays one).  The library
+// functions they replace were a third of k_laplacians' VALU instructions
+// (327 -> 212 per level; 52 -> 42.5 us per launch at h_elem 30, 63 levels) and a fifth of k_explicit's, and both kernels are bound by VALU
+// issue (85% and 66% busy).
+__device__ __forceinline__ bool ca_small(float x) { return __all(fabsf(x) <= 0.25f); }
+// log1p(x).  Small: 2 atanh(s), s = x / (2 + x), by its odd series to s^9 (|s| <=
+// 1/7: truncated below 1e-9).  Otherwise log(u) + (x - (u - 1)) / u with u the
+// rounded 1 + x: |log(u)| > 0.2, where the hardware log2's error is one unit.
+__device__ __forceinline__ float ca_log1p(float x, bool small) {
+    if (small) {
+        const float s = x * ca_rcp(2.0f + x), s2 = s * s;
+        const float z = fmaf(s2, fmaf(s2, fmaf(s2, fmaf(s2, 1.0f / 9.0f, 1.0f / 7.0f), 0.2f), 1.0f / 3.0f), 1.0f);
+        return 2.0f * s * z;
+    }
+    const float u = 1.0f + x;
+    return fmaf(__builtin_amdgcn_logf(u), 0.693147182f, (x - (u - 1.0f)) * ca_rcp(u));
+}
+// expm1(r), r = kex log1p(x).  Small (|r| <= 0.083): Taylor to r^6, truncated below
+// 1e-10.  Otherwise (1 + t)^4 - 1 with t = expm1(r / 4) by Taylor to its eighth
+// power for |r| <= 1.4, and exp(r) - 1 beyond, where it loses no digits.
+__device__ __forceinline__ float ca_expm1(float r, bool small) {
+    if (small)
+        return r * fmaf(r, fmaf(r, fmaf(r, fmaf(r, fmaf(r, 1.0f / 720.0f, 1.0f / 120.0f), 1.0f / 24.0f), 1.0f / 6.0f),
+                                0.5f),
+                        1.0f);
+    const float q = 0.25f * r;
+    float t = 1.0f / 40320.0f;
+    t = fmaf(t, q, 1.0f / 5040.0f);
+    t = fmaf(t, q, 1.0f / 720.0f);
+    t = fmaf(t, q, 1.0f / 120.0f);
+    t = fmaf(t, q, 1.0f / 24.0f);
+    t = fmaf(t, q, 1.0f / 6.0f);
+    t = fmaf(t, q, 0.5f);
+    t = q * fmaf(t, q, 1.0f);
+    const float e = t * fmaf(t, fmaf(t, 4.0f + t, 6.0f), 4.0f);
+    return fabsf(r) <= 1.4f ? e : __builtin_amdgcn_exp2f(1.44269504f * r) - 1.0f;
+}
+// (1 + x)^(7 kex) - 1, l = log1p(x)
+__device__ __forceinline__ float ca_pow2m1(const DevNum &n, float x, float l) {
+    const float y = 1.0f + x;
+    return fmaf(y * y, n.kex7r * l, x * (2.0f + x));
+}
 // ipa = 1 / pa
 __device__ __forceinline__ float ca_dPhiref(const DevNum &n, float pa, float ipa, float Pia, float pb) {
-    float lr = n.kex * log1pf((pb - pa) * ipa);
-    return -n.cp_d * (n.Tmr * lr + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * expm1f(7.0f * lr));
+    const float x = (pb - pa) * ipa;
+    const float l = ca_log1p(x, ca_small(x));
+    return -n.cp_d * (n.Tmr * (n.kex * l) + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * ca_pow2m1(n, x, l));
 }
-// Both differences from one log1p and one expm1: with x = expm1(lr),
-// Pi_b - Pi_a = Pi_a x and expm1(7 lr) = (1 + x)^7 - 1 expanded in x (no
-// cancellation for small x).
+// the same and Pi_b - Pi_a = Pi_a expm1(kex log1p(x))
 __device__ __forceinline__ void ca_dref(const DevNum &n, float pa, float ipa, float Pia, float pb, float &dPhr,
                                         float &dPi) {
-    const float lr = n.kex * log1pf((pb - pa) * ipa);
-    const float x = expm1f(lr);
-    const float e7 = x * (7.0f + x * (21.0f + x * (35.0f + x * (35.0f + x * (21.0f + x * (7.0f + x))))));
-    dPi = Pia * x;
-    dPhr = -n.cp_d * (n.Tmr * lr + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * e7);
+    const float x = (pb - pa) * ipa;
+    const bool small = ca_small(x);
+    const float l = ca_log1p(x, small);
+    dPi = Pia * ca_expm1(n.kex * l, small);
+    dPhr = -n.cp_d * (n.Tmr * (n.kex * l) + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * ca_pow2m1(n, x, l));
 }
 
 // horizontal metric at scale s (no topography): contravariant u^a = g^{ab} u_b / s^2

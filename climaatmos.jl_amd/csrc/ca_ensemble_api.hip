@@ -118,6 +118,7 @@ ca_status ens_create_impl(ca_ensemble *e, const ca_params *par, const ca_config 
     n.dp0inv = 1.0 / par->p_ref_theta;
     n.dkex = par->R_d / par->cp_d;
     n.dkex_r = n.dkex - 2.0 / 7.0;
+    n.kex7r = (float)(7.0 * n.dkex_r);
     if (std::fabs(n.dkex_r) > 1e-6)
         return efail(e, CA_ERR_ARG, "ca_ensemble_create: R_d / cp_d must be 2/7 to within 1e-6 (dry air; the float64 "
                                     "Exner function refines q^(2/7))");
