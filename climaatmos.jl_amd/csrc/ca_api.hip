@@ -75,6 +75,7 @@ struct ca_handle {
     int lap_chunk = 4;  // levels per work item of k_laplacians
     int dss_kind = 0;  // 0: LDS-staged per element cluster, 1: direct gather
     // reverse mode (ca_step_adjoint and the *_vjp hooks)
+    bool rev = false;             // inside such a call: the kernels' REV forms
     DevGeom gT{};                 // g with the transposed DSS tables
     DevGeom *cgeo = nullptr;      // per-column one-column views of g (Newton stage reverse)
     int adj_chunk = 8;            // levels per work item of k_explicit_vjp
@@ -302,6 +303,15 @@ ca_status dss_state(ca_handle *h, float *Y, hipStream_t st, int kid) {
     return dss_gather_state(h, h->raw, Y, 0, st, kid);
 }
 
+template <bool FIN, bool REV>
+void launch_explicit_sphere(const DevGeom &g, const DevNum &n, bool hy, bool vd, dim3 grid, const float *Y,
+                            const float *Lw, float *out, int ch, const FinFuse &fin, hipStream_t st) {
+    if (hy && !vd) k_explicit<true, true, false, FIN, REV><<<grid, 256, 0, st>>>(g, n, Y, Lw, out, ch, fin);
+    else if (!hy && !vd) k_explicit<true, false, false, FIN, REV><<<grid, 256, 0, st>>>(g, n, Y, Lw, out, ch, fin);
+    else if (hy && vd) k_explicit<true, true, true, FIN, REV><<<grid, 256, 0, st>>>(g, n, Y, Lw, out, ch, fin);
+    else k_explicit<true, false, true, FIN, REV><<<grid, 256, 0, st>>>(g, n, Y, Lw, out, ch, fin);
+}
+
 template <bool FIN>
 void launch_explicit(ca_handle *h, const float *Y, const float *Lw, float *out, const FinFuse &fin, hipStream_t st) {
     const DevGeom &g = h->g;
@@ -312,14 +322,21 @@ void launch_explicit(ca_handle *h, const float *Y, const float *Lw, float *out, 
     // with implicit diffusion the vertical diffusion is in the implicit tendency
     const bool hy = n.hyper != 0, vd = n.vdiff != 0 && !n.idiff;
     if (n.sphere) {
-        if (hy && !vd) k_explicit<true, true, false, FIN><<<grid, blk, 0, st>>>(g, n, Y, Lw, out, ch, fin);
-        else if (!hy && !vd) k_explicit<true, false, false, FIN><<<grid, blk, 0, st>>>(g, n, Y, Lw, out, ch, fin);
-        else if (hy && vd) k_explicit<true, true, true, FIN><<<grid, blk, 0, st>>>(g, n, Y, Lw, out, ch, fin);
-        else k_explicit<true, false, true, FIN><<<grid, blk, 0, st>>>(g, n, Y, Lw, out, ch, fin);
+        if (h->rev) launch_explicit_sphere<FIN, true>(g, n, hy, vd, grid, Y, Lw, out, ch, fin, st);
+        else launch_explicit_sphere<FIN, false>(g, n, hy, vd, grid, Y, Lw, out, ch, fin, st);
     } else {
-        if (vd) k_explicit<false, false, true, FIN><<<grid, blk, 0, st>>>(g, n, Y, h->L, out, ch, fin);
-        else k_explicit<false, false, false, FIN><<<grid, blk, 0, st>>>(g, n, Y, h->L, out, ch, fin);
+        if (vd) k_explicit<false, false, true, FIN, false><<<grid, blk, 0, st>>>(g, n, Y, h->L, out, ch, fin);
+        else k_explicit<false, false, false, FIN, false><<<grid, blk, 0, st>>>(g, n, Y, h->L, out, ch, fin);
     }
+}
+
+// the Laplacians at Y, before their DSS, into h->raw
+void launch_laplacians(const ca_handle *h, const float *Y, hipStream_t st) {
+    const dim3 grid(cdiv(h->g.ncol, 256), cdiv(h->g.nlev, h->lap_chunk));
+    if (h->rev)
+        k_laplacians<true><<<grid, 256, 0, st>>>(h->g, h->n, Y, h->raw, h->lap_chunk);
+    else
+        k_laplacians<false><<<grid, 256, 0, st>>>(h->g, h->n, Y, h->raw, h->lap_chunk);
 }
 
 // remaining_tendency!: Laplacians, their DSS, the fused explicit kernel.
@@ -337,8 +354,7 @@ ca_status explicit_tendency(ca_handle *h, float *Yt, const float *Y, hipStream_t
     if (n.sphere && n.hyper) {
         {
             Launch l(h, st, KID_LAPLACIANS);
-            k_laplacians<<<dim3(cdiv(g.ncol, 256), cdiv(g.nlev, h->lap_chunk)), 256, 0, st>>>(g, n, Y, h->raw,
-                                                                                       h->lap_chunk);
+            launch_laplacians(h, Y, st);
         }
         {
             Launch l(h, st, KID_DSS_LAPLACIAN);
@@ -491,6 +507,33 @@ void point_level_tables(DevGeom &g, int nl, const float *dlc, const float *dlf, 
     g.iJvf = dlf + 6 * nf;
     g.isf = dlf + 7 * nf;
     g.isJf = dlf + 8 * nf;
+}
+
+// Levels per work item of the explicit tendency, by a cost model fitted to
+// launches on one MI355X: a level of one wavefront occupies its SIMD for 0.8 us
+// (all wavefronts share this), a chunk's two halo centres cost 1.5 levels, and
+// the last wavefronts to finish add their own length c + 1.5 times 1 plus the
+// share of the slots that the last round leaves empty.  Measured (us, us at the
+// chosen c first): h_elem 30, 63 levels 95.7 at 11 against 101 at 7 or 13 and
+// 107 at 9; h_elem 22, 63 levels 50.9 at 6 against 48.3 at 13 and 53.6 at 5;
+// h_elem 16, 63 levels 31.0 at 7 against 29.6 at 6 and 34.2 at 3; h_elem 8, 30
+// levels 12.5 at 1 against 15.1 at 4; with vertical diffusion h_elem 13, 45
+// levels 29.2 at 4 against 33.3 at 2, h_elem 30, 50 levels 97.1 at 9 against
+// 106 at 7.
+int explicit_chunk(int64_t layer_waves, int nl, int waves_per_simd) {
+    const double slots = 1024.0 * waves_per_simd;
+    int best = 1;
+    double cost = 1e300;
+    for (int c = 1; c <= std::min(nl, 16); ++c) {
+        const int64_t n = (nl + c - 1) / c;
+        const double rounds = layer_waves * n / slots;
+        const double t = 0.8 * layer_waves * (nl + 1.5 * n) / 1024.0 + (c + 1.5) * (1.0 + std::ceil(rounds) - rounds);
+        if (t < cost) {
+            cost = t;
+            best = c;
+        }
+    }
+    return best;
 }
 
 // ca_create's body: fills h; on failure the caller frees h
@@ -713,19 +756,13 @@ ca_status create_impl(const ca_geometry *geom, const ca_params *par, const ca_co
     ars343(h);
     h->newton_variant = (nl + 1 <= 64) ? 1 : 0;
     // level chunks sized so that small grids still fill the chip: about
-    // 1024 wavefronts for the per-node sweeps, 1024 workgroups for the DSS.
-    // The explicit tendency's cap of 7 levels: its wavefronts are long and
-    // few (6 per SIMD fit), so the last partial round of them costs; at
-    // h_elem 30, 63 levels, chunks of 7 (9 per column) fill the slots almost
-    // exactly twice: 112.6 us against 114-115 us for chunks of 5 or 8.
+    // 1024 wavefronts for the per-node sweeps, 1024 workgroups for the DSS
     {
         const int64_t layer_waves = (nc + 63) / 64;
         const int64_t want = (1024 + layer_waves - 1) / layer_waves;
-        h->explicit_chunk = (int)std::min<int64_t>(7, std::max<int64_t>(4, (nl + want - 1) / want));
-        // the last explicit launch runs 4 wavefronts per SIMD; at h_elem 30,
-        // 63 levels its chunks of 11 (6 per column) fill the slots about twice:
-        // 165.8 us against 170.7 us with 7
-        h->final_chunk = (int)std::min<int64_t>(11, std::max<int64_t>(4, (nl + want - 1) / want));
+        // wavefronts of k_explicit a SIMD holds: 3 with vertical diffusion (147
+        // VGPRs), 4 without (105, 124 with the final combination)
+        h->explicit_chunk = h->final_chunk = explicit_chunk(layer_waves, nl, n.vdiff && !n.idiff ? 3 : 4);
         h->adj_chunk = (int)std::min<int64_t>(8, std::max<int64_t>(4, (nl + want - 1) / want));
         h->lap_chunk = (int)std::min<int64_t>(4, std::max<int64_t>(2, (nl + want - 1) / want));
         if (g.ncl > 0) {

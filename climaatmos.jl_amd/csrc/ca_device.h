@@ -203,16 +203,37 @@ __device__ __forceinline__ float ca_pow2m1(const DevNum &n, float x, float l) {
     const float y = 1.0f + x;
     return fmaf(y * y, n.kex7r * l, x * (2.0f + x));
 }
+// REV: trajectories that the reverse mode differentiates keep the library
+// functions.  The upwind side and the limiter's branch are chosen by the state's
+// last bits wherever they nearly tie, the gradient jumps with them (by 1e-4 of
+// its norm over 8 steps at h_elem 8, 30 levels), and recorded runs stay bitwise
+// what their gradients were checked with.  A template parameter, not a run-time
+// flag: the unused branch cost k_explicit 14 VGPRs (96 -> 107 us).
 // ipa = 1 / pa
+template <bool REV>
 __device__ __forceinline__ float ca_dPhiref(const DevNum &n, float pa, float ipa, float Pia, float pb) {
     const float x = (pb - pa) * ipa;
+    if (REV) {
+        const float lr = n.kex * log1pf(x);
+        return -n.cp_d * (n.Tmr * lr + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * expm1f(7.0f * lr));
+    }
     const float l = ca_log1p(x, ca_small(x));
     return -n.cp_d * (n.Tmr * (n.kex * l) + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * ca_pow2m1(n, x, l));
 }
-// the same and Pi_b - Pi_a = Pi_a expm1(kex log1p(x))
+// the same and Pi_b - Pi_a = Pi_a expm1(kex log1p(x)); with REV,
+// (1 + y)^7 - 1 is expanded in y = expm1(kex log1p(x))
+template <bool REV>
 __device__ __forceinline__ void ca_dref(const DevNum &n, float pa, float ipa, float Pia, float pb, float &dPhr,
                                         float &dPi) {
     const float x = (pb - pa) * ipa;
+    if (REV) {
+        const float lr = n.kex * log1pf(x);
+        const float y = expm1f(lr);
+        const float e7 = y * (7.0f + y * (21.0f + y * (35.0f + y * (35.0f + y * (21.0f + y * (7.0f + y))))));
+        dPi = Pia * y;
+        dPhr = -n.cp_d * (n.Tmr * lr + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * e7);
+        return;
+    }
     const bool small = ca_small(x);
     const float l = ca_log1p(x, small);
     dPi = Pia * ca_expm1(n.kex * l, small);
@@ -420,6 +441,7 @@ __device__ __forceinline__ void op_wcurl12(const Nod &q, const Met &m, float u3,
 // The s_d - s_d,r field is taken relative to its value at the element's first
 // node (a constant inside the element, annihilated by the gradient), which
 // removes the large geopotential part.
+template <bool REV>
 __device__ __forceinline__ void lap_point(const DevGeom &g, const DevNum &n, const Nod &q, float W, float iW,
                                           float Jh, float iJh, const ColMet &cm, int k, float rho, float u1,
                                           float u2, float rhoe, float u3a, float u3b, float out[4]) {
@@ -456,7 +478,7 @@ __device__ __forceinline__ void lap_point(const DevGeom &g, const DevNum &n, con
     out[2] = 0.0f - wc3;
     // scalar Laplacian of the dry static energy deviation
     const float p0 = ca_elem0(p), Pi0 = ca_elem0(Pi);
-    const float psi = n.cp_d * (T - ca_Tref(n, Pi)) - ca_dPhiref(n, p0, ca_rcp(p0), Pi0, p);
+    const float psi = n.cp_d * (T - ca_Tref(n, Pi)) - ca_dPhiref<REV>(n, p0, ca_rcp(p0), Pi0, p);
     float q1, q2;
     op_grad(q, psi, q1, q2);
     float v1, v2;

@@ -72,9 +72,10 @@ struct FinFuse {
 };
 
 // explicit tendency (ca_spectral.hip)
+template <bool REV>  // REV: for a trajectory the reverse mode differentiates
 __global__ void k_laplacians(DevGeom g, DevNum n, const float *Y, float *L, int chunk);
 // FIN: Yt receives U + the combination of FinFuse instead of the tendency at U
-template <bool SPH, bool HYPER, bool VDIFF, bool FIN>
+template <bool SPH, bool HYPER, bool VDIFF, bool FIN, bool REV>
 __global__ void k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int chunk,
                            FinFuse fin);
 

@@ -27,6 +27,7 @@ __device__ __forceinline__ float u3f_at(const DevGeom &g, const float *u3, int f
 // carrying u_3 of the face between two levels and the column's horizontal
 // metric in registers (each face and metric value is read once); chunk = 0
 // means the whole column.
+template <bool REV>
 __global__ void __launch_bounds__(256) k_laplacians(DevGeom g, DevNum n, const float *Y, float *L, int chunk) {
     const int col = blockIdx.x * blockDim.x + threadIdx.x;
     if (col >= g.ncol) return;
@@ -45,7 +46,7 @@ __global__ void __launch_bounds__(256) k_laplacians(DevGeom g, DevNum n, const f
         const float *Yk = Y + (int64_t)k * nc;
         const float u3b = k + 1 <= nl - 1 ? ca_ldo(u3 + (int64_t)(k + 1) * nc, cb) : 0.0f;
         float o[4];
-        lap_point(g, n, q, W, iW, Jh, iJh, cm, k, ca_ldo(Yk, cb), ca_ldo(Yk + nC, cb), ca_ldo(Yk + 2 * nC, cb),
+        lap_point<REV>(g, n, q, W, iW, Jh, iJh, cm, k, ca_ldo(Yk, cb), ca_ldo(Yk + nC, cb), ca_ldo(Yk + 2 * nC, cb),
                   ca_ldo(Yk + 3 * nC, cb), u3a, u3b, o);
         float *Lk = L + (int64_t)k * nc;
 #pragma unroll
@@ -53,6 +54,9 @@ __global__ void __launch_bounds__(256) k_laplacians(DevGeom g, DevNum n, const f
         u3a = u3b;
     }
 }
+
+template __global__ void k_laplacians<false>(DevGeom, DevNum, const float *, float *, int);
+template __global__ void k_laplacians<true>(DevGeom, DevNum, const float *, float *, int);
 
 // --------------------------------------------------------- explicit kernel
 struct ColState {
@@ -71,23 +75,22 @@ struct ColState {
 // face term of its top centre).  chunk = 0 means the whole column.
 // SPH / HYPER / VDIFF select the sphere (horizontal operators), the
 // hyperdiffusion and the vertical diffusion at compile time.
-// The sphere dynamics with hyperdiffusion and no vertical diffusion (the
-// large-grid case) is compiled for 6 wavefronts per SIMD (80 VGPRs, a 20-byte
-// spill) instead of the 5 that 93 VGPRs allow: its wavefronts are long and
-// few, so how evenly they fill the slots matters more than the spill.  With
-// 7-level chunks (the default for large grids) the grid fills 6 per SIMD
-// almost exactly twice; at h_elem 30, 63 levels this measured 112.7 us
-// against 116.1 us for 5 per SIMD at its best chunk (6).
+// Level k + 1 (and the face above it) is loaded while level k is computed: the
+// kernel issues about 300 VALU instructions per level, and with the loads at
+// their use it waited 63% of its wavefront cycles, mostly for them.  The nine
+// values in flight fit 105 VGPRs, 4 wavefronts per SIMD.  At h_elem 30, 63
+// levels: 96 us with them and chunks of 11; without, 111 us at 5 wavefronts per
+// SIMD and 120 us at 6 (80 VGPRs, a 36-byte spill).
 // FIN (the step's last explicit tendency, which also forms the final
-// combination) loads three earlier tendencies at the top of each level so
-// that they arrive during the level's arithmetic.  Those 15 values in flight
-// need registers: at 4 wavefronts per SIMD (110 VGPRs, no spill) the launch
-// measured 171 us at h_elem 30, 63 levels; at 5 (96 VGPRs, a 48-byte spill)
-// 224 us; with the loads at the store point instead, 280 us; a separate
-// tendency and combination kernel took 112 + 139 us.
-template <bool SPH, bool HYPER, bool VDIFF, bool FIN>
+// combination) also loads three earlier tendencies at the top of each level so
+// that they arrive during the level's arithmetic.  With these 24 values in
+// flight it is compiled for 3 wavefronts per SIMD: 148 us at the same size
+// against 169 us for 4 (124 VGPRs) and 163 us for 4 without the level
+// prefetch.
+// REV: see ca_dPhiref.
+template <bool SPH, bool HYPER, bool VDIFF, bool FIN, bool REV>
 __global__ void __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(SPH && HYPER && !VDIFF ? (FIN ? 4 : 6) : 1, 8)))
+__attribute__((amdgpu_waves_per_eu(SPH && HYPER && !VDIFF ? (FIN ? 3 : 4) : 1, 8)))
 k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int chunk, FinFuse fin) {
     int col = blockIdx.x * blockDim.x + threadIdx.x;
     if (col >= g.ncol) return;
@@ -118,6 +121,26 @@ k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int c
     const int kbeg = k0 > 0 ? k0 - 1 : 0;
     const int kend = k1;  // inclusive: face k1 closes the top owned centre
     float u3a = u3f_at(g, u3, kbeg, col);  // u_3 at face k
+    // the next level's state and Laplacians (L_3 alone at a halo centre) and the
+    // u_3 of the face above it
+    float nY[4] = {1.0f, 0.0f, 0.0f, 0.0f}, nL[4] = {0.0f, 0.0f, 0.0f, 0.0f}, nU = 0.0f;
+    auto fetch = [&](int k) {
+        nU = k + 1 <= nl - 1 ? ca_ldo(u3 + (int64_t)(k + 1) * nc, cb) : 0.0f;
+        if (k >= nl) return;
+        const float *Yk = Y + (int64_t)k * nc;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) nY[p] = ca_ldo(Yk + p * nC, cb);
+        if (SPH && HYPER) {
+            const float *Lk = L + (int64_t)k * nc;
+            if (k >= k0 && k < k1) {
+                nL[0] = ca_ldo(Lk, cb);
+                nL[1] = ca_ldo(Lk + nC, cb);
+                nL[3] = ca_ldo(Lk + 3 * nC, cb);
+            }
+            nL[2] = ca_ldo(Lk + 2 * nC, cb);
+        }
+    };
+    fetch(kbeg);
     for (int k = kbeg; k <= kend; ++k) {
         // FIN: the earlier stages' tendencies at centre k - 1 and face k, loaded
         // here so that their latency hides behind this level's arithmetic
@@ -132,11 +155,10 @@ k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int c
 #pragma unroll
                 for (int j = 0; j < 3; ++j) fe_f[j] = ca_ldo(fin.fe[j] + 4 * nC + (int64_t)k * nc, cb);
         }
-        float u3b = (k + 1 >= 1 && k + 1 <= nl - 1) ? ca_ldo(u3 + (int64_t)(k + 1) * nc, cb) : 0.0f;
+        const float rho = nY[0], u1 = nY[1], u2 = nY[2], rhoe = nY[3], u3b = nU;
+        const float X1 = nL[0], X2 = nL[1], X3 = nL[2], Ls = nL[3];
+        if (k < kend) fetch(k + 1);
         if (k < nl) {
-            const float *Yk = Y + (int64_t)k * nc;
-            float rho = ca_ldo(Yk, cb), u1 = ca_ldo(Yk + nC, cb), u2 = ca_ldo(Yk + 2 * nC, cb),
-                  rhoe = ca_ldo(Yk + 3 * nC, cb);
             float s = g.sc[k], s2 = s * s, is2 = g.is2c[k], Jv = g.Jvc[k];
             const Met m = ca_met(W, iW, Jh * s2 * Jv, iJh * g.isJc[k]);
             const float J = m.J;
@@ -176,7 +198,7 @@ k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int c
                 // u_h -= C12(grad(K + Phi - Phi_r) + cp_d (th' grad Pi + grad(th' Pi) - Pi grad th') / 2)
                 float p0 = ca_elem0(p), Pi0 = ca_elem0(Pi), ip0 = ca_rcp(p0);
                 float dPhr, dPi;
-                ca_dref(n, p0, ip0, Pi0, p, dPhr, dPi);
+                ca_dref<REV>(n, p0, ip0, Pi0, p, dPhr, dPi);
                 float A = K - dPhr;
                 float thPi = T - ca_Tref(n, Pi);
                 float th = thPi * ca_rcp(Pi);
@@ -189,7 +211,6 @@ k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int c
                 d2 -= g2 + n.cp_d * (th * a2 + b2 - Pi * c2) * 0.5f;
             }
             if (sph && HYPER && !own) {  // l4 alone, as below
-                const float X3 = ca_ldo(L + 2 * nC + (int64_t)k * nc, cb);
                 float cr1, cr2;
                 op_curl12(q, m, X3, cr1, cr2);
                 float cc1, cc2;
@@ -201,9 +222,6 @@ k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int c
             if (sph && own) {
                 // ---- apply_hyperdiffusion_tendency! (hyperdiffusion.jl:273-307)
                 if (HYPER) {
-                    const float *Lk = L + (int64_t)k * nc;
-                    float X1 = ca_ldo(Lk, cb), X2 = ca_ldo(Lk + nC, cb), X3 = ca_ldo(Lk + 2 * nC, cb),
-                          Ls = ca_ldo(Lk + 3 * nC, cb);
                     float v1, v2;
                     ca_contra(cm, is2, X1, X2, v1, v2);
                     float dv = op_div(q, m, v1, v2);
@@ -380,30 +398,22 @@ k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int c
     }
 }
 
-template __global__ void k_explicit<true, true, false, false>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<true, true, false, true>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<true, false, false, false>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<true, false, false, true>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<true, true, true, false>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<true, true, true, true>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<true, false, true, false>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<true, false, true, true>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<false, false, false, false>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<false, false, false, true>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<false, false, true, false>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
-template __global__ void k_explicit<false, false, true, true>(DevGeom, DevNum, const float *, const float *,
-                                                                    float *, int, FinFuse);
+#define CA_INST_EXPLICIT(SPH, HYPER, VDIFF, REV)                                                             \
+    template __global__ void k_explicit<SPH, HYPER, VDIFF, false, REV>(DevGeom, DevNum, const float *, const float *, \
+                                                                       float *, int, FinFuse);               \
+    template __global__ void k_explicit<SPH, HYPER, VDIFF, true, REV>(DevGeom, DevNum, const float *, const float *,  \
+                                                                      float *, int, FinFuse);
+CA_INST_EXPLICIT(true, true, false, false)
+CA_INST_EXPLICIT(true, true, true, false)
+CA_INST_EXPLICIT(true, false, false, false)
+CA_INST_EXPLICIT(true, false, true, false)
+CA_INST_EXPLICIT(true, true, false, true)
+CA_INST_EXPLICIT(true, true, true, true)
+CA_INST_EXPLICIT(true, false, false, true)
+CA_INST_EXPLICIT(true, false, true, true)
+CA_INST_EXPLICIT(false, false, false, false)
+CA_INST_EXPLICIT(false, false, true, false)
+#undef CA_INST_EXPLICIT
 
 // ------------------------------------------------------------ surface flux
 // surface_flux_tendency! (surface_flux.jl:101-145) with the surface conditions

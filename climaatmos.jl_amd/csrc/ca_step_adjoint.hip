@@ -219,7 +219,7 @@ __device__ __forceinline__ void loc_forward(Loc &c, const DevGeom &g, const DevN
     c.Pi0 = ca_elem0(c.Pi);
     const float ip0 = ca_rcp(c.p0);
     float dPhr, dPi;
-    ca_dref(n, c.p0, ip0, c.Pi0, c.p, dPhr, dPi);
+    ca_dref<true>(n, c.p0, ip0, c.Pi0, c.p, dPhr, dPi);
     const float A = K - dPhr;
     c.thPi = c.T - ca_Tref(n, c.Pi);
     c.th = c.thPi * ca_rcp(c.Pi);

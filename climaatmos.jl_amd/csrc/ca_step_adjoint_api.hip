@@ -6,6 +6,13 @@
 
 namespace {
 
+// for the time of a reverse-mode call, the forward kernels are their REV forms
+struct RevScope {
+    ca_handle *h;
+    explicit RevScope(ca_handle *h_) : h(h_) { h->rev = true; }
+    ~RevScope() { h->rev = false; }
+};
+
 // planes of the S-sized reverse-mode scratch h->aw_buf
 enum AdjBuf { AB_UB, AB_CB, AB_UTB1, AB_UTB2, AB_UTB3, AB_FEB, AB_FIB, AB_GB, AB_UBS, AB_Y, AB_YF, AB_COUNT };
 
@@ -281,6 +288,7 @@ ca_status ca_remaining_tendency_vjp(ca_handle *h, float *Yb, const float *Ytb, c
     if (h->n.idiff) return fail(h, CA_ERR_ARG, "ca_remaining_tendency_vjp: the reverse mode has no implicit diffusion");
     if (!h->vd_plain)
         return fail(h, CA_ERR_ARG, "ca_remaining_tendency_vjp: the reverse mode takes DecayWithHeightDiffusion with H = inf only");
+    const RevScope rev(h);
     hipStream_t st = (hipStream_t)stream;
     const DevGeom &g = h->g;
     ca_status s;
@@ -289,8 +297,7 @@ ca_status ca_remaining_tendency_vjp(ca_handle *h, float *Yb, const float *Ytb, c
     if (h->n.hyper) {  // the DSSed Laplacians at Y
         {
             Launch l(h, st, KID_LAPLACIANS);
-            k_laplacians<<<dim3(cdiv(g.ncol, 256), cdiv(g.nlev, h->lap_chunk)), 256, 0, st>>>(g, h->n, Y, h->raw,
-                                                                                       h->lap_chunk);
+            launch_laplacians(h, Y, st);
         }
         {
             Launch l(h, st, KID_DSS_LAPLACIAN);
@@ -312,6 +319,7 @@ ca_status ca_step_record(ca_handle *h, float *Y, double dt, int32_t nsteps, int3
     if (h->n.idiff) return fail(h, CA_ERR_ARG, "ca_step_record: the reverse mode has no implicit diffusion");
     if (!h->vd_plain)
         return fail(h, CA_ERR_ARG, "ca_step_record: the reverse mode takes DecayWithHeightDiffusion with H = inf only");
+    const RevScope rev(h);
     hipStream_t st = (hipStream_t)stream;
     const int64_t S = h->S;
     const bool all = every == 0;  // the stage records of every step, no checkpoints
@@ -341,6 +349,7 @@ ca_status ca_step_record(ca_handle *h, float *Y, double dt, int32_t nsteps, int3
 ca_status ca_step_pullback(ca_handle *h, const float *YbN, float *Yb0, float *D0b, void *stream) {
     if (!h || !YbN || !Yb0) return CA_ERR_ARG;
     if (!h->rec_valid) return fail(h, CA_ERR_ARG, "ca_step_pullback: no trajectory recorded (ca_step_record)");
+    const RevScope rev(h);
     hipStream_t st = (hipStream_t)stream;
     const int64_t S = h->S;
     const int nsteps = h->rec_nsteps, every = h->rec_every;
