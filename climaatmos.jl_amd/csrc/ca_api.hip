@@ -381,46 +381,75 @@ ca_status explicit_tendency(ca_handle *h, float *Yt, const float *Y, hipStream_t
 
 inline bool ca_al16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
-template <int TC, bool V4>
-void launch_pcr_tcv(ca_handle *h, const StageSrc &src, float dtg, int i, float *U, float *Ut, hipStream_t st,
-                    bool keep_fi) {
-    float *FI = keep_fi ? h->FI[i] : nullptr;
-    const DevGeom &g = h->g;
-    const dim3 grid(cdiv(g.ncol, TC)), blk(256);
-    if (src.nfull == 2 && src.nfi == 0)
-        k_newton_pcr<TC, 2, 0, V4><<<grid, blk, 0, st>>>(g, h->n, src, dtg, U, FI, Ut);
-    else if (src.nfull == 3 && src.nfi == 1)
-        k_newton_pcr<TC, 3, 1, V4><<<grid, blk, 0, st>>>(g, h->n, src, dtg, U, FI, Ut);
-    else if (src.nfull == 4 && src.nfi == 2)
-        k_newton_pcr<TC, 4, 2, V4><<<grid, blk, 0, st>>>(g, h->n, src, dtg, U, FI, Ut);
-    else
-        k_newton_pcr<TC, -1, -1, V4><<<grid, blk, 0, st>>>(g, h->n, src, dtg, U, FI, Ut);
-}
-
-// 16-byte row accesses when every row of every plane is 16-byte aligned:
-// ncol a multiple of 4 and all base pointers 16-byte aligned
-template <int TC>
-void launch_pcr_tc(ca_handle *h, const StageSrc &src, float dtg, int i, float *U, float *Ut, hipStream_t st,
-                   bool keep_fi) {
-    bool v4 = TC == 16 && h->g.ncol % 4 == 0 && ca_al16(U) && ca_al16(h->FI[i]) && (!Ut || ca_al16(Ut));
+// 16-byte row accesses of a Newton stage's tile when every row of every plane is
+// 16-byte aligned: ncol a multiple of 4 and all base pointers 16-byte aligned.
+// (The sources of the ARS343 stages are 2 full states, 3 and one implicit
+// tendency, or 4 and two.)
+inline bool stage_al16(const ca_handle *h, const StageSrc &src, int i, const float *U, const float *Ut) {
+    bool v4 = h->g.ncol % 4 == 0 && ca_al16(U) && ca_al16(h->FI[i]) && (!Ut || ca_al16(Ut));
     for (int t = 0; t < src.nfull; ++t) v4 = v4 && ca_al16(src.full[t]);
     for (int t = 0; t < src.nfi; ++t) v4 = v4 && ca_al16(src.fi[t]);
-    if (v4)
-        launch_pcr_tcv<16, true>(h, src, dtg, i, U, Ut, st, keep_fi);
-    else
-        launch_pcr_tcv<TC, false>(h, src, dtg, i, U, Ut, st, keep_fi);
+    return v4;
 }
 
-// the implicit stage i from src into U (h->U unless the caller records);
-// Ut (optional) receives the assembled U~; keep_fi = false leaves F_I
-// unstored (the step's last stage: the final combination does not read it)
-void launch_newton_pcr(ca_handle *h, const StageSrc &src, float dtg, int i, hipStream_t st, float *U = nullptr,
-                       float *Ut = nullptr, bool keep_fi = true) {
-    if (!U) U = h->U;
-    if (h->newton_variant == 2)
-        launch_pcr_tc<32>(h, src, dtg, i, U, Ut, st, keep_fi);
+template <int R, int W, int TC, int NT, bool V4>
+void launch_rows_v(const ca_handle *h, const StageSrc &src, float dtg, float *U, float *FI, hipStream_t st) {
+    const DevGeom &g = h->g;
+    const unsigned nb = cdiv(g.ncol, TC);
+    if (src.nfull == 2)
+        k_newton_rows<R, W, TC, NT, 2, 0, V4><<<nb, NT, 0, st>>>(g, h->n, src, dtg, U, FI);
+    else if (src.nfull == 3)
+        k_newton_rows<R, W, TC, NT, 3, 1, V4><<<nb, NT, 0, st>>>(g, h->n, src, dtg, U, FI);
     else
-        launch_pcr_tc<16>(h, src, dtg, i, U, Ut, st, keep_fi);
+        k_newton_rows<R, W, TC, NT, 4, 2, V4><<<nb, NT, 0, st>>>(g, h->n, src, dtg, U, FI);
+}
+template <int R, int W, int TC, int NT>
+void launch_rows(const ca_handle *h, bool v4, const StageSrc &src, float dtg, float *U, float *FI, hipStream_t st) {
+    if (v4) launch_rows_v<R, W, TC, NT, true>(h, src, dtg, U, FI, st);
+    else launch_rows_v<R, W, TC, NT, false>(h, src, dtg, U, FI, st);
+}
+
+// The implicit stage i from src into U, a column in a wavefront's registers
+// (nlev <= 128).  keep_fi = false leaves F_I unstored (the step's last stage:
+// the final combination does not read it).  The shapes and their measurements
+// are listed at k_newton_rows; two columns share a wavefront only on a sphere
+// (independent columns do not touch each other's lanes).  The shape does not
+// follow the alignment: an unaligned state steps bitwise like an aligned one.
+void launch_newton_rows(const ca_handle *h, const StageSrc &src, float dtg, int i, hipStream_t st, float *U,
+                        bool keep_fi) {
+    const DevGeom &g = h->g;
+    const int nl = g.nlev;
+    const bool v4 = stage_al16(h, src, i, U, nullptr);
+    float *FI = keep_fi ? h->FI[i] : nullptr;
+    if (nl >= 64) launch_rows<2, 64, 16, 256>(h, v4, src, dtg, U, FI, st);
+    else if (h->newton_variant == 2) launch_rows<1, 64, 32, 256>(h, v4, src, dtg, U, FI, st);  // 32-column tiles
+    else if (!h->n.sphere || (nl > 56 && g.ncol >= 16 * 4096)) launch_rows<1, 64, 16, 256>(h, v4, src, dtg, U, FI, st);
+    else if (nl > 32) launch_rows<2, 32, 16, 256>(h, v4, src, dtg, U, FI, st);
+    else launch_rows<1, 32, 16, 512>(h, v4, src, dtg, U, FI, st);
+}
+
+template <bool V4>
+void launch_pcr(const ca_handle *h, const StageSrc &src, float dtg, float *U, float *FI, float *Ut, hipStream_t st) {
+    const DevGeom &g = h->g;
+    const unsigned nb = cdiv(g.ncol, 16);
+    if (src.nfull == 2)
+        k_newton_pcr<16, 2, 0, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI, Ut);
+    else if (src.nfull == 3)
+        k_newton_pcr<16, 3, 1, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI, Ut);
+    else
+        k_newton_pcr<16, 4, 2, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI, Ut);
+}
+
+// The same for a trajectory the reverse mode differentiates (nlev <= 63), which
+// keeps k_newton_pcr's arithmetic bit for bit; Ut (optional) receives the
+// assembled U~.
+void launch_newton_pcr(const ca_handle *h, const StageSrc &src, float dtg, int i, hipStream_t st, float *U, float *Ut,
+                       bool keep_fi) {
+    float *FI = keep_fi ? h->FI[i] : nullptr;
+    if (stage_al16(h, src, i, U, Ut))
+        launch_pcr<true>(h, src, dtg, U, FI, Ut, st);
+    else
+        launch_pcr<false>(h, src, dtg, U, FI, Ut, st);
 }
 
 ca_status ensure_bands(ca_handle *h) {
@@ -958,7 +987,10 @@ ca_status one_step(ca_handle *h, float *Y, double dt, hipStream_t st, float *rec
             }
             continue;
         }
-        const bool pcr = h->newton_variant == 1 || h->newton_variant == 2;
+        // a wavefront per column up to 128 levels (64 in a trajectory the reverse
+        // mode differentiates), unless the caller asked for a thread per column
+        const bool pcr = h->rev && h->newton_variant >= 1;
+        const bool rows = !h->rev && (h->newton_variant >= 1 || (g.nlev >= 64 && g.nlev <= 128));
         if (rec && !pcr) {  // the PCR stage records U~ itself
             sadj::k_stage_state<<<dim3(cdiv(g.ncol, 256), g.nlev + 1), 256, 0, st>>>(g, src, rec_Ut(h, rec, i));
             if ((s = check_launch(h, "k_stage_state"))) return s;
@@ -966,7 +998,9 @@ ca_status one_step(ca_handle *h, float *Y, double dt, hipStream_t st, float *rec
         float *Ui = rec ? rec_U(h, rec, i) : h->U;
         {
             Launch l(h, st, KID_NEWTON_STAGE);
-            if (pcr)
+            if (rows)
+                launch_newton_rows(h, src, dtg, i, st, Ui, i < last);
+            else if (pcr)
                 launch_newton_pcr(h, src, dtg, i, st, Ui, rec ? rec_Ut(h, rec, i) : nullptr, i < last);
             else
                 k_newton_stage<<<cdiv(g.ncol, 128), 128, 0, st>>>(g, h->n, src, dtg, Ui, h->FI[i], h->scr);

@@ -9,7 +9,7 @@
 // (theta_v, theta_v - theta_vr, Pi^7, dp/drho) is formed once per centre and
 // exchanged, not recomputed on both faces, and the centre rows of the Jacobian
 // are formed on each face from the face fluxes q = I^f(rho J) g^33 and q h.
-// Included after ca_column.hip and ca_newton_pcr.hip.
+// Included by ca_newton_pcr.hip after its lane exchanges.
 #pragma once
 #include "ca_kernels.h"
 
@@ -101,7 +101,9 @@ __device__ __forceinline__ double temperature(const DevNum &n, double et, float 
 // The tridiagonal Schur system in float64 (the acoustic system is stiff:
 // dtg c / dz >> 1).  Two rows per lane: the odd row is eliminated into its
 // even neighbours first, which leaves one row per lane for parallel cyclic
-// reduction over the 64 lanes, and is substituted back.
+// reduction over the column's W lanes, and is substituted back.  With W = 32 the
+// exchanges across lanes 31 / 32 fetch the other column's finite values, which
+// meet exactly zero couplings.
 template <int R, int W>
 __device__ __forceinline__ void solve(const double (&L)[R], const double (&D)[R], const double (&U)[R],
                                       const double (&b)[R], float (&x)[R]) {
@@ -296,144 +298,3 @@ __device__ __forceinline__ void newton(const Lev<R> &t, const Met1 &m, const Dev
 }
 
 }  // namespace cst
-
-// The fused implicit stage.  A workgroup assembles a tile of TC columns into
-// LDS with coalesced row loads, each wavefront solves 64 / W columns at a time
-// from LDS, and the results leave through LDS.
-// The tile is unpadded; column c of row k lies at c ^ ((k >> 2) & (TC - 1)), so
-// that the lanes of a wavefront, which read one column down the rows, touch
-// every bank once (TC = 16).
-template <int R, int W, int TC, int NT, int OCC, int NF, int NI, bool V4>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1, 8)))
-k_newton_rows(DevGeom g, DevNum n, StageSrc src, float dtg, float *U, float *FI, float *Ut) {
-    constexpr int ROWS = R * W;
-    __shared__ float tU[5][ROWS][TC];
-    __shared__ float tF[3][ROWS][TC];
-    const int nl = g.nlev;
-    const int64_t nC = g.nC, nc = g.ncol;
-    const int col0 = ca_xcd_tile(blockIdx.x, gridDim.x) * TC;
-    const int tid = threadIdx.x;
-    constexpr int VW = V4 ? 4 : 1;
-    auto sw = [](int k, int c) { return c ^ ((k >> 2) & (TC - 1)); };
-    // ---- U~: rows 0 .. nl of the tile (row nl only holds u_3 = 0)
-    for (int idx = tid; idx < (nl + 1) * (TC / VW); idx += NT) {
-        const int r = idx / (TC / VW), c = VW * (idx - r * (TC / VW));
-        const int col = col0 + c;
-        const int64_t q = (int64_t)r * nc + col;
-        const bool ok = col < nc, cen = r < nl, face = r >= 1 && r < nl;
-        if constexpr (V4) {
-            float4 v[5];
-            assemble4<NF, NI>(src, nC, q, ok, cen, face, v);
-            if (cen)
-#pragma unroll
-                for (int p = 0; p < 5; ++p) {
-                    tU[p][r][sw(r, c)] = v[p].x;
-                    tU[p][r][sw(r, c + 1)] = v[p].y;
-                    tU[p][r][sw(r, c + 2)] = v[p].z;
-                    tU[p][r][sw(r, c + 3)] = v[p].w;
-                }
-            if (Ut && ok) {  // U~ for the reverse pass (when recording)
-                if (cen)
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) *reinterpret_cast<float4 *>(Ut + p * nC + q) = v[p];
-                *reinterpret_cast<float4 *>(Ut + 4 * nC + q) = v[4];
-            }
-        } else {
-            float v[5];
-            assemble<NF, NI>(src, nC, q, ok, cen, face, v);
-            if (cen)
-#pragma unroll
-                for (int p = 0; p < 5; ++p) tU[p][r][sw(r, c)] = v[p];
-            if (Ut && ok) {
-                if (cen)
-#pragma unroll
-                    for (int p = 0; p < 4; ++p) Ut[p * nC + q] = v[p];
-                Ut[4 * nC + q] = v[4];
-            }
-        }
-    }
-    __syncthreads();
-    // ---- 64 / W columns per wavefront, R rows per lane
-    {
-        constexpr int CPW = 64 / W;
-        const float idtg = 1.0f / dtg;
-        cst::Lev<R> t;
-        if (OCC == 0) cst::lev_load<R>(g, tid & (W - 1), t);
-        for (int cc = tid / W; cc < TC; cc += NT / 64 * CPW) {
-            const int col = col0 + cc;
-            if (col >= nc) break;  // uniform across the wavefront (W = 32: ncol is a multiple of 16)
-            if (OCC > 0) {
-                int lane = tid & (W - 1);
-                asm volatile("" : "+v"(lane));
-                cst::lev_load<R>(g, lane, t);
-            }
-            const cst::Met1 m = cst::met1_load(g, n, col);
-            float rho[R], u1[R], u2[R], rhoe[R], u3[R], fr[R], fe[R], fu[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int kc = min(t.k[r], nl - 1), c = sw(kc, cc);
-                rho[r] = tU[0][kc][c];
-                u1[r] = tU[1][kc][c];
-                u2[r] = tU[2][kc][c];
-                rhoe[r] = tU[3][kc][c];
-                u3[r] = t.intF[r] ? tU[4][kc][c] : 0.0f;
-            }
-            cst::newton<R, W>(t, m, n, nl, dtg, idtg, rho, u1, u2, rhoe, u3, fr, fe, fu);
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                if (t.hasC[r]) {
-                    const int k = t.k[r], c = sw(k, cc);
-                    tU[0][k][c] = rho[r];
-                    tU[3][k][c] = rhoe[r];
-                    tU[4][k][c] = u3[r];
-                    tF[0][k][c] = fr[r];
-                    tF[1][k][c] = fe[r];
-                    tF[2][k][c] = fu[r];
-                }
-        }
-    }
-    __syncthreads();
-    // ---- U and F_I out (face nl: zero)
-    for (int idx = tid; idx < (nl + 1) * (TC / VW); idx += NT) {
-        const int r = idx / (TC / VW), c = VW * (idx - r * (TC / VW));
-        const int col = col0 + c;
-        if (col >= nc) continue;
-        const int64_t q = (int64_t)r * nc + col;
-        auto put = [&](float *dst, const float (*tile)[TC], bool in) {
-            if constexpr (V4)
-                *reinterpret_cast<float4 *>(dst) = in ? make_float4(tile[r][sw(r, c)], tile[r][sw(r, c + 1)],
-                                                                    tile[r][sw(r, c + 2)], tile[r][sw(r, c + 3)])
-                                                      : make_float4(0.f, 0.f, 0.f, 0.f);
-            else
-                *dst = in ? tile[r][sw(r, c)] : 0.0f;
-        };
-        if (r < nl) {
-#pragma unroll
-            for (int p = 0; p < 4; ++p) put(U + p * nC + q, tU[p], true);
-            if (FI) {
-                put(FI + q, tF[0], true);
-                put(FI + nC + q, tF[1], true);
-            }
-        }
-        put(U + 4 * nC + q, tU[4], r < nl);
-        if (FI) put(FI + 2 * nC + q, tF[2], r < nl);
-    }
-}
-
-#define CA_INST_ROWS(R, W, NT, OCC, V4)                                                                          \
-    template __global__ void k_newton_rows<R, W, 16, NT, OCC, 2, 0, V4>(DevGeom, DevNum, StageSrc, float, float *, float *, \
-                                                               float *);                                    \
-    template __global__ void k_newton_rows<R, W, 16, NT, OCC, 3, 1, V4>(DevGeom, DevNum, StageSrc, float, float *, float *, \
-                                                               float *);                                    \
-    template __global__ void k_newton_rows<R, W, 16, NT, OCC, 4, 2, V4>(DevGeom, DevNum, StageSrc, float, float *, float *, \
-                                                               float *);
-CA_INST_ROWS(1, 32, 256, 0, true)
-CA_INST_ROWS(1, 32, 512, 0, true)
-CA_INST_ROWS(2, 32, 256, 0, true)
-CA_INST_ROWS(2, 32, 256, 4, true)
-CA_INST_ROWS(2, 64, 256, 0, true)
-CA_INST_ROWS(1, 64, 256, 0, true)
-CA_INST_ROWS(1, 64, 256, 5, true)
-CA_INST_ROWS(1, 64, 512, 6, true)
-CA_INST_ROWS(1, 64, 512, 4, true)
-#undef CA_INST_ROWS

@@ -58,6 +58,8 @@ template <int NF, int NI, bool V4>
 __global__ void k_newton_idiff_pcr(DevGeom g, DevNum n, StageSrc src, float dtg, float *U, float *FI);
 template <int TC, int NF, int NI, bool V4>
 __global__ void k_newton_pcr(DevGeom g, DevNum n, StageSrc src, float dtg, float *U, float *FI, float *Ut);
+template <int R, int W, int TC, int NT, int NF, int NI, bool V4>
+__global__ void k_newton_rows(DevGeom g, DevNum n, StageSrc src, float dtg, float *U, float *FI);
 
 // The final combination of an ARS343 step fused into its last explicit
 // tendency.  The implicit tableau is stiffly accurate (b_j = a_I[4][j]) and

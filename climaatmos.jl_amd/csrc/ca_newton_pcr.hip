@@ -90,6 +90,8 @@ __device__ __forceinline__ void pcr_nbrs(T v, int s, T &u, T &d) {
 
 }  // namespace pcr
 
+#include "ca_column_stage.h"
+
 // NF / NI: compile-time numbers of full-state and implicit-tendency sources
 // (the three ARS343 implicit stages have (2, 0), (3, 1), (4, 2)); -1 reads
 // the counts from src.
@@ -410,18 +412,154 @@ __global__ void __launch_bounds__(256) k_newton_pcr(DevGeom g, DevNum n, StageSr
     }
 }
 
-#define CA_INST_PCR(TC, NF, NI, V4)                                                                   \
-    template __global__ void k_newton_pcr<TC, NF, NI, V4>(DevGeom, DevNum, StageSrc, float, float *, float *, \
+#define CA_INST_PCR(NF, NI, V4)                                                                       \
+    template __global__ void k_newton_pcr<16, NF, NI, V4>(DevGeom, DevNum, StageSrc, float, float *, float *, \
                                                           float *);
-CA_INST_PCR(16, 2, 0, false)
-CA_INST_PCR(16, 3, 1, false)
-CA_INST_PCR(16, 4, 2, false)
-CA_INST_PCR(16, -1, -1, false)
-CA_INST_PCR(16, 2, 0, true)
-CA_INST_PCR(16, 3, 1, true)
-CA_INST_PCR(16, 4, 2, true)
-CA_INST_PCR(16, -1, -1, true)
-CA_INST_PCR(32, 2, 0, false)
-CA_INST_PCR(32, 3, 1, false)
-CA_INST_PCR(32, 4, 2, false)
-CA_INST_PCR(32, -1, -1, false)
+CA_INST_PCR(2, 0, false)
+CA_INST_PCR(3, 1, false)
+CA_INST_PCR(4, 2, false)
+CA_INST_PCR(2, 0, true)
+CA_INST_PCR(3, 1, true)
+CA_INST_PCR(4, 2, true)
+#undef CA_INST_PCR
+
+// The same stage with the column algebra of ca_column_stage.h: 64 / W columns
+// per wavefront, R rows per lane (nlev <= R W).  NT threads, TC columns per tile.
+// W = 32 needs ncol to be a multiple of 16 (every lane pair of columns exists).
+// What bounds it, per stage at h_elem 30, 63 levels (5400 tiles): the VALU is
+// 77% busy with two sources, 55% with six, where the loads are the rest; 155 us
+// averaged over the three stages for k_newton_pcr, 144 here, against 108 for
+// its bytes at the copy rate.  The column algebra takes 590 VALU instructions
+// against 700: see ca_column_stage.h.
+// Shapes (launch_newton_rows chooses):
+//   64 < nlev <= 128   R = 2, W = 64: 54 us per stage at h_elem 16, 90 levels,
+//       against 927 us for the thread-per-column stage, whose 384 wavefronts
+//       walk their columns four times on 1024 SIMDs
+//   32 < nlev < 64     R = 2, W = 32: the tridiagonal solve of two columns costs
+//       one local elimination and five exchanges instead of twice six; 149
+//       VGPRs, 3 wavefronts per SIMD.  23.2 us at h_elem 10, 45 levels against
+//       25.6 for R = 1, W = 64 (28 for k_newton_pcr); 97.6 against 98.9 at
+//       h_elem 26, 45 levels
+//   nlev > 56 and at least 4096 tiles   R = 1, W = 64: its 4 wavefronts per SIMD
+//       win where the lanes are full and the grid is many rounds deep (144 us
+//       against 147 at h_elem 30, 63 levels)
+//   nlev <= 32         R = 1, W = 32, 512 threads (each wavefront two columns,
+//       once): 12.8 us at h_elem 8, 30 levels against 18.6 for k_newton_pcr, 79
+//       us at h_elem 30, 30 levels against 110
+// The tile is unpadded; column c of row k lies at c ^ ((k >> 2) & (TC - 1)), so
+// that the lanes of a wavefront, which read one column down the rows, touch
+// every bank once (TC = 16).
+template <int R, int W, int TC, int NT, int NF, int NI, bool V4>
+__global__ void __launch_bounds__(NT) k_newton_rows(DevGeom g, DevNum n, StageSrc src, float dtg, float *U, float *FI) {
+    constexpr int ROWS = R * W;
+    __shared__ float tU[5][ROWS][TC];
+    __shared__ float tF[3][ROWS][TC];
+    const int nl = g.nlev;
+    const int64_t nC = g.nC, nc = g.ncol;
+    const int col0 = ca_xcd_tile(blockIdx.x, gridDim.x) * TC;
+    const int tid = threadIdx.x;
+    constexpr int VW = V4 ? 4 : 1;
+    auto sw = [](int k, int c) { return c ^ ((k >> 2) & (TC - 1)); };
+    // ---- U~: rows 0 .. nl of the tile (row nl only holds u_3 = 0)
+    for (int idx = tid; idx < (nl + 1) * (TC / VW); idx += NT) {
+        const int r = idx / (TC / VW), c = VW * (idx - r * (TC / VW));
+        const int col = col0 + c;
+        const int64_t q = (int64_t)r * nc + col;
+        const bool ok = col < nc, cen = r < nl, face = r >= 1 && r < nl;
+        if constexpr (V4) {
+            float4 v[5];
+            assemble4<NF, NI>(src, nC, q, ok, cen, face, v);
+            if (cen)
+#pragma unroll
+                for (int p = 0; p < 5; ++p) {
+                    tU[p][r][sw(r, c)] = v[p].x;
+                    tU[p][r][sw(r, c + 1)] = v[p].y;
+                    tU[p][r][sw(r, c + 2)] = v[p].z;
+                    tU[p][r][sw(r, c + 3)] = v[p].w;
+                }
+        } else {
+            float v[5];
+            assemble<NF, NI>(src, nC, q, ok, cen, face, v);
+            if (cen)
+#pragma unroll
+                for (int p = 0; p < 5; ++p) tU[p][r][sw(r, c)] = v[p];
+        }
+    }
+    __syncthreads();
+    // ---- 64 / W columns per wavefront, R rows per lane
+    {
+        constexpr int CPW = 64 / W;
+        const float idtg = 1.0f / dtg;
+        cst::Lev<R> t;
+        cst::lev_load<R>(g, tid & (W - 1), t);
+        for (int cc = tid / W; cc < TC; cc += NT / 64 * CPW) {
+            const int col = col0 + cc;
+            if (col >= nc) break;  // uniform across the wavefront (W = 32: ncol is a multiple of 16)
+            const cst::Met1 m = cst::met1_load(g, n, col);
+            float rho[R], u1[R], u2[R], rhoe[R], u3[R], fr[R], fe[R], fu[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int kc = min(t.k[r], nl - 1), c = sw(kc, cc);
+                rho[r] = tU[0][kc][c];
+                u1[r] = tU[1][kc][c];
+                u2[r] = tU[2][kc][c];
+                rhoe[r] = tU[3][kc][c];
+                u3[r] = t.intF[r] ? tU[4][kc][c] : 0.0f;
+            }
+            cst::newton<R, W>(t, m, n, nl, dtg, idtg, rho, u1, u2, rhoe, u3, fr, fe, fu);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (t.hasC[r]) {
+                    const int k = t.k[r], c = sw(k, cc);
+                    tU[0][k][c] = rho[r];
+                    tU[3][k][c] = rhoe[r];
+                    tU[4][k][c] = u3[r];
+                    tF[0][k][c] = fr[r];
+                    tF[1][k][c] = fe[r];
+                    tF[2][k][c] = fu[r];
+                }
+        }
+    }
+    __syncthreads();
+    // ---- U and F_I out (face nl: zero)
+    for (int idx = tid; idx < (nl + 1) * (TC / VW); idx += NT) {
+        const int r = idx / (TC / VW), c = VW * (idx - r * (TC / VW));
+        const int col = col0 + c;
+        if (col >= nc) continue;
+        const int64_t q = (int64_t)r * nc + col;
+        auto put = [&](float *dst, const float (*tile)[TC], bool in) {
+            if constexpr (V4)
+                *reinterpret_cast<float4 *>(dst) = in ? make_float4(tile[r][sw(r, c)], tile[r][sw(r, c + 1)],
+                                                                    tile[r][sw(r, c + 2)], tile[r][sw(r, c + 3)])
+                                                      : make_float4(0.f, 0.f, 0.f, 0.f);
+            else
+                *dst = in ? tile[r][sw(r, c)] : 0.0f;
+        };
+        if (r < nl) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p) put(U + p * nC + q, tU[p], true);
+            if (FI) {
+                put(FI + q, tF[0], true);
+                put(FI + nC + q, tF[1], true);
+            }
+        }
+        put(U + 4 * nC + q, tU[4], r < nl);
+        if (FI) put(FI + 2 * nC + q, tF[2], r < nl);
+    }
+}
+
+#define CA_INST_ROWS(R, W, TC, NT, V4)                                                                            \
+    template __global__ void k_newton_rows<R, W, TC, NT, 2, 0, V4>(DevGeom, DevNum, StageSrc, float, float *, float *); \
+    template __global__ void k_newton_rows<R, W, TC, NT, 3, 1, V4>(DevGeom, DevNum, StageSrc, float, float *, float *); \
+    template __global__ void k_newton_rows<R, W, TC, NT, 4, 2, V4>(DevGeom, DevNum, StageSrc, float, float *, float *);
+CA_INST_ROWS(1, 32, 16, 512, true)
+CA_INST_ROWS(2, 32, 16, 256, true)
+CA_INST_ROWS(1, 64, 16, 256, true)
+CA_INST_ROWS(2, 64, 16, 256, true)
+CA_INST_ROWS(1, 32, 16, 512, false)
+CA_INST_ROWS(2, 32, 16, 256, false)
+CA_INST_ROWS(1, 64, 16, 256, false)
+CA_INST_ROWS(2, 64, 16, 256, false)
+CA_INST_ROWS(1, 64, 32, 256, true)
+CA_INST_ROWS(1, 64, 32, 256, false)
+#undef CA_INST_ROWS

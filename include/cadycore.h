@@ -230,10 +230,12 @@ ca_status ca_dss_fv(ca_handle *h, const ca_fieldvector *Y, double t, void *strea
 
 /* Launch-schedule knobs (the autotuner's search space).  Results do not
  * depend on them beyond float32 rounding order.
- *   CA_TUNE_NEWTON:         0 = one thread per column (Thomas sweep),
- *                           1 = one wavefront per column, 16-column tiles (PCR),
- *                           2 = one wavefront per column, 32-column tiles (PCR);
- *                           1 and 2 need nlev + 1 <= 64.
+ *   CA_TUNE_NEWTON:         0 = one thread per column (Thomas sweep) below 64
+ *                           and above 128 levels, one wavefront per column,
+ *                           two levels per lane, between (the default there),
+ *                           1 = one or two columns per wavefront, 16-column
+ *                           tiles (PCR), 2 = one column per wavefront,
+ *                           32-column tiles (PCR); 1 and 2 need nlev + 1 <= 64.
  *   CA_TUNE_EXPLICIT_CHUNK: levels per work item of the explicit-tendency
  *                           kernel (0 = whole column).  Setting it sets the
  *                           chunk of ca_step's last explicit launch (which
