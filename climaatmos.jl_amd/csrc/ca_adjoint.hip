@@ -6,7 +6,7 @@
 // gradient-free calibration (calibration/).  Given the cotangent of the
 // state after nsteps steps, k_ensemble_adjoint returns the cotangent of the
 // initial state and of each member's vertical diffusivity D0 and Rayleigh
-// coefficient alpha_w, for the same step k_ensemble takes:
+// coefficient alpha_w, for the same step ca_ensemble_step takes:
 //
 //   forward:  u -> FE_0 = T_E(u); for i = 1..3: U~_i = u + dt sum_j<i (aE FE_j + aI FI_j),
 //             U_i = Newton_i(U~_i) (+ upwind correction), FI_i = (U_i - U~_i) / dtg_i,

@@ -29,11 +29,12 @@ enum KernelId {
     KID_DSS_STATE,
     KID_HOOKS,
     KID_EXPLICIT_FINAL,  // the last explicit tendency with the final combination
+    KID_COLUMN_STEPS,    // whole steps of a column grid
     KID_COUNT
 };
 const char *kKernelNames[KID_COUNT] = {"k_laplacians",   "k_explicit",   "k_dss(tendency)", "k_dss(laplacians)",
                                        "k_newton_stage", "k_final",      "k_dss(state)",    "hook kernels",
-                                       "k_explicit_final"};
+                                       "k_explicit_final", "k_column_steps"};
 
 struct ProfRec {
     int id;
@@ -1019,6 +1020,34 @@ ca_status one_step(ca_handle *h, float *Y, double dt, hipStream_t st, float *rec
     return CA_OK;
 }
 
+// A column grid whose steps run as whole-step launches (k_column_steps): up to
+// 128 levels, no surface fluxes and no implicit diffusion, and no request for
+// the thread-per-column stage.
+bool column_steps_apply(const ca_handle *h) {
+    const int nl = h->g.nlev;
+    if (h->g.nelem > 0 || h->n.sflux || h->n.idiff || nl > 128) return false;
+    return nl >= 64 || h->newton_variant >= 1;
+}
+ca_status column_steps(ca_handle *h, float *Y, double dt, int nsteps, hipStream_t st) {
+    const DevGeom &g = h->g;
+    EnsTab tab;
+    for (int i = 0; i < 4; ++i) {
+        for (int j = 0; j < 4; ++j) {
+            tab.aE[i][j] = (float)h->aE[i][j];
+            tab.aI[i][j] = (float)h->aI[i][j];
+        }
+        tab.b[i] = (float)h->b[i];
+    }
+    {
+        Launch l(h, st, KID_COLUMN_STEPS);
+        if (g.nlev <= 64)
+            k_column_steps<1><<<g.ncol, 64, 0, st>>>(g, ColumnSet{}, h->n, Y, tab, (float)dt, nsteps);
+        else
+            k_column_steps<2><<<g.ncol, 64, 0, st>>>(g, ColumnSet{}, h->n, Y, tab, (float)dt, nsteps);
+    }
+    return check_launch(h, "k_column_steps");
+}
+
 }  // namespace
 
 extern "C" {
@@ -1180,6 +1209,8 @@ ca_status ca_step(ca_handle *h, float *Y, double dt, int32_t nsteps, void *strea
     hipStream_t st = (hipStream_t)stream;
     ca_status s;
     if ((s = poison_work(h, st))) return s;
+    // a column grid's steps filter the state as they load it
+    if (nsteps > 0 && column_steps_apply(h)) return column_steps(h, Y, dt, nsteps, st);
     if ((s = step_prologue(h, Y, st))) return s;
     for (int stp = 0; stp < nsteps; ++stp)
         if ((s = one_step(h, Y, dt, st, nullptr))) return s;
@@ -1200,7 +1231,7 @@ ca_status ca_step_graph(ca_handle *h, float *Y, double dt, int32_t nsteps, void 
         // buffers a stage allocates on first use are allocated before the capture
         if (h->n.idiff && (s = ensure_bands(h))) return s;
         HIPCHK(h, hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
-        ca_status cs = one_step(h, Y, dt, st, nullptr);
+        ca_status cs = column_steps_apply(h) ? column_steps(h, Y, dt, 1, st) : one_step(h, Y, dt, st, nullptr);
         hipGraph_t graph = nullptr;
         const hipError_t e = hipStreamEndCapture(st, &graph);
         if (cs) {

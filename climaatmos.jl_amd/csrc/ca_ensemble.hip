@@ -1,5 +1,5 @@
 // ca_ensemble.hip -- batched single-column ensembles of uneven vertical sizes
-// with per-member parameters, stepped by one persistent launch.
+// with per-member parameters: the step of one member in LDS.
 //
 // Each member is an independent column (ColumnGrid, simulation/grids.jl:110-129)
 // with its own face heights, Rayleigh coefficient alpha_w
@@ -10,13 +10,13 @@
 // the Schur complement on u_3 and the post-Newton upwind correction, and the
 // final combination with the impenetrability filter.
 //
-// Mapping: one workgroup of LPM lanes per member (LPM = 64, 128 or 256, the
-// autotuner picks it), levels strided over the lanes.  The member's state,
-// its four explicit and three implicit stage tendencies and the stage state
-// stay in LDS for all nsteps steps; HBM is read once and written once per
-// launch.  The u_3 Schur system (faces 1 .. nlev - 1; the boundary faces
-// carry u_3 = 0) is solved by parallel cyclic reduction in float64 through
-// LDS.  The member order (as given, or longest first) is a second knob.
+// The forward launch is k_column_steps (ca_column_steps.hip).  The functions here
+// are the same step with a member in a workgroup's LDS, levels strided over LPM
+// lanes: the adjoint (ca_adjoint.hip) re-runs its trajectories with them, so
+// that the stage states its reverse sweep reads are in LDS, and its gradients
+// stay bitwise what they were checked with.  The u_3 Schur system (faces 1 ..
+// nlev - 1; the boundary faces carry u_3 = 0) is solved by parallel cyclic
+// reduction in float64 through LDS.
 #include "ca_kernels.h"
 
 #define CA_ENS_MAXL 128             // centre levels per member, at most
@@ -445,39 +445,3 @@ __device__ void step_once(SharedT<NF> &S, const DevGeom &g, const DevNum &n, con
 }
 
 }  // namespace ens
-
-// Persistent ensemble step: workgroup b steps member order[b] nsteps times.
-template <int LPM, int NF>
-__global__ void __launch_bounds__(LPM) k_ensemble(const DevGeom *__restrict__ mg, DevNum n, const int *__restrict__ order,
-                                                  const int64_t *__restrict__ off, float *__restrict__ Y, EnsTab tab,
-                                                  float dt, int nsteps) {
-    using namespace ens;
-    __shared__ SharedT<NF> S;
-    const int m = order[blockIdx.x];
-    const DevGeom &g = mg[m];
-    const int nl = g.nlev;
-    const int tid = threadIdx.x;
-    float *Ym = Y + off[m];
-    // load, with the impenetrability filter on u_3
-    for (int k = tid; k < nl; k += LPM)
-        for (int p = 0; p < 4; ++p) S.u[p][k] = Ym[p * nl + k];
-    for (int f = tid; f <= nl; f += LPM) S.u[4][f] = (f == 0 || f == nl) ? 0.0f : Ym[4 * nl + f];
-    sync();
-    for (int st = 0; st < nsteps; ++st) step_once<LPM>(S, g, n, tab, dt, tid);
-    for (int k = tid; k < nl; k += LPM)
-        for (int p = 0; p < 4; ++p) Ym[p * nl + k] = S.u[p][k];
-    for (int f = tid; f <= nl; f += LPM) Ym[4 * nl + f] = S.u[4][f];
-}
-
-#define CA_ENS_INST(LPM, NF)                                                                                    \
-    template __global__ void k_ensemble<LPM, NF>(const DevGeom *, DevNum, const int *, const int64_t *, float *, EnsTab, \
-                                                 float, int);
-CA_ENS_INST(64, 33)
-CA_ENS_INST(128, 33)
-CA_ENS_INST(64, 65)
-CA_ENS_INST(128, 65)
-CA_ENS_INST(256, 65)
-CA_ENS_INST(64, 129)
-CA_ENS_INST(128, 129)
-CA_ENS_INST(256, 129)
-#undef CA_ENS_INST

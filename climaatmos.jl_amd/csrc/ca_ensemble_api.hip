@@ -21,7 +21,8 @@ struct ca_ensemble {
     DevGeom *geoms = nullptr;
     int *order[2] = {nullptr, nullptr};  // 0: as given, 1: longest first
     int64_t *doff = nullptr;
-    int lanes = 64;
+    int lanes = 64;           // the lanes knob: of the adjoint's workgroups
+    bool lanes_set = false;   // set by the caller; otherwise ens_adjoint_launch chooses
     int order_kind = 1;
     int nf = CA_ENS_NF;  // LDS face rows per member: 33, 65 or 129, from the tallest member
     std::string err;
@@ -74,22 +75,11 @@ void ens_drop_graph(ca_ensemble *e) {
 }
 
 ca_status ens_launch(ca_ensemble *e, float *Y, float dt, int nsteps, hipStream_t st) {
-    const int *ord = e->order[e->order_kind];
-    const dim3 grid(e->M);
-#define CA_ENS_GO(LPM, NF) k_ensemble<LPM, NF><<<grid, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, Y, e->tab, dt, nsteps)
-    if (e->nf == 33) {  // at most 32 levels: 256 lanes would idle, run 128
-        if (e->lanes == 64) CA_ENS_GO(64, 33);
-        else CA_ENS_GO(128, 33);
-    } else if (e->nf == 65) {
-        if (e->lanes == 64) CA_ENS_GO(64, 65);
-        else if (e->lanes == 128) CA_ENS_GO(128, 65);
-        else CA_ENS_GO(256, 65);
-    } else {
-        if (e->lanes == 64) CA_ENS_GO(64, 129);
-        else if (e->lanes == 128) CA_ENS_GO(128, 129);
-        else CA_ENS_GO(256, 129);
-    }
-#undef CA_ENS_GO
+    const ColumnSet cs{e->geoms, e->order[e->order_kind], e->doff};
+    if (e->nf <= 65)  // at most 64 levels
+        k_column_steps<1><<<e->M, 64, 0, st>>>(DevGeom{}, cs, e->n, Y, e->tab, dt, nsteps);
+    else
+        k_column_steps<2><<<e->M, 64, 0, st>>>(DevGeom{}, cs, e->n, Y, e->tab, dt, nsteps);
     EHIPCHK(e, hipGetLastError());
     return CA_OK;
 }
@@ -258,15 +248,16 @@ ca_status ens_adjoint_launch(ca_ensemble *e, const float *Y0, const float *YbN, 
                              float *Yb0, float *D0b, float *awb, float *ck, float *sg, hipStream_t st) {
     const int *ord = e->order[e->order_kind];
     const dim3 grid(e->M);
-    // lanes: 64 for members of at most 32 levels; otherwise 64 or 128 (the
-    // 256-lane forward schedule runs its adjoint with 128)
+    // lanes: 64 for members of at most 32 levels; otherwise 128 unless the caller
+    // asked for 64
+    const bool l64 = e->lanes_set && e->lanes == 64;
 #define CA_ADJ_GO(LPM, NF)                                                                                       \
     k_ensemble_adjoint<LPM, NF><<<grid, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, Y0, YbN, Yb0, D0b, awb, ck, sg, \
                                                       e->tab, (float)dt, nsteps, every)
     if (e->nf == 33) CA_ADJ_GO(64, 33);
-    else if (e->nf == 65 && e->lanes == 64) CA_ADJ_GO(64, 65);
+    else if (e->nf == 65 && l64) CA_ADJ_GO(64, 65);
     else if (e->nf == 65) CA_ADJ_GO(128, 65);
-    else if (e->lanes == 64) CA_ADJ_GO(64, 129);
+    else if (l64) CA_ADJ_GO(64, 129);
     else CA_ADJ_GO(128, 129);
 #undef CA_ADJ_GO
     EHIPCHK(e, hipGetLastError());
@@ -365,6 +356,7 @@ ca_status ca_ensemble_set_tuning(ca_ensemble *e, int32_t knob, int32_t value) {
     if (knob == CA_ENS_LANES) {
         if (value != 64 && value != 128 && value != 256) return efail(e, CA_ERR_ARG, "lanes per member: 64, 128 or 256");
         e->lanes = value;
+        e->lanes_set = true;
         return CA_OK;
     }
     if (knob == CA_ENS_ORDER) {
@@ -391,38 +383,35 @@ ca_status ca_ensemble_autotune(ca_ensemble *e, const float *Y, double dt, int32_
     EHIPCHK(e, hipMalloc(&work, (size_t)e->S * sizeof(float)));
     hipEvent_t a = nullptr, b = nullptr;
     ca_status s = CA_OK;
-    const int lanes[3] = {64, 128, 256};
     double best = 1e300;
-    int bl = e->lanes, bo = e->order_kind;
+    int bo = e->order_kind;
     if (hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) s = efail(e, CA_ERR_DEVICE, "hipEventCreate");
-    for (int li = 0; li < 3 && s == CA_OK; ++li)
-        for (int o = 0; o < 2 && s == CA_OK; ++o) {
-            e->lanes = lanes[li];
-            e->order_kind = o;
-            double ms_best = 1e300;
-            for (int rep = 0; rep < 2 && s == CA_OK; ++rep) {  // first repetition warms up
-                if (hipMemcpyAsync(work, Y, (size_t)e->S * sizeof(float), hipMemcpyDeviceToDevice, st) != hipSuccess ||
-                    hipEventRecord(a, st) != hipSuccess) {
-                    s = efail(e, CA_ERR_DEVICE, "autotune: copy / event");
-                    break;
-                }
-                if ((s = ens_launch(e, work, (float)dt, nsteps, st))) break;
-                float ms = 0.0f;
-                if (hipEventRecord(b, st) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
-                    hipEventElapsedTime(&ms, a, b) != hipSuccess) {
-                    s = efail(e, CA_ERR_DEVICE, "autotune: timing");
-                    break;
-                }
-                ms_best = std::min(ms_best, (double)ms);
+    // the lanes knob does not change the forward launch: one time per order
+    for (int o = 0; o < 2 && s == CA_OK; ++o) {
+        e->order_kind = o;
+        double ms_best = 1e300;
+        for (int rep = 0; rep < 2 && s == CA_OK; ++rep) {  // first repetition warms up
+            if (hipMemcpyAsync(work, Y, (size_t)e->S * sizeof(float), hipMemcpyDeviceToDevice, st) != hipSuccess ||
+                hipEventRecord(a, st) != hipSuccess) {
+                s = efail(e, CA_ERR_DEVICE, "autotune: copy / event");
+                break;
             }
-            if (times_ms) times_ms[2 * li + o] = ms_best;
-            if (ms_best < best) {
-                best = ms_best;
-                bl = lanes[li];
-                bo = o;
+            if ((s = ens_launch(e, work, (float)dt, nsteps, st))) break;
+            float ms = 0.0f;
+            if (hipEventRecord(b, st) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
+                hipEventElapsedTime(&ms, a, b) != hipSuccess) {
+                s = efail(e, CA_ERR_DEVICE, "autotune: timing");
+                break;
             }
+            ms_best = std::min(ms_best, (double)ms);
         }
-    e->lanes = bl;
+        if (times_ms)
+            for (int li = 0; li < 3; ++li) times_ms[2 * li + o] = ms_best;
+        if (ms_best < best) {
+            best = ms_best;
+            bo = o;
+        }
+    }
     e->order_kind = bo;
     if (a) (void)hipEventDestroy(a);
     if (b) (void)hipEventDestroy(b);

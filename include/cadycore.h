@@ -319,14 +319,15 @@ ca_status ca_ensemble_step(ca_ensemble *e, float *Y, double dt, int32_t nsteps, 
  * nsteps, the schedule and the stream stay the same); stream must not be
  * NULL (the legacy stream cannot be captured) */
 ca_status ca_ensemble_step_graph(ca_ensemble *e, float *Y, double dt, int32_t nsteps, void *stream);
-/* schedule knobs: CA_ENS_LANES = lanes per member (64, 128, 256);
+/* schedule knobs: CA_ENS_LANES = lanes per member of ca_ensemble_adjoint (64, 128;
+ * 256 runs it with 128; the steps take a wavefront per member whatever it is);
  * CA_ENS_ORDER = member-to-workgroup order (0 as given, 1 longest first) */
 typedef enum ca_ens_knob { CA_ENS_LANES = 0, CA_ENS_ORDER = 1 } ca_ens_knob;
 ca_status ca_ensemble_set_tuning(ca_ensemble *e, int32_t knob, int32_t value);
 ca_status ca_ensemble_get_tuning(const ca_ensemble *e, int32_t knob, int32_t *value);
-/* times every schedule on a device copy of Y (Y is not modified), keeps the
- * fastest; times_ms (optional, 6 entries) receives lanes 64/128/256 x order
- * 0/1 in that order */
+/* times both member orders on a device copy of Y (Y is not modified) and keeps
+ * the faster; times_ms (optional, 6 entries) receives lanes 64/128/256 x order
+ * 0/1 in that order (the steps do not depend on the lanes) */
 ca_status ca_ensemble_autotune(ca_ensemble *e, const float *Y, double dt, int32_t nsteps, void *stream,
                                double *times_ms);
 /* new per-member alpha_w and / or D0 (host arrays of nmembers; NULL keeps) */
@@ -339,7 +340,8 @@ ca_status ca_ensemble_set_params(ca_ensemble *e, const double *alpha_w, const do
  * nsteps steps, writes the cotangent of Y0 to Yb0 (ragged, like Y0) and of
  * each member's D0 and alpha_w to D0b, awb (device arrays of nmembers).
  * Recomputes the forward trajectory itself; runs with 64 lanes per member
- * when every member has at most 32 levels or CA_ENS_LANES is 64, else 128. */
+ * when every member has at most 32 levels or CA_ENS_LANES was set to 64, else
+ * 128. */
 ca_status ca_ensemble_adjoint(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int32_t nsteps,
                               int32_t every, float *Yb0, float *D0b, float *awb, void *stream);
 /* ca_ensemble_adjoint without any device allocation.  No counterpart in the
