@@ -73,6 +73,7 @@ struct ca_handle {
     int explicit_chunk = 8;
     int final_chunk = 8;  // the last explicit launch's (the step's final combination)
     int dss_chunk = 8;
+    int hook_chunk = 4;  // of k_implicit_tendency, k_update_jacobian and k_correct
     int lap_chunk = 4;  // levels per work item of k_laplacians
     int dss_kind = 0;  // 0: LDS-staged per element cluster, 1: direct gather
     // reverse mode (ca_step_adjoint and the *_vjp hooks)
@@ -441,7 +442,27 @@ void launch_pcr(const ca_handle *h, const StageSrc &src, float dtg, float *U, fl
         k_newton_pcr<16, 4, 2, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI, Ut);
 }
 
-// The same for a trajectory the reverse mode differentiates (nlev <= 63), which
+// ldiv! from the stored bands (nlev <= 128).  The band planes of ensure_bands are
+// 16-byte aligned with ncol a multiple of 4; two columns share a wavefront on a
+// sphere only, as in the fused stage.
+template <int R, int W>
+void launch_ldiv_rw(const ca_handle *h, float *dY, const float *Rv, hipStream_t st) {
+    const DevGeom &g = h->g;
+    const unsigned nb = cdiv(g.ncol, 16);
+    if (g.ncol % 4 == 0 && ca_al16(Rv) && ca_al16(dY) && ca_al16(h->bands))
+        k_ldiv_rows<R, W, true><<<nb, 256, 0, st>>>(g, h->B, dY, Rv);
+    else
+        k_ldiv_rows<R, W, false><<<nb, 256, 0, st>>>(g, h->B, dY, Rv);
+}
+void launch_ldiv_rows(const ca_handle *h, float *dY, const float *Rv, hipStream_t st) {
+    const int nl = h->g.nlev;
+    if (nl > 64) launch_ldiv_rw<2, 64>(h, dY, Rv, st);
+    else if (!h->n.sphere) launch_ldiv_rw<1, 64>(h, dY, Rv, st);
+    else if (nl > 32) launch_ldiv_rw<2, 32>(h, dY, Rv, st);
+    else launch_ldiv_rw<1, 32>(h, dY, Rv, st);
+}
+
+// The implicit stage of a trajectory the reverse mode differentiates (nlev <= 63), which
 // keeps k_newton_pcr's arithmetic bit for bit; Ut (optional) receives the
 // assembled U~.
 void launch_newton_pcr(const ca_handle *h, const StageSrc &src, float dtg, int i, hipStream_t st, float *U, float *Ut,
@@ -452,6 +473,8 @@ void launch_newton_pcr(const ca_handle *h, const StageSrc &src, float dtg, int i
     else
         launch_pcr<false>(h, src, dtg, U, FI, Ut, st);
 }
+
+inline dim3 hook_grid(const ca_handle *h) { return dim3(cdiv(h->g.ncol, 128), cdiv(h->g.nlev, h->hook_chunk)); }
 
 ca_status ensure_bands(ca_handle *h) {
     if (h->bands) return CA_OK;
@@ -793,6 +816,10 @@ ca_status create_impl(const ca_geometry *geom, const ca_params *par, const ca_co
         // wavefronts of k_explicit a SIMD holds: 3 with vertical diffusion (147
         // VGPRs), 4 without (105, 124 with the final combination)
         h->explicit_chunk = h->final_chunk = explicit_chunk(layer_waves, nl, n.vdiff && !n.idiff ? 3 : 4);
+        // the hook kernels' sweeps: 4 levels measured best at h_elem 16, 63 levels
+        // (17.6, 19.8 and 20.3 us per implicit tendency with 4, 2 and 8), fewer
+        // while that leaves less than 4 wavefronts per SIMD
+        h->hook_chunk = (int)std::min<int64_t>(4, std::max<int64_t>(1, layer_waves * nl / 4096));
         h->adj_chunk = (int)std::min<int64_t>(8, std::max<int64_t>(4, (nl + want - 1) / want));
         h->lap_chunk = (int)std::min<int64_t>(4, std::max<int64_t>(2, (nl + want - 1) / want));
         if (g.ncl > 0) {
@@ -907,17 +934,17 @@ ca_status idiff_stage(ca_handle *h, const StageSrc &src, float dtg, int i, float
     if ((s = ensure_bands(h))) return s;
     float *Ut = h->raw, *T = h->FI[i];
     const unsigned nb = cdiv(h->S, 256);
-    const dim3 cl(cdiv(g.ncol, 128), g.nlev), fl(cdiv(g.ncol, 128), g.nlev + 1);
+    const dim3 cl(cdiv(g.ncol, 128), g.nlev);
     k_stage_sum<<<nb, 256, 0, st>>>(g, src, Ut);
-    k_implicit_tendency<<<fl, 128, 0, st>>>(g, n, T, Ut);
+    k_implicit_tendency<<<hook_grid(h), 128, 0, st>>>(g, n, T, Ut, h->hook_chunk);
     k_vdiff_add<<<cl, 128, 0, st>>>(g, n, Ut, T);
-    k_update_jacobian<<<fl, 128, 0, st>>>(g, n, Ut, dtg, h->B);
+    k_update_jacobian<<<hook_grid(h), 128, 0, st>>>(g, n, Ut, dtg, h->B, h->hook_chunk);
     k_diffusion_jacobian<<<cl, 128, 0, st>>>(g, n, Ut, dtg, h->E);
     k_ldiv_approx<<<cdiv(g.ncol, 128), 128, 0, st>>>(g, h->B, h->E, n.siters, dtg, U, T, h->idw);
     k_newton_update<<<nb, 256, 0, st>>>(g, Ut, U, U);
     const float *C = nullptr;
     if (n.upw != 0) {
-        k_correct<<<cl, 128, 0, st>>>(g, n, T, U);
+        k_correct<<<hook_grid(h), 128, 0, st>>>(g, n, T, U, h->hook_chunk);
         C = T;
     }
     k_stage_finish<<<nb, 256, 0, st>>>(g, Ut, C, dtg, U, h->FI[i]);
@@ -1117,7 +1144,7 @@ ca_status ca_implicit_tendency(ca_handle *h, float *Yt, const float *Y, void *st
     if ((s = poison_work(h, st))) return s;
     {
         Launch l(h, st, KID_HOOKS);
-        k_implicit_tendency<<<dim3(cdiv(g.ncol, 128), g.nlev + 1), 128, 0, st>>>(g, h->n, Yt, Y);
+        k_implicit_tendency<<<hook_grid(h), 128, 0, st>>>(g, h->n, Yt, Y, h->hook_chunk);
         if (h->n.idiff) k_vdiff_add<<<dim3(cdiv(g.ncol, 128), g.nlev), 128, 0, st>>>(g, h->n, Y, Yt);
     }
     return check_launch(h, "k_implicit_tendency");
@@ -1133,7 +1160,7 @@ ca_status ca_update_jacobian(ca_handle *h, const float *Y, double dtgamma, void 
     if (h->poison && (s = fill_words(h, h->bands, 4 * g.nC + 11 * g.nF, kNaNBits, st))) return s;
     {
         Launch l(h, st, KID_HOOKS);
-        k_update_jacobian<<<dim3(cdiv(g.ncol, 128), g.nlev + 1), 128, 0, st>>>(g, h->n, Y, (float)dtgamma, h->B);
+        k_update_jacobian<<<hook_grid(h), 128, 0, st>>>(g, h->n, Y, (float)dtgamma, h->B, h->hook_chunk);
         if (h->n.idiff)
             k_diffusion_jacobian<<<dim3(cdiv(g.ncol, 128), g.nlev), 128, 0, st>>>(g, h->n, Y, (float)dtgamma, h->E);
     }
@@ -1153,7 +1180,9 @@ ca_status ca_ldiv(ca_handle *h, float *dY, const float *R, void *stream) {
             k_ldiv_approx_pcr<<<cdiv(g.ncol, 8), 256, 0, st>>>(g, h->B, h->E, h->n.siters, 1.0f, dY, R);
         else if (h->n.idiff)
             k_ldiv_approx<<<cdiv(g.ncol, 128), 128, 0, st>>>(g, h->B, h->E, h->n.siters, 1.0f, dY, R, h->idw);
-        else
+        else if (g.nlev <= 128 && (h->newton_variant >= 1 || g.nlev >= 64))
+            launch_ldiv_rows(h, dY, R, st);
+        else  // the thread-per-column schedule, or more than 128 levels
             k_ldiv<<<cdiv(g.ncol, 128), 128, 0, st>>>(g, h->B, dY, R, h->scr);
     }
     return check_launch(h, "k_ldiv");
@@ -1167,7 +1196,7 @@ ca_status ca_correct_implicit_advection(ca_handle *h, float *Yt, const float *Y,
     if ((s = poison_work(h, st))) return s;
     {
         Launch l(h, st, KID_HOOKS);
-        k_correct<<<dim3(cdiv(g.ncol, 128), g.nlev), 128, 0, st>>>(g, h->n, Yt, Y);
+        k_correct<<<hook_grid(h), 128, 0, st>>>(g, h->n, Yt, Y, h->hook_chunk);
     }
     return check_launch(h, "k_correct");
 }

@@ -32,54 +32,53 @@ struct FvArg {
     ca_layout lay[5];
 };
 
-constexpr int kTL = 16;  // levels per transpose tile
+constexpr int kTL = 32;  // levels per transpose tile
 constexpr int kTC = 64;  // columns per transpose tile
 
 }  // namespace
 
-// One (16 levels x 64 columns) tile of component p between a strided field
-// and a native plane, through LDS.  dir 0: strided -> native, 1: native ->
-// strided.  The strided side is walked levels fastest when its level stride
-// is 1 (VIJFH), columns fastest otherwise; the native side columns fastest.
-__global__ void __launch_bounds__(256) k_fv_tile(FvArg a, int p, int nl, int ncol, float *plane, int dir) {
+// Tiles of (32 levels x 64 columns) between a FieldVector's strided components
+// p0 .. p0 + gridDim.z - 1 and the native state Y, through LDS.  dir 0: strided ->
+// native, 1: native -> strided.  The strided side is walked levels fastest when
+// its level stride is 1 (VIJFH), columns fastest otherwise; the native side
+// columns fastest.  All components go in one launch: five launches of 5.5 us
+// each moved a state at h_elem 16, 63 levels (62 MB), one takes CA_FV us; 32 levels
+// per tile make each column's piece of a VIJFH array a whole cache line.
+__global__ void __launch_bounds__(256) k_fv_move(FvArg a, int p0, int nlev, int ncol, float *Y, int dir) {
     __shared__ float t[kTL][kTC + 1];
-    const ca_layout L = a.lay[p];
-    const float *base = p < 4 ? a.c : a.f;
+    const int p = p0 + blockIdx.z;
+    const int nl = p < 4 ? nlev : nlev + 1;
     const int k0 = blockIdx.y * kTL, c0 = blockIdx.x * kTC, tid = threadIdx.x;
+    if (k0 >= nl) return;  // the grid covers the face component's rows
+    const ca_layout L = a.lay[p];
+    float *base = p < 4 ? a.c : a.f;
+    float *plane = Y + (int64_t)p * nlev * ncol;
     const bool lev_fast = L.s_v == 1;
-    auto src_index = [&](int lv, int cc) {
+    const bool full = k0 + kTL <= nl && c0 + kTC <= ncol;
+    auto strided = [&](int lv, int cc) {
         const int col = c0 + cc, k = k0 + lv;
         const int h = col >> 4, j = (col >> 2) & 3, i = col & 3;
         return L.offset + (int64_t)k * L.s_v + (int64_t)i * L.s_i + (int64_t)j * L.s_j + (int64_t)h * L.s_h;
     };
-    if (dir == 0) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const bool str = (half == 0) == (dir == 0);  // this half touches the strided side
+        if (half == 1) __syncthreads();
+#pragma unroll
         for (int q = tid; q < kTL * kTC; q += 256) {
-            const int lv = lev_fast ? q % kTL : q / kTC, cc = lev_fast ? q / kTL : q % kTC;
-            if (k0 + lv < nl && c0 + cc < ncol) t[lv][cc] = base[src_index(lv, cc)];
-        }
-        __syncthreads();
-        for (int q = tid; q < kTL * kTC; q += 256) {
-            const int lv = q / kTC, cc = q % kTC;
-            if (k0 + lv < nl && c0 + cc < ncol) plane[(int64_t)(k0 + lv) * ncol + c0 + cc] = t[lv][cc];
-        }
-    } else {
-        for (int q = tid; q < kTL * kTC; q += 256) {
-            const int lv = q / kTC, cc = q % kTC;
-            if (k0 + lv < nl && c0 + cc < ncol) t[lv][cc] = plane[(int64_t)(k0 + lv) * ncol + c0 + cc];
-        }
-        __syncthreads();
-        float *out = p < 4 ? a.c : a.f;
-        for (int q = tid; q < kTL * kTC; q += 256) {
-            const int lv = lev_fast ? q % kTL : q / kTC, cc = lev_fast ? q / kTL : q % kTC;
-            if (k0 + lv < nl && c0 + cc < ncol) out[src_index(lv, cc)] = t[lv][cc];
+            const int lv = str && lev_fast ? q % kTL : q / kTC, cc = str && lev_fast ? q / kTL : q % kTC;
+            if (!full && (k0 + lv >= nl || c0 + cc >= ncol)) continue;
+            float *x = str ? base + strided(lv, cc) : plane + (int64_t)(k0 + lv) * ncol + c0 + cc;
+            if (half == 0) t[lv][cc] = *x;
+            else *x = t[lv][cc];
         }
     }
 }
 
-// zero of one strided component (remaining_tendency!'s Yt_lim .= 0)
-__global__ void __launch_bounds__(256) k_fv_zero(FvArg a, int p, int nl, int ncol) {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
-    if (col >= ncol || k >= nl) return;
+// zero of every strided component (remaining_tendency!'s Yt_lim .= 0)
+__global__ void __launch_bounds__(256) k_fv_zero(FvArg a, int nlev, int ncol) {
+    const int col = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y, p = blockIdx.z;
+    if (col >= ncol || k >= (p < 4 ? nlev : nlev + 1)) return;
     const ca_layout L = a.lay[p];
     float *base = p < 4 ? a.c : a.f;
     const int h = col >> 4, j = (col >> 2) & 3, i = col & 3;
@@ -130,12 +129,8 @@ ca_status fv_staging(ca_handle *h) {
 // strided -> native (dir 0) or native -> strided (dir 1), components [p0, p1)
 ca_status fv_move(ca_handle *h, const ca_fieldvector *v, float *Y, int dir, hipStream_t st, int p0 = 0, int p1 = 5) {
     const DevGeom &g = h->g;
-    const FvArg a = fv_arg(v);
-    for (int p = p0; p < p1; ++p) {
-        const int nl = p < 4 ? g.nlev : g.nlev + 1;
-        k_fv_tile<<<dim3(cdiv(g.ncol, kTC), cdiv(nl, kTL)), 256, 0, st>>>(a, p, nl, g.ncol, Y + (int64_t)p * g.nC,
-                                                                          dir);
-    }
+    k_fv_move<<<dim3(cdiv(g.ncol, kTC), cdiv(g.nlev + 1, kTL), p1 - p0), 256, 0, st>>>(fv_arg(v), p0, g.nlev, g.ncol, Y,
+                                                                                      dir);
     return check_launch(h, dir == 0 ? "FieldVector gather" : "FieldVector scatter");
 }
 
@@ -205,11 +200,7 @@ ca_status ca_remaining_tendency_fv(ca_handle *h, const ca_fieldvector *Yt, const
     const DevGeom &g = h->g;
     // Yt_lim .= 0: the dry model has no limited (tracer) tendencies
     if (Yt_lim) {
-        const FvArg a = fv_arg(Yt_lim);
-        for (int p = 0; p < 5; ++p) {
-            const int nl = p < 4 ? g.nlev : g.nlev + 1;
-            k_fv_zero<<<dim3(cdiv(g.ncol, 256), nl), 256, 0, st>>>(a, p, nl, g.ncol);
-        }
+        k_fv_zero<<<dim3(cdiv(g.ncol, 256), g.nlev + 1, 5), 256, 0, st>>>(fv_arg(Yt_lim), g.nlev, g.ncol);
         if ((s = check_launch(h, "Yt_lim zero"))) return s;
     }
     float *y = nullptr;

@@ -47,10 +47,12 @@ struct FinalSrc {
 
 // column kernels (ca_column.hip)
 __global__ void k_precompute(DevGeom g, DevNum n, float *Y, float *K, float *T, float *p, float *h);
-__global__ void k_implicit_tendency(DevGeom g, DevNum n, float *Yt, const float *Y);
-__global__ void k_update_jacobian(DevGeom g, DevNum n, const float *Y, float dtg, Bands B);
+__global__ void k_implicit_tendency(DevGeom g, DevNum n, float *Yt, const float *Y, int chunk);
+__global__ void k_update_jacobian(DevGeom g, DevNum n, const float *Y, float dtg, Bands B, int chunk);
 __global__ void k_ldiv(DevGeom g, Bands B, float *dY, const float *R, float *scr);
-__global__ void k_correct(DevGeom g, DevNum n, float *Yt, const float *Y);
+template <int R, int W, bool V4>
+__global__ void k_ldiv_rows(DevGeom g, Bands B, float *dY, const float *Rv);
+__global__ void k_correct(DevGeom g, DevNum n, float *Yt, const float *Y, int chunk);
 __global__ void k_newton_stage(DevGeom g, DevNum n, StageSrc src, float dtg, float *U, float *FI, float *scr);
 __global__ void k_ldiv_approx_pcr(DevGeom g, Bands A, DiffBands E, int iters, float rscale, float *dY,
                                   const float *R);

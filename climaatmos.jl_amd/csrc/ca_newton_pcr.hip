@@ -563,3 +563,148 @@ CA_INST_ROWS(2, 64, 16, 256, false)
 CA_INST_ROWS(1, 64, 32, 256, true)
 CA_INST_ROWS(1, 64, 32, 256, false)
 #undef CA_INST_ROWS
+
+// ldiv! from the stored bands: Schur complement on u_3 and back-substitution,
+// BlockArrowheadSolve(rho, rho e_tot; alg2 = BlockLowerTriangularSolve(u_h))
+// (manual_sparse_jacobian.jl:579-584), a tile of 16 columns per workgroup.
+// Thread by (row, 4 columns) forms the Schur rows of a face from the bands and
+// the two centre rows beside it and leaves them in LDS, each wavefront solves
+// its columns there (cst::solve, float64), and the threads substitute back.
+// The boundary rows are diagonal (u_3 = 0 there in the state, so their
+// couplings vanish): x = R / d.
+// What bounds it: the 15 band planes and R in, dY out, and the centre rows read
+// again for the back-substitution, 33 planes; 43 us at h_elem 16, 63 levels (4.8
+// TB/s of them), against 130 us for a thread per column (384 wavefronts on 1024
+// SIMDs, two dependent sweeps of 63 rows).
+// W = 32 needs ncol to be a multiple of 16.  nlev <= R W.
+template <int R, int W, bool V4>
+__global__ void __launch_bounds__(256) k_ldiv_rows(DevGeom g, Bands B, float *dY, const float *Rv) {
+    constexpr int TC = 16, ROWS = R * W, VW = V4 ? 4 : 1;
+    __shared__ float tS[4][ROWS][TC];  // L, D, U, r of the face rows; then x in plane 3
+    struct Vec {
+        float v[VW];
+    };
+    auto ld = [](const float *p, int64_t q) {
+        Vec x;
+        if constexpr (V4) {
+            const float4 y = ca_ld4(p + q);
+            x.v[0] = y.x;
+            x.v[1] = y.y;
+            x.v[2] = y.z;
+            x.v[3] = y.w;
+        } else {
+            x.v[0] = p[q];
+        }
+        return x;
+    };
+    auto stv = [](float *p, int64_t q, const Vec &x) {
+        if constexpr (V4)
+            *reinterpret_cast<float4 *>(p + q) = make_float4(x.v[0], x.v[1], x.v[2], x.v[3]);
+        else
+            p[q] = x.v[0];
+    };
+    const int nl = g.nlev;
+    const int64_t nC = g.nC, nc = g.ncol;
+    const int col0 = ca_xcd_tile(blockIdx.x, gridDim.x) * TC;
+    const int tid = threadIdx.x;
+    auto sw = [](int k, int c) { return c ^ ((k >> 2) & (TC - 1)); };
+    for (int idx = tid; idx < nl * (TC / VW); idx += 256) {
+        const int f = idx / (TC / VW), c = VW * (idx - f * (TC / VW));
+        const int64_t b = (int64_t)f * nc + col0 + c, a = b - nc;
+        if (col0 + c >= nc) {  // beyond the grid: identity rows
+            for (int w = 0; w < VW; ++w) {
+                tS[0][f][sw(f, c + w)] = tS[2][f][sw(f, c + w)] = tS[3][f][sw(f, c + w)] = 0.0f;
+                tS[1][f][sw(f, c + w)] = 1.0f;
+            }
+            continue;
+        }
+        Vec L = ld(B.lo, b), D = ld(B.d, b), U = ld(B.up, b), r = ld(Rv + 4 * nC, b);
+        if (f >= 1) {
+            const Vec r0 = ld(B.Aur0, b), r1 = ld(B.Aur1, b), e0 = ld(B.Aue0, b), e1 = ld(B.Aue1, b);
+            const Vec ra0 = ld(B.Aru0, a), ra1 = ld(B.Aru1, a), ea0 = ld(B.Aeu0, a), ea1 = ld(B.Aeu1, a);
+            const Vec rb0 = ld(B.Aru0, b), rb1 = ld(B.Aru1, b), eb0 = ld(B.Aeu0, b), eb1 = ld(B.Aeu1, b);
+            const Vec Ra = ld(Rv, a), Rb = ld(Rv, b), Ea = ld(Rv + 3 * nC, a), Eb = ld(Rv + 3 * nC, b);
+            const Vec h0a = ld(B.Auh0a, b), h0b = ld(B.Auh0b, b), h1a = ld(B.Auh1a, b), h1b = ld(B.Auh1b, b);
+            const Vec a1 = ld(Rv + nC, a), a2 = ld(Rv + 2 * nC, a), b1 = ld(Rv + nC, b), b2 = ld(Rv + 2 * nC, b);
+#pragma unroll
+            for (int w = 0; w < VW; ++w) {
+                L.v[w] += r0.v[w] * ra0.v[w] + e0.v[w] * ea0.v[w];
+                D.v[w] += r0.v[w] * ra1.v[w] + e0.v[w] * ea1.v[w] + r1.v[w] * rb0.v[w] + e1.v[w] * eb0.v[w];
+                U.v[w] += r1.v[w] * rb1.v[w] + e1.v[w] * eb1.v[w];
+                r.v[w] += r0.v[w] * Ra.v[w] + r1.v[w] * Rb.v[w] + e0.v[w] * Ea.v[w] + e1.v[w] * Eb.v[w];
+                r.v[w] += h0a.v[w] * a1.v[w] + h0b.v[w] * a2.v[w] + h1a.v[w] * b1.v[w] + h1b.v[w] * b2.v[w];
+            }
+        }
+#pragma unroll
+        for (int w = 0; w < VW; ++w) {
+            const int s = sw(f, c + w);
+            tS[0][f][s] = L.v[w];
+            tS[1][f][s] = D.v[w];
+            tS[2][f][s] = U.v[w];
+            tS[3][f][s] = r.v[w];
+        }
+    }
+    __syncthreads();
+    constexpr int CPW = 64 / W;
+    for (int cc = tid / W; cc < TC; cc += 4 * CPW) {
+        double L[R], D[R], U[R], b[R];
+        float x[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int k = R * (tid & (W - 1)) + r, kc = min(k, nl - 1), s = sw(kc, cc);
+            const bool in = k < nl;
+            L[r] = in && k >= 1 ? (double)tS[0][kc][s] : 0.0;
+            D[r] = in ? (double)tS[1][kc][s] : 1.0;
+            U[r] = k + 1 < nl ? (double)tS[2][kc][s] : 0.0;
+            b[r] = in ? (double)tS[3][kc][s] : 0.0;
+        }
+        cst::solve<R, W>(L, D, U, b, x);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int k = R * (tid & (W - 1)) + r;
+            if (k < nl) tS[3][k][sw(k, cc)] = x[r];
+        }
+    }
+    __syncthreads();
+    for (int idx = tid; idx < nl * (TC / VW); idx += 256) {
+        const int k = idx / (TC / VW), c = VW * (idx - k * (TC / VW));
+        if (col0 + c >= nc) continue;
+        const int64_t q = (int64_t)k * nc + col0 + c;
+        const bool top = k == nl - 1;
+        // R is read before dY is written: the two may be the same buffer
+        const Vec a0 = ld(B.Aru0, q), a1 = ld(B.Aru1, q), e0 = ld(B.Aeu0, q), e1 = ld(B.Aeu1, q);
+        const Vec Rr = ld(Rv, q), R1 = ld(Rv + nC, q), R2 = ld(Rv + 2 * nC, q), Re = ld(Rv + 3 * nC, q);
+        Vec x0, x1, yr, y1, y2, ye;
+        if (top) {
+            const Vec rt = ld(Rv + 4 * nC, q + nc), dt = ld(B.d, q + nc);
+#pragma unroll
+            for (int w = 0; w < VW; ++w) x1.v[w] = rt.v[w] / dt.v[w];
+        } else {
+#pragma unroll
+            for (int w = 0; w < VW; ++w) x1.v[w] = tS[3][k + 1][sw(k + 1, c + w)];
+        }
+#pragma unroll
+        for (int w = 0; w < VW; ++w) {
+            x0.v[w] = tS[3][k][sw(k, c + w)];
+            yr.v[w] = a0.v[w] * x0.v[w] + a1.v[w] * x1.v[w] - Rr.v[w];
+            ye.v[w] = e0.v[w] * x0.v[w] + e1.v[w] * x1.v[w] - Re.v[w];
+            y1.v[w] = -R1.v[w];
+            y2.v[w] = -R2.v[w];
+        }
+        stv(dY, q, yr);
+        stv(dY + nC, q, y1);
+        stv(dY + 2 * nC, q, y2);
+        stv(dY + 3 * nC, q, ye);
+        stv(dY + 4 * nC, q, x0);
+        if (top) stv(dY + 4 * nC, q + nc, x1);
+    }
+}
+
+#define CA_INST_LDIV(R, W)                                                               \
+    template __global__ void k_ldiv_rows<R, W, true>(DevGeom, Bands, float *, const float *); \
+    template __global__ void k_ldiv_rows<R, W, false>(DevGeom, Bands, float *, const float *);
+CA_INST_LDIV(1, 32)
+CA_INST_LDIV(2, 32)
+CA_INST_LDIV(1, 64)
+CA_INST_LDIV(2, 64)
+#undef CA_INST_LDIV
