@@ -42,7 +42,7 @@ constexpr int kTC = 64;  // columns per transpose tile
 // native, 1: native -> strided.  The strided side is walked levels fastest when
 // its level stride is 1 (VIJFH), columns fastest otherwise; the native side
 // columns fastest.  All components go in one launch: five launches of 5.5 us
-// each moved a state at h_elem 16, 63 levels (62 MB), one takes CA_FV us; 32 levels
+// each moved a state at h_elem 16, 63 levels (62 MB), one takes 12 us (5.1 TB/s); 32 levels
 // per tile make each column's piece of a VIJFH array a whole cache line.
 __global__ void __launch_bounds__(256) k_fv_move(FvArg a, int p0, int nlev, int ncol, float *Y, int dir) {
     __shared__ float t[kTL][kTC + 1];
@@ -54,24 +54,53 @@ __global__ void __launch_bounds__(256) k_fv_move(FvArg a, int p0, int nlev, int 
     float *base = p < 4 ? a.c : a.f;
     float *plane = Y + (int64_t)p * nlev * ncol;
     const bool lev_fast = L.s_v == 1;
-    const bool full = k0 + kTL <= nl && c0 + kTC <= ncol;
-    auto strided = [&](int lv, int cc) {
-        const int col = c0 + cc, k = k0 + lv;
-        const int h = col >> 4, j = (col >> 2) & 3, i = col & 3;
-        return L.offset + (int64_t)k * L.s_v + (int64_t)i * L.s_i + (int64_t)j * L.s_j + (int64_t)h * L.s_h;
+    // A thread's eight values of the native side are 4 rows apart, of a
+    // level-fastest strided side 8 columns apart: the node index i stays, j
+    // alternates between two values and the element advances every second one.
+    constexpr int N = kTL * kTC / 256;
+    static_assert(kTL == 32 && kTC == 64, "the strided walk steps 8 columns");
+    auto native = [&](int s, int &lv, int &cc) {
+        lv = (tid >> 6) + 4 * s;
+        cc = tid & 63;
+        return plane + (int64_t)(k0 + lv) * ncol + c0 + cc;
     };
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const bool str = (half == 0) == (dir == 0);  // this half touches the strided side
-        if (half == 1) __syncthreads();
-#pragma unroll
-        for (int q = tid; q < kTL * kTC; q += 256) {
-            const int lv = str && lev_fast ? q % kTL : q / kTC, cc = str && lev_fast ? q / kTL : q % kTC;
-            if (!full && (k0 + lv >= nl || c0 + cc >= ncol)) continue;
-            float *x = str ? base + strided(lv, cc) : plane + (int64_t)(k0 + lv) * ncol + c0 + cc;
-            if (half == 0) t[lv][cc] = *x;
-            else *x = t[lv][cc];
+    const int cc0 = tid >> 5, j0 = (cc0 >> 2) & 1;  // cc0 < 8; c0 is a multiple of 64
+    const int64_t st0 = L.offset + (int64_t)(k0 + (tid & 31)) * L.s_v + (int64_t)(cc0 & 3) * L.s_i +
+                        (int64_t)(c0 >> 4) * L.s_h;
+    const int64_t je = st0 + (int64_t)j0 * L.s_j, jo = st0 + (int64_t)(j0 + 2) * L.s_j;
+    auto strided = [&](int s, int &lv, int &cc) {
+        if (lev_fast) {
+            lv = tid & 31;
+            cc = cc0 + 8 * s;
+            return base + ((s & 1) ? jo : je) + (int64_t)(s >> 1) * L.s_h;
         }
+        lv = (tid >> 6) + 4 * s;
+        cc = tid & 63;
+        const int col = c0 + cc, h = col >> 4, jj = (col >> 2) & 3, ii = col & 3;
+        return base + L.offset + (int64_t)(k0 + lv) * L.s_v + (int64_t)ii * L.s_i + (int64_t)jj * L.s_j +
+               (int64_t)h * L.s_h;
+    };
+    auto in = [&](int lv, int cc) { return k0 + lv < nl && c0 + cc < ncol; };
+    float v[N];
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+        int lv, cc;
+        const float *x = dir == 0 ? strided(s, lv, cc) : native(s, lv, cc);
+        v[s] = in(lv, cc) ? *x : 0.0f;
+    }
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+        int lv, cc;
+        if (dir == 0) strided(s, lv, cc);
+        else native(s, lv, cc);
+        t[lv][cc] = v[s];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < N; ++s) {
+        int lv, cc;
+        float *x = dir == 0 ? native(s, lv, cc) : strided(s, lv, cc);
+        if (in(lv, cc)) *x = t[lv][cc];
     }
 }
 
