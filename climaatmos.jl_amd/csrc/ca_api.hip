@@ -90,6 +90,7 @@ struct ca_handle {
     int64_t aw_ck_n = 0;
     // the trajectory ca_step_record last stored (for ca_step_pullback)
     bool rec_valid = false;
+    bool rec_tail = false;  // aw_rec holds the stage records of its last segment
     double rec_dt = 0.0;
     int rec_nsteps = 0, rec_every = 0;
     // debug: fill the scratch no call carries over with NaN at every entry
@@ -820,7 +821,10 @@ ca_status create_impl(const ca_geometry *geom, const ca_params *par, const ca_co
         // (17.6, 19.8 and 20.3 us per implicit tendency with 4, 2 and 8), fewer
         // while that leaves less than 4 wavefronts per SIMD
         h->hook_chunk = (int)std::min<int64_t>(4, std::max<int64_t>(1, layer_waves * nl / 4096));
-        h->adj_chunk = (int)std::min<int64_t>(8, std::max<int64_t>(4, (nl + want - 1) / want));
+        // k_explicit_vjp holds 2 wavefronts per SIMD; the same model: 3.80 against
+        // 3.93 ms per gradient of 8 steps with chunks of 4 at h_elem 8, 30 levels,
+        // 1.77 against 2.04 at h_elem 4, 16 levels (6 steps)
+        h->adj_chunk = explicit_chunk(layer_waves, nl, 2);
         h->lap_chunk = (int)std::min<int64_t>(4, std::max<int64_t>(2, (nl + want - 1) / want));
         if (g.ncl > 0) {
             const int64_t wantd = (1024 + g.ncl - 1) / g.ncl;

@@ -337,9 +337,14 @@ ca_status ca_step_record(ca_handle *h, float *Y, double dt, int32_t nsteps, int3
         if (!all && t % every == 0)
             HIPCHK(h, hipMemcpyAsync(h->aw_ck + (int64_t)(t / every) * S, Y, (size_t)S * sizeof(float),
                                      hipMemcpyDeviceToDevice, st));
-        if ((s = one_step(h, Y, dt, st, all ? h->aw_rec + (int64_t)t * RS : nullptr))) return s;
+        // the last segment's stage records are kept as well: the pullback starts
+        // with it and need not run it again
+        float *rec = all ? h->aw_rec + (int64_t)t * RS : nullptr;
+        if (!all && t / every == nseg - 1) rec = h->aw_rec + (int64_t)(t % every) * RS;
+        if ((s = one_step(h, Y, dt, st, rec))) return s;
     }
     h->rec_valid = true;
+    h->rec_tail = true;
     h->rec_dt = dt;
     h->rec_nsteps = nsteps;
     h->rec_every = every;
@@ -357,8 +362,8 @@ ca_status ca_step_pullback(ca_handle *h, const float *YbN, float *Yb0, float *D0
     const bool all = every == 0;
     const int nseg = all ? 0 : (nsteps + every - 1) / every;
     ca_status s;
-    // with every step's records kept by the forward, they are the input here
-    if ((s = poison_reverse(h, st, !all))) return s;
+    // the records the forward kept (of every step, or of the last segment) are input here
+    if ((s = poison_reverse(h, st, !all && !h->rec_tail))) return s;
     float *Yw = abuf(h, AB_Y);
     if ((s = zero_d0(h, st))) return s;
     HIPCHK(h, hipMemcpyAsync(abuf(h, AB_UB), YbN, (size_t)S * sizeof(float), hipMemcpyDeviceToDevice, st));
@@ -367,12 +372,16 @@ ca_status ca_step_pullback(ca_handle *h, const float *YbN, float *Yb0, float *D0
         for (int j = nsteps - 1; j >= 0; --j)
             if ((s = reverse_step(h, h->aw_rec + (int64_t)j * RS, dt, st))) return s;
     // per segment (last first): re-run it from its checkpoint with stage records, then reverse its steps
+    // (the last one only if its records were overwritten by an earlier pullback)
     for (int sg = nseg - 1; sg >= 0; --sg) {
         const int len = std::min(every, nsteps - sg * every);
-        HIPCHK(h, hipMemcpyAsync(Yw, h->aw_ck + (int64_t)sg * S, (size_t)S * sizeof(float), hipMemcpyDeviceToDevice,
-                                 st));
-        for (int j = 0; j < len; ++j)
-            if ((s = one_step(h, Yw, dt, st, h->aw_rec + j * RS))) return s;
+        if (!(sg == nseg - 1 && h->rec_tail)) {
+            h->rec_tail = false;
+            HIPCHK(h, hipMemcpyAsync(Yw, h->aw_ck + (int64_t)sg * S, (size_t)S * sizeof(float),
+                                     hipMemcpyDeviceToDevice, st));
+            for (int j = 0; j < len; ++j)
+                if ((s = one_step(h, Yw, dt, st, h->aw_rec + j * RS))) return s;
+        }
         for (int j = len - 1; j >= 0; --j)
             if ((s = reverse_step(h, h->aw_rec + j * RS, dt, st))) return s;
     }
