@@ -898,26 +898,30 @@ std::string check_create_args(const ca_geometry *geom, const ca_params *par, con
     return std::string();
 }
 
-// The implicit stage i with implicit vertical diffusion, composed from the
-// hook kernels as ClimaTimeSteppers composes it from the hooks: U~ into
-// h->raw, R = dtg T_imp(U~) (the Newton iteration starts at U~), the Jacobian
-// at U~, dU = solve(A, R) into U, U = U~ - dU, the post-Newton upwind
-// correction at U, and F_I = (U - U~) / dtg with all five components.
-template <bool V4>
-void launch_idiff_pcr(ca_handle *h, const StageSrc &src, float dtg, int i, float *U, hipStream_t st, bool keep_fi) {
+template <int R, int W, bool V4>
+void launch_idiff_v(const ca_handle *h, const StageSrc &src, float dtg, float *U, float *FI, hipStream_t st) {
     const DevGeom &g = h->g;
     const unsigned nb = cdiv(g.ncol, 16);
-    float *FI = keep_fi ? h->FI[i] : nullptr;
-    if (src.nfull == 2 && src.nfi == 0)
-        k_newton_idiff_pcr<2, 0, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI);
-    else if (src.nfull == 3 && src.nfi == 1)
-        k_newton_idiff_pcr<3, 1, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI);
-    else if (src.nfull == 4 && src.nfi == 2)
-        k_newton_idiff_pcr<4, 2, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI);
+    if (src.nfull == 2)
+        k_newton_idiff_rows<R, W, 2, 0, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI);
+    else if (src.nfull == 3)
+        k_newton_idiff_rows<R, W, 3, 1, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI);
     else
-        k_newton_idiff_pcr<-1, -1, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI);
+        k_newton_idiff_rows<R, W, 4, 2, V4><<<nb, 256, 0, st>>>(g, h->n, src, dtg, U, FI);
+}
+template <int R, int W>
+void launch_idiff(const ca_handle *h, const StageSrc &src, float dtg, int i, float *U, float *FI, hipStream_t st) {
+    if (stage_al16(h, src, i, U, nullptr)) launch_idiff_v<R, W, true>(h, src, dtg, U, FI, st);
+    else launch_idiff_v<R, W, false>(h, src, dtg, U, FI, st);
 }
 
+// The implicit stage i with implicit vertical diffusion: the fused stage up to
+// 128 levels (two columns share a wavefront on a sphere only), otherwise, or with
+// the thread-per-column schedule, composed from the hook kernels as
+// ClimaTimeSteppers composes it from the hooks: U~ into h->raw, R = dtg T_imp(U~)
+// (the Newton iteration starts at U~), the Jacobian at U~, dU = solve(A, R) into
+// U, U = U~ - dU, the post-Newton upwind correction at U, and F_I = (U - U~) / dtg
+// with all five components.
 // keep_fi = false: the fused stage does not store F_I (the step's last stage,
 // whose F_I nothing reads); the hook-kernel stage uses F_I as its scratch.
 ca_status idiff_stage(ca_handle *h, const StageSrc &src, float dtg, int i, float *U, hipStream_t st,
@@ -925,14 +929,12 @@ ca_status idiff_stage(ca_handle *h, const StageSrc &src, float dtg, int i, float
     const DevGeom &g = h->g;
     const DevNum &n = h->n;
     ca_status s;
-    if (h->newton_variant >= 1) {  // the fused wavefront-per-column stage (nlev + 1 <= 64)
-        bool v4 = g.ncol % 4 == 0 && ca_al16(U) && ca_al16(h->FI[i]);
-        for (int t = 0; t < src.nfull; ++t) v4 = v4 && ca_al16(src.full[t]);
-        for (int t = 0; t < src.nfi; ++t) v4 = v4 && ca_al16(src.fi[t]);
-        if (v4)
-            launch_idiff_pcr<true>(h, src, dtg, i, U, st, keep_fi);
-        else
-            launch_idiff_pcr<false>(h, src, dtg, i, U, st, keep_fi);
+    if (h->newton_variant >= 1 || (g.nlev >= 64 && g.nlev <= 128)) {  // the fused stage
+        float *FI = keep_fi ? h->FI[i] : nullptr;
+        if (g.nlev > 64) launch_idiff<2, 64>(h, src, dtg, i, U, FI, st);
+        else if (!n.sphere) launch_idiff<1, 64>(h, src, dtg, i, U, FI, st);
+        else if (g.nlev > 32) launch_idiff<2, 32>(h, src, dtg, i, U, FI, st);
+        else launch_idiff<1, 32>(h, src, dtg, i, U, FI, st);
         return check_launch(h, "implicit-diffusion stage");
     }
     if ((s = ensure_bands(h))) return s;

@@ -93,6 +93,12 @@ __device__ __forceinline__ Met1 met1_load(const DevGeom &g, const DevNum &n, int
     return m;
 }
 
+// 1 / d from the hardware reciprocal (1 ulp) and one Newton-Raphson step
+__device__ __forceinline__ float rcp_nr(float d) {
+    const float r = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
+
 // Temperature in float64 from rho e_tot / rho (et), the kinetic energy and Phi
 __device__ __forceinline__ double temperature(const DevNum &n, double et, float K, double Phid) {
     return fmax(n.dT_0 + (et - (double)K - Phid + n.dR_d * n.dT_0) * n.dicv_d, n.dTmin);
@@ -143,6 +149,35 @@ __device__ __forceinline__ void solve(const double (&L)[R], const double (&D)[R]
     const double xe = rd * ca_drcp(Dd);
     x[0] = (float)xe;
     if constexpr (R == 2) x[1] = (float)(ro - Lo * xe - Uo * pcr::dn1(xe));
+}
+
+// correct_implicit_advection_tendency! (implicit_tendency.jl:322-339): the rho e_tot
+// tendency of the upwind minus the central enthalpy flux, from u_3, h (made
+// relative to the lowest cell, which cancels) and rho J of the new state
+template <int R, int W>
+__device__ __forceinline__ void correction(const Lev<R> &t, const Met1 &m, const DevNum &n, int nl, const float (&u3)[R],
+                                           float (&hr)[R], const float (&rJn)[R], float (&corr)[R]) {
+    const float href = first<W>(hr[0]);
+#pragma unroll
+    for (int r = 0; r < R; ++r) hr[r] -= href;
+    float h1[R], h2[R], h4[R], rJm[R], dF[R], dF1[R];
+    prev<R>(hr, h1);
+    prev<R>(h1, h2);
+    next<R>(hr, h4);
+    prev<R>(rJn, rJm);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        dF[r] = 0.0f;
+        if (t.intF[r]) {
+            const float v = u3[r] * t.g0[r];
+            const float up = upwind_product(n.upw, t.k[r], nl, v, n.dt, h2[r], h1[r], hr[r], h4[r]);
+            dF[r] = 0.5f * (rJm[r] + rJn[r]) * (up - v * (0.5f * (h1[r] + hr[r])));
+        }
+    }
+    next<R>(dF, dF1);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        corr[r] = t.hasC[r] ? ((t.upF[r] ? 0.0f - dF1[r] : 0.0f) + dF[r]) * (m.iJh * t.isJ[r]) : 0.0f;
 }
 
 // One implicit stage of one column: U~ (rho, u1, u2, rhoe, u3 with u3 = 0 off
@@ -271,30 +306,355 @@ __device__ __forceinline__ void newton(const Lev<R> &t, const Met1 &m, const Dev
         hr[r] = (float)(et + n.dR_d * temperature(n, et, K, t.Phid[r]));
         rJn[r] = rho[r] * t.sJ[r] * m.Jh;
     }
-    const float href = first<W>(hr[0]);
-#pragma unroll
-    for (int r = 0; r < R; ++r) hr[r] -= href;
-    float h1[R], h2[R], h4[R], rJm[R], dF[R], dF1[R];
-    prev<R>(hr, h1);
-    prev<R>(h1, h2);
-    next<R>(hr, h4);
-    prev<R>(rJn, rJm);
+    float corr[R];
+    correction<R, W>(t, m, n, nl, u3, hr, rJn, corr);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        dF[r] = 0.0f;
-        if (t.intF[r]) {
-            const float v = u3[r] * t.g0[r];
-            const float up = upwind_product(n.upw, t.k[r], nl, v, n.dt, h2[r], h1[r], hr[r], h4[r]);
-            dF[r] = 0.5f * (rJm[r] + rJn[r]) * (up - v * (0.5f * (h1[r] + hr[r])));
+        rhoe[r] += dtg * corr[r];
+        fe[r] += corr[r];
+    }
+}
+
+// ------------------------------------------------ implicit vertical diffusion
+// a tridiagonal system in float32 with N right-hand sides (solved in place):
+// the diffusion blocks, -I minus a diffusion operator, are diagonally dominant.
+// Row elimination as in solve.
+template <int R, int W, int N>
+__device__ __forceinline__ void tri32(const float (&L)[R], const float (&D)[R], const float (&U)[R], float (&b)[N][R]) {
+    float Ls, Ds, Us, r[N], Lo = 0.0f, Uo = 0.0f, ro[N];
+    if constexpr (R == 1) {
+        Ls = L[0];
+        Ds = D[0];
+        Us = U[0];
+#pragma unroll
+        for (int i = 0; i < N; ++i) r[i] = b[i][0];
+    } else {
+        const float iD = rcp_nr(D[1]);
+        Lo = L[1] * iD;
+        Uo = U[1] * iD;
+        const float Lp = pcr::up1(Lo), Up = pcr::up1(Uo);
+        Ds = D[0] - L[0] * Up - U[0] * Lo;
+        Ls = -L[0] * Lp;
+        Us = -U[0] * Uo;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            ro[i] = b[i][1] * iD;
+            r[i] = b[i][0] - L[0] * pcr::up1(ro[i]) - U[0] * ro[i];
         }
     }
-    next<R>(dF, dF1);
+#pragma unroll
+    for (int s = 1; s < W; s <<= 1) {
+        const float iD = rcp_nr(Ds);
+        const float Ln = Ls * iD, Un = Us * iD;
+        float La, Ua, Lb, Ub;
+        pcr::pcr_nbrs(Ln, s, La, Lb);
+        pcr::pcr_nbrs(Un, s, Ua, Ub);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            float ra, rb;
+            pcr::pcr_nbrs(r[i] * iD, s, ra, rb);
+            r[i] = r[i] - Ls * ra - Us * rb;
+        }
+        Ds = Ds - Ls * Ua - Us * Lb;
+        Ls = -Ls * La;
+        Us = -Us * Ub;
+    }
+    const float iD = rcp_nr(Ds);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const float x = r[i] * iD;
+        b[i][0] = x;
+        if constexpr (R == 2) b[i][1] = ro[i] - Lo * x - Uo * pcr::dn1(x);
+    }
+}
+
+// level tables of the diffusion
+template <int R>
+struct Dif {
+    float fJ[R];         // face k: s^2 Jv g^33
+    float s[R], is[R];   // centre k: s and 1 / s on a sphere, 1 on columns
+    float dis[R];        // 1 / s_k - 1 / s_{k-1}
+    float kdec[R];
+};
+template <int R>
+__device__ __forceinline__ void dif_load(const DevGeom &g, const DevNum &n, int lane, Dif<R> &d) {
+    const int nl = g.nlev;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const float corr = t.hasC[r] ? ((t.upF[r] ? 0.0f - dF1[r] : 0.0f) + dF[r]) * (m.iJh * t.isJ[r]) : 0.0f;
-        rhoe[r] += dtg * corr;
-        fe[r] += corr;
+        const int k = R * lane + r, kc = min(k, nl - 1), km = max(kc - 1, 0), kf = min(k, nl);
+        d.fJ[r] = g.sf[kf] * g.sf[kf] * g.Jvf[kf] * g.g33f[kf];
+        const float s = n.sphere ? g.sc[kc] : 1.0f, sm = n.sphere ? g.sc[km] : 1.0f;
+        d.s[r] = s;
+        d.is[r] = 1.0f / s;
+        d.dis[r] = (sm - s) * (1.0f / s) * (1.0f / sm);
+        d.kdec[r] = n.vdk == 0 ? g.kdec[kc] : 1.0f;
     }
+}
+
+// The implicit stage with implicit vertical diffusion: as newton, with the
+// diffusion of rho e_tot and u_h in T_imp, its blocks in the Jacobian, and the
+// approximate block-arrowhead solve (manual_sparse_jacobian.jl:538-578) of
+// n.siters iterations.  U overwrites U~ in all five components.
+// The momentum diffusion is formed on u_i / s: the Cartesian velocity is
+// (u_1 a^1 + u_2 a^2) / s with the column's level-independent basis, and its
+// flux divergence projects back with a_i, whose products with a^j are delta_ij.
+template <int R, int W>
+__device__ __forceinline__ void newton_idiff(const Lev<R> &t, const Dif<R> &df, const Met1 &m, const DevNum &n, int nl,
+                                             float D0, float dtg, float (&rho)[R], float (&u1)[R], float (&u2)[R],
+                                             float (&rhoe)[R], float (&u3)[R]) {
+    float u3m[R], u3p[R];
+    prev<R>(u3, u3m);
+    next<R>(u3, u3p);
+    float h[R], dp[R], thv[R], c1[R], c2[R], iK[R], irho[R];
+    double Td[R], thd[R], Pid[R], Pi7[R];
+    float spd[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        u3p[r] = t.upF[r] ? u3p[r] : 0.0f;
+        c1[r] = t.is2[r] * (m.gu11 * u1[r] + m.gu12 * u2[r]);
+        c2[r] = t.is2[r] * (m.gu12 * u1[r] + m.gu22 * u2[r]);
+        const float uu = u1[r] * c1[r] + u2[r] * c2[r];
+        spd[r] = sqrtf(uu);
+        const float K = 0.5f * (uu + 0.5f * (u3[r] * t.g0[r] * u3[r] + u3p[r] * t.gp[r] * u3p[r]));
+        const double et = (double)rhoe[r] * ca_drcp((double)rho[r]);
+        Td[r] = temperature(n, et, K, t.Phid[r]);
+        const double pd = (double)rho[r] * n.dR_d * Td[r];
+        iK[r] = (float)pd;  // the pressure; becomes 1 / K_h below
+        Pid[r] = ca_dexner(n, pd * n.dp0inv);
+        h[r] = (float)(et + n.dR_d * Td[r]);
+        thv[r] = (float)Td[r] * ca_rcp((float)Pid[r]);
+        Pi7[r] = ca_dpow7(Pid[r]);
+        thd[r] = (Td[r] - (n.dTmr + (n.dTsr - n.dTmr) * Pi7[r])) * ca_drcp(Pid[r]);
+        dp[r] = n.kap * (n.T_0 * n.cp_d - K - t.Phic[r]);
+        irho[r] = rcp_nr(rho[r]);
+    }
+    const float spd0 = n.vdk == 1 ? first<W>(spd[0]) : 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {  // ca_Kc
+        float K = D0 * df.kdec[r];
+        if (n.vdk == 1) {
+            const float p = iK[r], x = (85000.0f - p) * 1.0e-4f;
+            K = n.CE * spd0 * n.za * (p > 85000.0f ? 1.0f : expf(-(x * x)));
+        }
+        iK[r] = 1.0f / fmaxf(K, 1.1920929e-07f);
+    }
+    float ra[R], ha[R], dpa[R], thva[R], iKa[R], u1a[R], u2a[R], c1a[R], c2a[R], irm[R], irp[R];
+    double Tda[R], thda[R], Pia[R], Pi7a[R];
+    prev<R>(rho, ra);
+    prev<R>(h, ha);
+    prev<R>(dp, dpa);
+    prev<R>(thv, thva);
+    prev<R>(iK, iKa);
+    prev<R>(u1, u1a);
+    prev<R>(u2, u2a);
+    prev<R>(c1, c1a);
+    prev<R>(c2, c2a);
+    prev<R>(irho, irm);
+    next<R>(irho, irp);
+    prev<R>(Td, Tda);
+    prev<R>(thd, thda);
+    prev<R>(Pid, Pia);
+    prev<R>(Pi7, Pi7a);
+    float q[R], qh[R], cf[R], Fs[R], F1[R], F2[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {  // faces: advective and diffusive fluxes, 0 off the interior
+        q[r] = qh[r] = cf[r] = Fs[r] = F1[r] = F2[r] = 0.0f;
+        if (t.intF[r]) {
+            q[r] = 0.5f * (ra[r] * t.sJm[r] + rho[r] * t.sJ[r]) * m.Jh * t.g0[r];
+            qh[r] = q[r] * (0.5f * (ha[r] + h[r]));
+            const float rK = (0.5f * (ra[r] + rho[r])) * (1.0f / (0.5f * (iKa[r] + iK[r])));
+            cf[r] = m.Jh * df.fJ[r] * rK;
+            // s_d(k) - s_d(k - 1) from the float64 temperatures, u_i / s from the
+            // differences plus the metric step: no difference of near equals
+            Fs[r] = -cf[r] * (n.cp_d * (float)(Td[r] - Tda[r]) + (float)t.dPhid[r]);
+            F1[r] = -cf[r] * ((u1[r] - u1a[r]) * df.is[r] + u1a[r] * df.dis[r]);
+            F2[r] = -cf[r] * ((u2[r] - u2a[r]) * df.is[r] + u2a[r] * df.dis[r]);
+        }
+    }
+    float qm[R], qhm[R], qp[R], qhp[R], cfp[R], Fsp[R], F1p[R], F2p[R];
+    prev<R>(q, qm);
+    prev<R>(qh, qhm);
+    next<R>(q, qp);
+    next<R>(qh, qhp);
+    next<R>(cf, cfp);
+    next<R>(Fs, Fsp);
+    next<R>(F1, F1p);
+    next<R>(F2, F2p);
+    const float kcv = n.cp_d / n.cv_d;
+    float a0[R], a1[R], e0[R], e1[R], Rr[R], Re[R], elo[R], ed[R], eup[R], hlo[R], hd[R], hup[R], bh[2][R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const bool up = t.upF[r];
+        qp[r] = up ? qp[r] : 0.0f;
+        qhp[r] = up ? qhp[r] : 0.0f;
+        const float iJ = m.iJh * t.isJ[r], c = dtg * iJ;
+        a0[r] = c * q[r];
+        a1[r] = -c * qp[r];
+        e0[r] = c * qh[r];
+        e1[r] = -c * qhp[r];
+        Rr[r] = -c * (qp[r] * u3p[r] - q[r] * u3[r]);
+        Re[r] = -c * ((qhp[r] * u3p[r] - qh[r] * u3[r]) + ((up ? Fsp[r] : 0.0f) - Fs[r]));
+        const float ch = -c * df.s[r] * irho[r];
+        bh[0][r] = ch * ((up ? F1p[r] : 0.0f) - F1[r]);
+        bh[1][r] = ch * ((up ? F2p[r] : 0.0f) - F2[r]);
+        const float dlo = cf[r] * c, dup = up ? cfp[r] * c : 0.0f, dd = -(dlo + dup);
+        elo[r] = t.intF[r] ? dlo * (kcv * irm[r]) : 0.0f;
+        ed[r] = dd * (kcv * irho[r]) - 1.0f;
+        eup[r] = up ? dup * (kcv * irp[r]) : 0.0f;
+        hlo[r] = irho[r] * dlo;
+        hd[r] = irho[r] * dd - 1.0f;
+        hup[r] = irho[r] * dup;
+        if (!t.hasC[r]) {  // beyond the column: identity rows
+            a0[r] = a1[r] = e0[r] = e1[r] = Rr[r] = Re[r] = bh[0][r] = bh[1][r] = 0.0f;
+            elo[r] = eup[r] = hlo[r] = hup[r] = 0.0f;
+            ed[r] = hd[r] = 1.0f;
+        }
+    }
+    // y_e = inv(A_ee) b_e
+    float ye[1][R], yea[R], eda[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) ye[0][r] = Re[r];
+    tri32<R, W, 1>(elo, ed, eup, ye);
+    prev<R>(ye[0], yea);
+    prev<R>(ed, eda);
+    // face rows, b_w' = b_w - A_wrho y_rho - A_we y_e, and the preconditioner's u_3
+    // block with diag(A_ee) in place of A_ee
+    float r0[R], r1[R], ef[R], lo[R], dd[R], up_[R], h0a[R], h0b[R], h1a[R], h1b[R], bw[R];
+    double Pl[R], Pd[R], Pu[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        r0[r] = r1[r] = ef[r] = lo[r] = up_[r] = h0a[r] = h0b[r] = h1a[r] = h1b[r] = bw[r] = 0.0f;
+        dd[r] = 1.0f;
+        Pl[r] = Pu[r] = 0.0;
+        Pd[r] = 1.0;
+        if (t.intF[r]) {
+            const float cm = dtg * (m.iJh * t.isJm[r]);
+            const bool two = t.k[r] >= 2;
+            const float q0 = two ? qm[r] : 0.0f, qh0 = two ? qhm[r] : 0.0f, w0 = two ? u3m[r] : 0.0f;
+            const float pa0 = cm * q0, pa1 = -cm * q[r], pe0 = cm * qh0, pe1 = -cm * qh[r];
+            const float pRr = -cm * (q[r] * u3[r] - q0 * w0);
+            const float pg = ca_rcp(0.5f * (ra[r] + rho[r]));
+            const double dPid = Pid[r] - Pia[r];
+            const float buoy = n.cp_d * (0.5f * (thva[r] + thv[r])) * (float)dPid * pg;
+            r0[r] = dtg * (pg * dpa[r] + 0.5f * buoy);
+            r1[r] = dtg * (0.5f * buoy - pg * dp[r]);
+            ef[r] = dtg * (pg * n.kap);
+            const float ka = -dtg * n.kap * ra[r] * pg, kb = dtg * n.kap * rho[r] * pg;
+            const float beta = m.aw * t.zf[r];
+            lo[r] = ka * (0.5f * w0 * t.gm[r]);
+            dd[r] = (ka + kb) * (0.5f * u3[r] * t.g0[r]) - dtg * beta - 1.0f;
+            up_[r] = kb * (0.5f * u3p[r] * t.gp[r]);
+            h0a[r] = ka * c1a[r];
+            h0b[r] = ka * c2a[r];
+            h1a[r] = kb * c1[r];
+            h1b[r] = kb * c2[r];
+            const double sg = dPid * ca_drcp(Pia[r] + Pid[r]), s2 = sg * sg;
+            double z = 1.0 / 19.0;
+#pragma unroll
+            for (int j = 17; j >= 1; j -= 2) z = fma(z, s2, 1.0 / j);
+            const double dPhr =
+                -n.dcp_d * (n.dTmr * (2.0 * sg * z) + (n.dTsr - n.dTmr) * (1.0 / 7.0) * (Pi7[r] - Pi7a[r]));
+            const float pgf = (float)(-((t.dPhid[r] - dPhr) + n.dcp_d * (0.5 * (thda[r] + thd[r])) * dPid));
+            bw[r] = dtg * (pgf - beta * u3[r]) + r0[r] * pRr + r1[r] * Rr[r] - ef[r] * (yea[r] - ye[0][r]);
+            const float ia = ef[r] * rcp_nr(eda[r]), ib = ef[r] * rcp_nr(ed[r]);
+            Pl[r] = lo[r] + r0[r] * pa0 - ia * pe0;
+            Pd[r] = dd[r] + r0[r] * pa1 + r1[r] * a0[r] - ia * pe1 + ib * e0[r];
+            Pu[r] = up_[r] + r1[r] * a1[r] + ib * e1[r];
+        }
+    }
+    float xh1[R], xh2[R], xw[R], xwp[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) xh1[r] = xh2[r] = xw[r] = 0.0f;
+    for (int it = 0; it < n.siters; ++it) {
+        float rh[2][R], rw[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            rh[0][r] = bh[0][r];
+            rh[1][r] = bh[1][r];
+            rw[r] = bw[r];
+        }
+        if (it > 0) {  // r = b' - S x
+            float x1m[R], x1p[R], x2m[R], x2p[R], xwm[R], mm[1][R], mma[R], pA[R], pAa[R];
+            prev<R>(xh1, x1m);
+            next<R>(xh1, x1p);
+            prev<R>(xh2, x2m);
+            next<R>(xh2, x2p);
+            prev<R>(xw, xwm);
+            next<R>(xw, xwp);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {  // hlo, hup and the couplings are 0 where a neighbour is missing
+                const float wp = t.upF[r] ? xwp[r] : 0.0f;
+                rh[0][r] -= hd[r] * xh1[r] + (t.intF[r] ? hlo[r] * x1m[r] : 0.0f) + (t.upF[r] ? hup[r] * x1p[r] : 0.0f);
+                rh[1][r] -= hd[r] * xh2[r] + (t.intF[r] ? hlo[r] * x2m[r] : 0.0f) + (t.upF[r] ? hup[r] * x2p[r] : 0.0f);
+                mm[0][r] = e0[r] * xw[r] + e1[r] * wp;  // A_ew x_w
+                pA[r] = a0[r] * xw[r] + a1[r] * wp;     // A_rho,w x_w
+            }
+            tri32<R, W, 1>(elo, ed, eup, mm);
+            prev<R>(mm[0], mma);
+            prev<R>(pA, pAa);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (t.intF[r]) {
+                    float sx = dd[r] * xw[r] + (t.k[r] >= 2 ? lo[r] * xwm[r] : 0.0f) + (t.upF[r] ? up_[r] * xwp[r] : 0.0f);
+                    sx += h0a[r] * x1m[r] + h0b[r] * x2m[r] + h1a[r] * xh1[r] + h1b[r] * xh2[r];
+                    sx += r0[r] * pAa[r] + r1[r] * pA[r] - ef[r] * (mma[r] - mm[0][r]);
+                    rw[r] -= sx;
+                }
+        }
+        // z_h = inv(A_hh) r_h (two components); z_w = inv(P_ww) (r_w - A_wh z_h)
+        tri32<R, W, 2>(hlo, hd, hup, rh);
+        float z1m[R], z2m[R], zw[R];
+        double rd[R];
+        prev<R>(rh[0], z1m);
+        prev<R>(rh[1], z2m);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (t.intF[r]) rw[r] -= h0a[r] * z1m[r] + h0b[r] * z2m[r] + h1a[r] * rh[0][r] + h1b[r] * rh[1][r];
+            rd[r] = rw[r];
+        }
+        solve<R, W>(Pl, Pd, Pu, rd, zw);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            xh1[r] += rh[0][r];
+            xh2[r] += rh[1][r];
+            xw[r] += t.intF[r] ? zw[r] : 0.0f;
+        }
+    }
+    next<R>(xw, xwp);
+    float xe[1][R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        xwp[r] = t.upF[r] ? xwp[r] : 0.0f;
+        xe[0][r] = Re[r] - (e0[r] * xw[r] + e1[r] * xwp[r]);
+    }
+    tri32<R, W, 1>(elo, ed, eup, xe);
+    // Newton update
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        rho[r] -= a0[r] * xw[r] + a1[r] * xwp[r] - Rr[r];
+        u1[r] -= xh1[r];
+        u2[r] -= xh2[r];
+        rhoe[r] -= xe[0][r];
+        u3[r] -= xw[r];  // 0 off the interior faces
+    }
+    if (n.upw == 0) return;
+    // post-Newton upwind correction at the new state
+    float hr[R], rJn[R];
+    next<R>(u3, u3p);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float w1 = t.upF[r] ? u3p[r] : 0.0f;
+        const float d1 = t.is2[r] * (m.gu11 * u1[r] + m.gu12 * u2[r]);
+        const float d2 = t.is2[r] * (m.gu12 * u1[r] + m.gu22 * u2[r]);
+        const float K = 0.5f * ((u1[r] * d1 + u2[r] * d2) + 0.5f * (u3[r] * t.g0[r] * u3[r] + w1 * t.gp[r] * w1));
+        const double et = (double)rhoe[r] * ca_drcp((double)rho[r]);
+        hr[r] = (float)(et + n.dR_d * temperature(n, et, K, t.Phid[r]));
+        rJn[r] = rho[r] * t.sJ[r] * m.Jh;
+    }
+    float corr[R];
+    correction<R, W>(t, m, n, nl, u3, hr, rJn, corr);
+#pragma unroll
+    for (int r = 0; r < R; ++r) rhoe[r] += dtg * corr[r];
 }
 
 }  // namespace cst

@@ -270,18 +270,12 @@ __global__ void __launch_bounds__(128) k_ldiv_approx(DevGeom g, Bands A, DiffBan
 }
 
 // ---------------------------------------------------------------------------
-// The whole implicit stage with implicit diffusion as one kernel, built like
-// k_newton_pcr: a workgroup assembles a tile of 16 columns into LDS, each
-// wavefront then takes one column with lane k = centre k and face k, and the
-// results leave through LDS.  Per column: U~, T_imp (advection, u_3 pressure
-// gradient and buoyancy, Rayleigh, and the vertical diffusion of rho e_tot and
-// u_h), the manual Jacobian and the diffusion blocks, the approximate
-// arrowhead solve, the Newton update, the upwind correction and
-// F_I = (U - U~) / dtg, all in registers.  The tridiagonal solves are parallel
-// cyclic reductions across the 64 lanes: float32 for the diffusion blocks
-// A_ee and A_hh (-I minus a diffusion operator: diagonally dominant), float64
-// for the u_3 Schur complement (stiff, as in the dry stage).  Same algebra as
-// the hook kernels above; the order of the roundings differs.
+// The arrowhead solve of one column held by a wavefront, lane k = centre k and
+// face k, from stored bands (the hook ca_ldiv): the tridiagonal solves are
+// parallel cyclic reductions across the 64 lanes, float32 for the diffusion
+// blocks A_ee and A_hh (-I minus a diffusion operator: diagonally dominant),
+// float64 for the u_3 Schur complement (stiff, as in the dry stage).  The fused
+// stage below solves the same system with cst::newton_idiff.
 
 namespace idp {
 
@@ -444,308 +438,130 @@ __device__ __forceinline__ Sol arrowhead_solve(int k, int nl, bool hasC, bool in
 
 }  // namespace idp
 
-// V4: 16-byte row accesses in phases 1 and 3 (ncol a multiple of 4 and every
-// plane 16-byte aligned; the host checks).  Compiled for 3 wavefronts per
-// SIMD (at most 168 VGPRs: 167 and no spill with V4; the 4-byte fallback
-// spills 36-52 bytes).
-template <int NF, int NI, bool V4>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8))) k_newton_idiff_pcr(DevGeom g, DevNum n, StageSrc src, float dtg, float *U, float *FI) {
-    constexpr int TC = 16, R = TC + 1;
-    __shared__ float tU[5][64][R];
-    __shared__ float tF[5][64][R];
+// The fused stage, the column in a wavefront's registers (cst::newton_idiff): tile,
+// row and column mapping as k_newton_rows.  F_I carries all five components.
+// What bounds it: the column algebra.  With one level per lane and one column
+// per wavefront (the same algebra on CV structures) the four float32 and one
+// float64 reductions were six exchange steps each per column; two levels per
+// lane and two columns per wavefront take one local elimination and five steps
+// for both, face quantities are formed once, and the momentum diffusion needs
+// two components instead of three Cartesian ones.  Per stage, averaged over the
+// three: h_elem 30, 63 levels 338 -> 219 us (R = 1, W = 64: 216; at h_elem 16, 45
+// levels 68 against 62), h_elem 8, 30 levels 37 -> 20; h_elem 16, 90 levels, where
+// the stage was a sequence of thread-per-column kernels, 1602 -> 123.
+template <int R, int W, int NF, int NI, bool V4>
+__global__ void __launch_bounds__(256) k_newton_idiff_rows(DevGeom g, DevNum n, StageSrc src, float dtg, float *U,
+                                                           float *FI) {
+    constexpr int TC = 16, ROWS = R * W, VW = V4 ? 4 : 1;
+    __shared__ float tU[5][ROWS][TC];
+    __shared__ float tF[5][ROWS][TC];
     const int nl = g.nlev;
     const int64_t nC = g.nC, nc = g.ncol;
     const int col0 = ca_xcd_tile(blockIdx.x, gridDim.x) * TC;
     const int tid = threadIdx.x;
-    const int nf = NF >= 0 ? NF : src.nfull;
-    const int ni = NI >= 0 ? NI : src.nfi;
-
-    // ---- phase 1: U~ = sum cf full + sum ci F_I over all five components
-    // (F_I carries u_h here), u_3 zero on the boundary faces
-    if constexpr (V4) {
-        for (int idx = tid; idx < 16 * TC; idx += 256) {
-            const int r = idx / (TC / 4), c4 = 4 * (idx - r * (TC / 4));
-            const int col = col0 + c4;
-            const int64_t q = (int64_t)r * nc + col;
-            const bool ok = col < nc;
+    auto sw = [](int k, int c) { return c ^ ((k >> 2) & (TC - 1)); };
+    // ---- U~ = sum cf full + sum ci F_I over all five components, u_3 zero on the boundary faces
+    for (int idx = tid; idx < nl * (TC / VW); idx += 256) {
+        const int r = idx / (TC / VW), c = VW * (idx - r * (TC / VW));
+        const int64_t q = (int64_t)r * nc + col0 + c;
+        const bool ok = col0 + c < nc;
 #pragma unroll
-            for (int comp = 0; comp < 5; ++comp) {
-                const bool in = ok && (comp < 4 ? r < nl : (r >= 1 && r <= nl - 1));
+        for (int p = 0; p < 5; ++p) {
+            const bool in = ok && (p < 4 || r >= 1);
+            const int64_t o = p * nC + q;
+            if constexpr (V4) {
                 float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 if (in) {
-                    const int64_t o = comp * nC + q;
 #pragma unroll
-                    for (int t = 0; t < (NF >= 0 ? NF : CA_MAX_SRC); ++t)
-                        if (t < nf) ca_fma4(src.cf[t], ca_ld4(src.full[t] + o), v);
+                    for (int t = 0; t < NF; ++t) ca_fma4(src.cf[t], ca_ld4(src.full[t] + o), v);
 #pragma unroll
-                    for (int t = 0; t < (NI >= 0 ? NI : CA_MAX_SRC); ++t)
-                        if (t < ni) ca_fma4(src.ci[t], ca_ld4(src.fi[t] + o), v);
+                    for (int t = 0; t < NI; ++t) ca_fma4(src.ci[t], ca_ld4(src.fi[t] + o), v);
                 }
-                tU[comp][r][c4] = v.x;
-                tU[comp][r][c4 + 1] = v.y;
-                tU[comp][r][c4 + 2] = v.z;
-                tU[comp][r][c4 + 3] = v.w;
-            }
-        }
-    } else
-    for (int idx = tid; idx < 64 * TC; idx += 256) {
-        const int r = idx / TC, cc = idx - r * TC;
-        const int col = col0 + cc;
-        const int64_t q = (int64_t)r * nc + col;
-        const bool ok = col < nc;
-#pragma unroll
-        for (int comp = 0; comp < 5; ++comp) {
-            const bool in = ok && (comp < 4 ? r < nl : (r >= 1 && r <= nl - 1));
-            float v = 0.0f;
-            if (in) {
-                const int64_t o = comp * nC + q;
-#pragma unroll
-                for (int t = 0; t < (NF >= 0 ? NF : CA_MAX_SRC); ++t)
-                    if (t < nf) v = fmaf(src.cf[t], src.full[t][o], v);
-#pragma unroll
-                for (int t = 0; t < (NI >= 0 ? NI : CA_MAX_SRC); ++t)
-                    if (t < ni) v = fmaf(src.ci[t], src.fi[t][o], v);
-            }
-            tU[comp][r][cc] = v;
-        }
-    }
-    __syncthreads();
-
-    // ---- phase 2: one column per wavefront
-    const int k = tid & 63;
-    const int wid = tid >> 6;
-    const bool hasC = k < nl;
-    const bool intF = k >= 1 && k <= nl - 1;
-    const bool isF = k <= nl;
-    const int kc = hasC ? k : nl - 1;
-    const int kf = isF ? k : nl;
-    const float g33 = g.g33f[kf];
-    const float g33p = g.g33f[kc + 1];
-    const float kcv = n.cp_d / n.cv_d;
-    const float idtg = 1.0f / dtg;
-    for (int cc = wid; cc < TC; cc += 4) {
-        const int col = col0 + cc;
-        if (col >= nc) break;  // uniform across the wavefront
-        const float rho = tU[0][kc][cc], u1 = tU[1][kc][cc], u2 = tU[2][kc][cc], rhoe = tU[3][kc][cc];
-        const float u3 = intF ? tU[4][k][cc] : 0.0f;
-        const float u3p = pcr::dn1(u3);
-        const float u3m = pcr::up1(u3);
-        const CV c = cv_make(g, n, kc, col, rho, u1, u2, rhoe, u3, hasC ? u3p : 0.0f);
-        const float rJ = c.rho * c.J;
-        const float rJm = pcr::up1(rJ), hm = pcr::up1(c.h);
-        const float rJp = pcr::dn1(rJ), hp = pcr::dn1(c.h);
-        // centre row k: A(rho,u3), A(rhoe,u3) and the advective residuals
-        float a0 = 0.0f, a1 = 0.0f, e0 = 0.0f, e1 = 0.0f, Rr = 0.0f, Te = 0.0f;
-        if (hasC) {
-            float Fm = 0.0f, Fp = 0.0f, Hm = 0.0f, Hp = 0.0f;
-            if (k >= 1) {
-                const float rJf = 0.5f * (rJm + rJ);
-                a0 = dtg * (rJf * c.iJ) * g33;
-                e0 = a0 * (0.5f * (hm + c.h));
-                Fm = rJf * (u3 * g33);
-                Hm = Fm * (0.5f * (hm + c.h));
-            }
-            if (k + 1 <= nl - 1) {
-                const float rJf = 0.5f * (rJ + rJp);
-                a1 = dtg * (-rJf * c.iJ) * g33p;
-                e1 = a1 * (0.5f * (c.h + hp));
-                Fp = rJf * (u3p * g33p);
-                Hp = Fp * (0.5f * (c.h + hp));
-            }
-            Rr = dtg * (-(Fp - Fm) * c.iJ);
-            Te = -(Hp - Hm) * c.iJ;
-        }
-        // centre k - 1 (lane k - 1)
-        CV a;
-        a.rho = pcr::up1(c.rho);
-        a.u1 = pcr::up1(c.u1);
-        a.u2 = pcr::up1(c.u2);
-        a.K = pcr::up1(c.K);
-        a.Td = pcr::up1(c.Td);
-        a.pd = pcr::up1(c.pd);
-        a.Pid = pcr::up1(c.Pid);
-        a.T = (float)a.Td;
-        a.p = (float)a.pd;
-        a.Pi = (float)a.Pid;
-        a.ct1 = pcr::up1(c.ct1);
-        a.ct2 = pcr::up1(c.ct2);
-        // vertical diffusion: fluxes through face k, the tendency of centre k
-        // the centre's diffusivity, and the lowest centre's wind speed (lane 0)
-        const float spd0 = n.vdk == 1 ? pcr::lane0(sqrtf(c.u1 * c.ct1 + c.u2 * c.ct2)) : 0.0f;
-        const float Kd = ca_Kc(g, n, col, kc, c.p, spd0);
-        const float Kdm = pcr::up1(Kd), Kdp = pcr::dn1(Kd);
-        float Fs = 0.0f, Fu0 = 0.0f, Fu1 = 0.0f, Fu2 = 0.0f;
-        if (intF) vdiff_face(g, n, col, k, a, c, Kdm, Kd, Fs, Fu0, Fu1, Fu2);
-        const float Fs1 = pcr::dn1(Fs), Fu01 = pcr::dn1(Fu0), Fu11 = pcr::dn1(Fu1), Fu21 = pcr::dn1(Fu2);
-        float Rh1 = 0.0f, Rh2 = 0.0f;
-        if (hasC) {
-            const float iJc = c.iJ;
-            Te -= (Fs1 - Fs) * iJc;
-            const float d0 = (Fu01 - Fu0) * iJc, d1 = (Fu11 - Fu1) * iJc, d2 = (Fu21 - Fu2) * iJc;
-            float c1, c2;
-            if (n.sphere) {
-                const float *B = g.basis;
-                const float sk = g.sc[kc];
-                c1 = sk * (d0 * B[6 * nc + col] + d1 * B[7 * nc + col] + d2 * B[8 * nc + col]);
-                c2 = sk * (d0 * B[9 * nc + col] + d1 * B[10 * nc + col] + d2 * B[11 * nc + col]);
+                tU[p][r][sw(r, c)] = v.x;
+                tU[p][r][sw(r, c + 1)] = v.y;
+                tU[p][r][sw(r, c + 2)] = v.z;
+                tU[p][r][sw(r, c + 3)] = v.w;
             } else {
-                c1 = d0;
-                c2 = d1;
+                float v = 0.0f;
+                if (in) {
+#pragma unroll
+                    for (int t = 0; t < NF; ++t) v = fmaf(src.cf[t], src.full[t][o], v);
+#pragma unroll
+                    for (int t = 0; t < NI; ++t) v = fmaf(src.ci[t], src.fi[t][o], v);
+                }
+                tU[p][r][sw(r, c)] = v;
             }
-            const float irho = idp::rcp_nr(c.rho);
-            Rh1 = dtg * (0.0f - c1 * irho);
-            Rh2 = dtg * (0.0f - c2 * irho);
-        }
-        const float Re = dtg * Te;
-        // diffusion blocks of centre k (rows >= nl: identity)
-        float elo = 0.0f, ed = 1.0f, eup = 0.0f, hlo = 0.0f, hd = 1.0f, hup = 0.0f;
-        if (hasC) {
-            const float rm = a.rho, rp = pcr::dn1(c.rho), r0 = c.rho;
-            const float iJc = idp::rcp_nr(c.J);
-            const float irm = idp::rcp_nr(rm), ir0 = idp::rcp_nr(r0), irp = idp::rcp_nr(rp);
-            float dlo = 0.0f, dup = 0.0f;
-            if (k >= 1) {
-                const float sf = g.sf[k];
-                dlo = (g.Jh[col] * sf * sf * g.Jvf[k]) * g.g33f[k] * ca_rhoK(rm, r0, Kdm, Kd) * iJc;
-            }
-            if (k + 1 <= nl - 1) {
-                const float sf = g.sf[k + 1];
-                dup = (g.Jh[col] * sf * sf * g.Jvf[k + 1]) * g.g33f[k + 1] * ca_rhoK(r0, rp, Kd, Kdp) * iJc;
-            }
-            const float dd = -(dlo + dup);
-            elo = k >= 1 ? dtg * dlo * (kcv * irm) : 0.0f;
-            ed = dtg * dd * (kcv * ir0) - 1.0f;
-            eup = k + 1 <= nl - 1 ? dtg * dup * (kcv * irp) : 0.0f;
-            hlo = dtg * ir0 * dlo;
-            hd = dtg * ir0 * dd - 1.0f;
-            hup = dtg * ir0 * dup;
-        }
-        // face row k and its residual
-        FaceRow fr;
-        fr.r0 = fr.r1 = fr.e0 = fr.e1 = fr.h0a = fr.h0b = fr.h1a = fr.h1b = fr.lo = fr.up = 0.0f;
-        fr.d = 1.0f;
-        float Ru3 = 0.0f;
-        if (intF) {
-            fr = jac_face_row(g, n, k, col, a, c, u3m, u3, u3p, dtg);
-            Ru3 = dtg * (pgf_u3(g, n, k, a, c) - beta_w(g, n, k, col) * u3);
-        } else if (isF) {
-            fr.d = -dtg * beta_w(g, n, k, col) - 1.0f;
-        }
-        // ---- ApproximateBlockArrowheadIterativeSolve
-        idp::Centre cb;
-        cb.a0 = a0;
-        cb.a1 = a1;
-        cb.e0 = e0;
-        cb.e1 = e1;
-        cb.elo = hasC ? elo : 0.0f;
-        cb.ed = hasC ? ed : 1.0f;
-        cb.eup = hasC ? eup : 0.0f;
-        cb.hlo = hasC ? hlo : 0.0f;
-        cb.hd = hasC ? hd : 1.0f;
-        cb.hup = hasC ? hup : 0.0f;
-        cb.br = Rr;
-        cb.be = hasC ? Re : 0.0f;
-        cb.bh1 = hasC ? Rh1 : 0.0f;
-        cb.bh2 = hasC ? Rh2 : 0.0f;
-        const idp::Sol x = idp::arrowhead_solve(k, nl, hasC, intF, isF, cb, fr, Ru3, n.siters);
-        const float xh1 = x.xh1, xh2 = x.xh2, xe = x.xe, xw = x.xw, xr = x.xr;
-        // Newton update
-        const float rho_n = rho - xr;
-        const float u1_n = u1 - xh1, u2_n = u2 - xh2;
-        float rhoe_n = rhoe - xe;
-        const float u3_n = intF ? u3 - xw : 0.0f;
-        // post-Newton upwind correction at the new state
-        if (n.upw != 0) {
-            const float u3_np = pcr::dn1(u3_n);
-            const float hn = cv_enthalpy(g, n, kc, col, rho_n, u1_n, u2_n, rhoe_n, u3_n, hasC ? u3_np : 0.0f);
-            const float href = pcr::lane0(hn);
-            const float hr = hn - href;
-            const float sk = g.sc[kc];
-            const float rJn = rho_n * (g.Jh[col] * sk * sk * g.Jvc[kc]);
-            const float h2 = pcr::up(hr, 2), h1 = pcr::up1(hr), h4 = pcr::dn1(hr);
-            const float rJn1 = pcr::up1(rJn);
-            float dF = 0.0f;
-            if (intF) {
-                const float v = u3_n * g33;
-                const float rJf = 0.5f * (rJn1 + rJn);
-                const float upw = upwind_product(n.upw, k, nl, v, n.dt, h2, h1, hr, h4);
-                const float cen = upwind_product(0, k, nl, v, n.dt, 0.0f, h1, hr, 0.0f);
-                dF = rJf * upw - rJf * cen;
-            }
-            const float dF1 = pcr::dn1(dF);
-            const float corr = hasC ? -(dF1 - dF) * (g.iJh[col] * g.isJc[kc]) : 0.0f;
-            rhoe_n += dtg * corr;
-        }
-        // U and F_I = (U - U~) / dtg
-        if (hasC) {
-            tU[0][k][cc] = rho_n;
-            tU[1][k][cc] = u1_n;
-            tU[2][k][cc] = u2_n;
-            tU[3][k][cc] = rhoe_n;
-            tF[0][k][cc] = (rho_n - rho) * idtg;
-            tF[1][k][cc] = (u1_n - u1) * idtg;
-            tF[2][k][cc] = (u2_n - u2) * idtg;
-            tF[3][k][cc] = (rhoe_n - rhoe) * idtg;
-        }
-        if (isF) {
-            tU[4][k][cc] = u3_n;
-            tF[4][k][cc] = (u3_n - u3) * idtg;
         }
     }
     __syncthreads();
-
-    // ---- phase 3: coalesced stores of U and F_I
-    if constexpr (V4) {
-        for (int idx = tid; idx < 16 * TC; idx += 256) {
-            const int r = idx / (TC / 4), c4 = 4 * (idx - r * (TC / 4));
-            const int col = col0 + c4;
-            if (col >= nc) continue;
-            const int64_t q = (int64_t)r * nc + col;
-            auto row4 = [&](const float (*t)[R]) {
-                return make_float4(t[r][c4], t[r][c4 + 1], t[r][c4 + 2], t[r][c4 + 3]);
-            };
-            if (r < nl) {
+    {
+        const float idtg = 1.0f / dtg;
+        cst::Lev<R> t;
+        cst::lev_load<R>(g, tid & (W - 1), t);
+        cst::Dif<R> df;
+        cst::dif_load<R>(g, n, tid & (W - 1), df);
+        for (int cc = tid / W; cc < TC; cc += 256 / W) {
+            const int col = col0 + cc;
+            if (col >= nc) break;  // uniform across the wavefront (W = 32: ncol is a multiple of 16)
+            const cst::Met1 m = cst::met1_load(g, n, col);
+            const float D0 = n.vdk == 0 ? g.D0_col[col] : 0.0f;
+            float v[5][R], f[5][R];
 #pragma unroll
-                for (int comp = 0; comp < 4; ++comp) {
-                    *reinterpret_cast<float4 *>(U + comp * nC + q) = row4(tU[comp]);
-                    if (FI) *reinterpret_cast<float4 *>(FI + comp * nC + q) = row4(tF[comp]);
+            for (int r = 0; r < R; ++r) {
+                const int kc = min(t.k[r], nl - 1), c = sw(kc, cc);
+#pragma unroll
+                for (int p = 0; p < 5; ++p) v[p][r] = p < 4 || t.intF[r] ? tU[p][kc][c] : 0.0f;
+            }
+            cst::newton_idiff<R, W>(t, df, m, n, nl, D0, dtg, v[0], v[1], v[2], v[3], v[4]);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (t.hasC[r]) {
+                    const int k = t.k[r], c = sw(k, cc);
+#pragma unroll
+                    for (int p = 0; p < 5; ++p) {
+                        f[p][r] = (v[p][r] - tU[p][k][c]) * idtg;  // F_I = (U - U~) / dtg
+                        tU[p][k][c] = v[p][r];
+                        tF[p][k][c] = f[p][r];
+                    }
                 }
-            }
-            if (r <= nl) {
-                *reinterpret_cast<float4 *>(U + 4 * nC + q) = row4(tU[4]);
-                if (FI) *reinterpret_cast<float4 *>(FI + 4 * nC + q) = row4(tF[4]);
-            }
         }
-        return;
     }
-    for (int idx = tid; idx < 64 * TC; idx += 256) {
-        const int r = idx / TC, cc = idx - r * TC;
-        const int col = col0 + cc;
-        if (col >= nc) continue;
-        const int64_t q = (int64_t)r * nc + col;
-        if (r < nl) {
+    __syncthreads();
+    // ---- U and F_I out (face nl: zero)
+    for (int idx = tid; idx < (nl + 1) * (TC / VW); idx += 256) {
+        const int r = idx / (TC / VW), c = VW * (idx - r * (TC / VW));
+        if (col0 + c >= nc) continue;
+        const int64_t q = (int64_t)r * nc + col0 + c;
+        auto put = [&](float *dst, const float (*tile)[TC], bool in) {
+            if constexpr (V4)
+                *reinterpret_cast<float4 *>(dst) = in ? make_float4(tile[r][sw(r, c)], tile[r][sw(r, c + 1)],
+                                                                    tile[r][sw(r, c + 2)], tile[r][sw(r, c + 3)])
+                                                      : make_float4(0.f, 0.f, 0.f, 0.f);
+            else
+                *dst = in ? tile[r][sw(r, c)] : 0.0f;
+        };
 #pragma unroll
-            for (int comp = 0; comp < 4; ++comp) {
-                U[comp * nC + q] = tU[comp][r][cc];
-                if (FI) FI[comp * nC + q] = tF[comp][r][cc];
-            }
-        }
-        if (r <= nl) {
-            U[4 * nC + q] = tU[4][r][cc];
-            if (FI) FI[4 * nC + q] = tF[4][r][cc];
+        for (int p = 0; p < 5; ++p) {
+            if (p < 4 && r == nl) continue;
+            put(U + p * nC + q, tU[p], r < nl);
+            if (FI) put(FI + p * nC + q, tF[p], r < nl);
         }
     }
 }
 
-#define CA_INST_IDIFF(NF, NI, V4)                                                                          \
-    template __global__ void k_newton_idiff_pcr<NF, NI, V4>(DevGeom, DevNum, StageSrc, float, float *, float *);
-#define CA_INST_IDIFF_ALL(V4) \
-    CA_INST_IDIFF(2, 0, V4)   \
-    CA_INST_IDIFF(3, 1, V4)   \
-    CA_INST_IDIFF(4, 2, V4)   \
-    CA_INST_IDIFF(-1, -1, V4)
-CA_INST_IDIFF_ALL(false)
-CA_INST_IDIFF_ALL(true)
+#define CA_INST_IDIFF(R, W, V4)                                                                                      \
+    template __global__ void k_newton_idiff_rows<R, W, 2, 0, V4>(DevGeom, DevNum, StageSrc, float, float *, float *); \
+    template __global__ void k_newton_idiff_rows<R, W, 3, 1, V4>(DevGeom, DevNum, StageSrc, float, float *, float *); \
+    template __global__ void k_newton_idiff_rows<R, W, 4, 2, V4>(DevGeom, DevNum, StageSrc, float, float *, float *);
+CA_INST_IDIFF(1, 32, true)
+CA_INST_IDIFF(1, 32, false)
+CA_INST_IDIFF(2, 32, true)
+CA_INST_IDIFF(2, 32, false)
+CA_INST_IDIFF(1, 64, true)
+CA_INST_IDIFF(1, 64, false)
+CA_INST_IDIFF(2, 64, true)
+CA_INST_IDIFF(2, 64, false)
+#undef CA_INST_IDIFF
 
 // ldiv! with implicit diffusion from the stored bands (the hook entry point
 // ca_ldiv after ca_update_jacobian): dY = solve(A, rscale R) with the
