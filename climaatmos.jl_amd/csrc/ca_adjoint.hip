@@ -19,9 +19,11 @@
 //             Jacobian entries, which are taken in forward mode over the 11
 //             values a face row reads (dual numbers, float64).
 //
-// Checkpointing: the forward pass stores the state every `every` steps; the
-// reverse pass recomputes each segment's step states from its checkpoint and
-// each step's stage states from its start state.  The non-smooth points
+// Forward states: where every step's stage states fit in memory they are kept
+// (k_ens_adj_forward / record / reverse).  Otherwise the forward pass stores the
+// state every `every` steps and the reverse pass recomputes each segment's step
+// states from its checkpoint and each step's stage states from its start state
+// (k_ensemble_adjoint).  Both run the same functions.  The non-smooth points
 // (the T_min clamp, the van Leer limiter branches) take the derivative of the
 // branch the forward pass took.
 #include "ca_kernels.h"
@@ -219,9 +221,11 @@ struct AdjSharedT {
     float fib[3][3][NF];      // of F_I_i (rho, rho e_tot, u_3)
     float Ub[5][NF];          // of U_i, then of the pre-correction state V_i
     float Utb[5][NF];         // of U~_i
-    float W[24][NF];          // scratch of the local reverse passes
     double lam[NF];           // transposed Schur solution
-    double red[2][128];       // block reduction of the parameter cotangents (LPM <= 128)
+    union {
+        float W[24][NF];      // scratch of the local reverse passes
+        double red[2][128];   // block reduction of the parameter cotangents (LPM <= 128)
+    };
 };
 
 // The part of AdjSharedT one implicit stage's reverse uses (newton_vjp alone)
@@ -957,6 +961,74 @@ __device__ void reverse_step(AdjSharedT<NF> &A, const DevGeom &g, const DevNum &
     sync();
 }
 
+// The level tables of one member in LDS: a step reads them in every phase, and
+// a phase between two barriers cannot hide a load from the L2 (128 members,
+// 16 steps: forward 435 -> 408 us, reverse 1107 -> 1041 us).
+template <int NF>
+struct LevelsLds {
+    double phic[NF], dphif[NF];
+    float c[7][NF], f[7][NF];
+};
+// copies g's tables into L and returns g with its pointers moved there
+template <int LPM, int NF>
+__device__ __forceinline__ DevGeom stage_levels(LevelsLds<NF> &L, const DevGeom &g, int tid) {
+    const int nl = g.nlev;
+    for (int k = tid; k <= nl; k += LPM) {
+        if (k < nl) {
+            L.phic[k] = g.Phic_d[k];
+            L.c[0][k] = g.Jvc[k];
+            L.c[1][k] = g.iJvc[k];
+            L.c[2][k] = g.is2c[k];
+            L.c[3][k] = g.isJc[k];
+            L.c[4][k] = g.sc[k];
+            L.c[5][k] = g.Phic[k];
+            L.c[6][k] = g.zeta_c[k];
+        }
+        L.dphif[k] = g.dPhif_d[k];
+        L.f[0][k] = g.Jvf[k];
+        L.f[1][k] = g.sf[k];
+        L.f[2][k] = g.g33f[k];
+        L.f[3][k] = g.iJvf[k];
+        L.f[4][k] = g.isf[k];
+        L.f[5][k] = g.isJf[k];
+        L.f[6][k] = g.zeta_f[k];
+    }
+    DevGeom r = g;
+    r.Phic_d = L.phic;
+    r.dPhif_d = L.dphif;
+    r.Jvc = L.c[0];
+    r.iJvc = L.c[1];
+    r.is2c = L.c[2];
+    r.isJc = L.c[3];
+    r.sc = L.c[4];
+    r.Phic = L.c[5];
+    r.zeta_c = L.c[6];
+    r.Jvf = L.f[0];
+    r.sf = L.f[1];
+    r.g33f = L.f[2];
+    r.iJvf = L.f[3];
+    r.isf = L.f[4];
+    r.isJf = L.f[5];
+    r.zeta_f = L.f[6];
+    sync();
+    return r;
+}
+
+// member state <-> S.u (u_3 filtered on load)
+template <int LPM, class SH>
+__device__ __forceinline__ void state_load(SH &S, int nl, const float *src, int tid) {
+    for (int k = tid; k < nl; k += LPM)
+        for (int p = 0; p < 4; ++p) S.u[p][k] = src[p * nl + k];
+    for (int f = tid; f <= nl; f += LPM) S.u[4][f] = (f == 0 || f == nl) ? 0.0f : src[4 * nl + f];
+    sync();
+}
+template <int LPM, class SH>
+__device__ __forceinline__ void state_store(const SH &S, int nl, float *dst, int tid) {
+    for (int k = tid; k < nl; k += LPM)
+        for (int p = 0; p < 4; ++p) dst[p * nl + k] = S.u[p][k];
+    for (int f = tid; f <= nl; f += LPM) dst[4 * nl + f] = S.u[4][f];
+}
+
 }  // namespace adj
 
 // Adjoint of nsteps ensemble steps: workgroup b reverses member order[b].
@@ -985,17 +1057,8 @@ __global__ void __launch_bounds__(LPM) k_ensemble_adjoint(const DevGeom *__restr
     const int nseg = (nsteps + every - 1) / every;
     float *ck = ckpt + (int64_t)(nseg + 1) * off[m];
     float *sg = seg + (int64_t)every * off[m];
-    auto load = [&](const float *src) {  // member state -> S.u (u_3 filtered)
-        for (int k = tid; k < nl; k += LPM)
-            for (int p = 0; p < 4; ++p) S.u[p][k] = src[p * nl + k];
-        for (int f = tid; f <= nl; f += LPM) S.u[4][f] = (f == 0 || f == nl) ? 0.0f : src[4 * nl + f];
-        sync();
-    };
-    auto store = [&](float *dst) {
-        for (int k = tid; k < nl; k += LPM)
-            for (int p = 0; p < 4; ++p) dst[p * nl + k] = S.u[p][k];
-        for (int f = tid; f <= nl; f += LPM) dst[4 * nl + f] = S.u[4][f];
-    };
+    auto load = [&](const float *src) { state_load<LPM>(S, nl, src, tid); };
+    auto store = [&](float *dst) { state_store<LPM>(S, nl, dst, tid); };
     // forward, storing a checkpoint every `every` steps
     load(Y0 + off[m]);
     store(ck);
@@ -1054,3 +1117,112 @@ CA_ADJ_INST(128, 65)
 CA_ADJ_INST(64, 129)
 CA_ADJ_INST(128, 129)
 #undef CA_ADJ_INST
+
+// The adjoint in three launches, for runs whose step and stage states are
+// kept: the forward steps (serial per member), the stage states of all steps
+// (a workgroup per member and step: every step starts from its kept state),
+// and the reverse (serial per member).  Member m's part of seg starts at
+// nsteps off[m], of rec at 6 nsteps off[m].
+//
+// What bounds it is the serial chain: one step of one member after the other,
+// two wavefronts per member, most of whose time is waits between barriers.
+// k_ensemble_adjoint's chain is the forward, nearly as many steps again for the
+// segments' states, and one more per reversed step; here the chain is the
+// forward and the reverse, and the recorded steps run side by side.  128
+// members of 30 to 128 levels, 16 steps: 2628 us there, here 408 + 134 + 1041.
+template <int LPM, int NF>
+__global__ void __launch_bounds__(LPM) k_ens_adj_forward(const DevGeom *__restrict__ mg, DevNum n,
+                                                         const int *__restrict__ order,
+                                                         const int64_t *__restrict__ off,
+                                                         const float *__restrict__ Y0, float *__restrict__ seg,
+                                                         EnsTab tab, float dt, int nsteps) {
+    __shared__ ens::SharedT<NF> S;
+    __shared__ adj::LevelsLds<NF> L;
+    const int m = order[blockIdx.x];
+    const int tid = threadIdx.x;
+    const DevGeom g = adj::stage_levels<LPM>(L, mg[m], tid);
+    const int nl = g.nlev;
+    const int64_t Sm = 5 * (int64_t)nl + 1;
+    float *sg = seg + nsteps * off[m];
+    adj::state_load<LPM>(S, nl, Y0 + off[m], tid);
+    adj::state_store<LPM>(S, nl, sg, tid);
+    for (int st = 1; st < nsteps; ++st) {
+        ens::step_once<LPM>(S, g, n, tab, dt, tid);
+        adj::state_store<LPM>(S, nl, sg + st * Sm, tid);
+    }
+}
+
+template <int LPM, int NF>
+__global__ void __launch_bounds__(LPM) k_ens_adj_record(const DevGeom *__restrict__ mg, DevNum n,
+                                                        const int *__restrict__ order,
+                                                        const int64_t *__restrict__ off,
+                                                        const float *__restrict__ seg, float *__restrict__ rec,
+                                                        EnsTab tab, float dt, int nsteps) {
+    __shared__ ens::SharedT<NF> S;
+    __shared__ adj::LevelsLds<NF> L;
+    __shared__ float R[6][5][NF];  // U~_1..3, U_1..3
+    const int m = order[blockIdx.x];
+    const int tid = threadIdx.x;
+    const DevGeom g = adj::stage_levels<LPM>(L, mg[m], tid);
+    const int nl = g.nlev;
+    const int64_t Sm = 5 * (int64_t)nl + 1;
+    adj::state_load<LPM>(S, nl, seg + nsteps * off[m] + blockIdx.y * Sm, tid);
+    ens::step_once<LPM>(S, g, n, tab, dt, tid, &R[0], &R[3]);
+    float *dst = rec + 6 * (nsteps * off[m] + blockIdx.y * Sm);
+    for (int s = 0; s < 6; ++s, dst += Sm) {
+        for (int k = tid; k < nl; k += LPM)
+            for (int p = 0; p < 4; ++p) dst[p * nl + k] = R[s][p][k];
+        for (int f = tid; f <= nl; f += LPM) dst[4 * nl + f] = R[s][4][f];
+    }
+}
+
+template <int LPM, int NF>
+__global__ void __launch_bounds__(LPM) k_ens_adj_reverse(const DevGeom *__restrict__ mg, DevNum n,
+                                                         const int *__restrict__ order,
+                                                         const int64_t *__restrict__ off,
+                                                         const float *__restrict__ YbN, float *__restrict__ Yb0,
+                                                         float *__restrict__ D0b, float *__restrict__ awb,
+                                                         const float *__restrict__ seg,
+                                                         const float *__restrict__ rec, EnsTab tab, float dt,
+                                                         int nsteps) {
+    using namespace adj;
+    __shared__ AdjSharedT<NF> A;
+    __shared__ LevelsLds<NF> L;
+    const int m = order[blockIdx.x];
+    const int tid = threadIdx.x;
+    const DevGeom g = adj::stage_levels<LPM>(L, mg[m], tid);
+    const int nl = g.nlev;
+    const int64_t Sm = 5 * (int64_t)nl + 1;
+    const float *ybn = YbN + off[m];
+    for (int k = tid; k < nl; k += LPM)
+        for (int p = 0; p < 4; ++p) A.ub[p][k] = ybn[p * nl + k];
+    for (int f = tid; f <= nl; f += LPM) A.ub[4][f] = (f == 0 || f == nl) ? 0.0f : ybn[4 * nl + f];
+    double kb = 0.0, ab = 0.0;
+    for (int j = nsteps - 1; j >= 0; --j) {
+        const float *src = rec + 6 * (nsteps * off[m] + j * Sm);
+        for (int s = 0; s < 6; ++s, src += Sm) {
+            float (*R)[NF] = s < 3 ? A.Ut[s] : A.Us[s - 3];
+            for (int k = tid; k < nl; k += LPM)
+                for (int p = 0; p < 4; ++p) R[p][k] = src[p * nl + k];
+            for (int f = tid; f <= nl; f += LPM) R[4][f] = src[4 * nl + f];
+        }
+        state_load<LPM>(A.S, nl, seg + nsteps * off[m] + j * Sm, tid);
+        reverse_step<LPM>(A, g, n, tab, dt, tid, kb, ab);
+    }
+    float *yb0 = Yb0 + off[m];
+    for (int k = tid; k < nl; k += LPM)
+        for (int p = 0; p < 4; ++p) yb0[p * nl + k] = A.ub[p][k];
+    for (int f = tid; f <= nl; f += LPM) yb0[4 * nl + f] = A.ub[4][f];
+    A.red[0][tid] = kb;
+    A.red[1][tid] = ab;
+    sync();
+    if (tid == 0) {
+        double s0 = 0.0, s1 = 0.0;
+        for (int t = 0; t < LPM; ++t) {
+            s0 += A.red[0][t];
+            s1 += A.red[1][t];
+        }
+        D0b[m] = (float)s0;
+        awb[m] = (float)s1;
+    }
+}

@@ -37,7 +37,7 @@ struct ca_ensemble {
     float *cols = nullptr;
     std::vector<float> hcols;
     // adjoint scratch: checkpoints and segment states
-    float *ckpt = nullptr, *segb = nullptr;
+    float *ckpt = nullptr, *segb = nullptr, *recb = nullptr;
     int ck_nsteps = -1, ck_every = -1;
     // this device's copy of the file-scope scratch array (ca_ensemble_adjoint_noalloc)
     float *noalloc_scratch = nullptr;
@@ -264,6 +264,31 @@ ca_status ens_adjoint_launch(ca_ensemble *e, const float *Y0, const float *YbN, 
     return CA_OK;
 }
 
+// the same in three launches (k_ens_adj_*): sg holds nsteps * S floats, rc 6 nsteps * S
+ca_status ens_adjoint_split(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int nsteps, float *Yb0,
+                            float *D0b, float *awb, float *sg, float *rc, hipStream_t st) {
+    const int *ord = e->order[e->order_kind];
+    const dim3 grid(e->M);
+    const bool l64 = e->lanes_set && e->lanes == 64;
+#define CA_ADJ_GO(LPM, NF)                                                                                      \
+    do {                                                                                                        \
+        k_ens_adj_forward<LPM, NF><<<grid, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, Y0, sg, e->tab, (float)dt, \
+                                                         nsteps);                                               \
+        k_ens_adj_record<LPM, NF><<<dim3(e->M, nsteps), LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sg, rc, e->tab, \
+                                                                      (float)dt, nsteps);                       \
+        k_ens_adj_reverse<LPM, NF><<<grid, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, YbN, Yb0, D0b, awb, sg, rc, \
+                                                         e->tab, (float)dt, nsteps);                            \
+    } while (0)
+    if (e->nf == 33) CA_ADJ_GO(64, 33);
+    else if (e->nf == 65 && l64) CA_ADJ_GO(64, 65);
+    else if (e->nf == 65) CA_ADJ_GO(128, 65);
+    else if (l64) CA_ADJ_GO(64, 129);
+    else CA_ADJ_GO(128, 129);
+#undef CA_ADJ_GO
+    EHIPCHK(e, hipGetLastError());
+    return CA_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -301,7 +326,7 @@ ca_status ca_ensemble_create(const ca_params *params, const ca_config *config, i
 ca_status ca_ensemble_destroy(ca_ensemble *e) {
     if (!e) return CA_ERR_ARG;
     ens_drop_graph(e);
-    for (void *p : {(void *)e->ckpt, (void *)e->segb})
+    for (void *p : {(void *)e->ckpt, (void *)e->segb, (void *)e->recb})
         if (p) (void)hipFree(p);
     for (void *p : e->allocs) (void)hipFree(p);
     delete e;
@@ -434,18 +459,33 @@ ca_status ca_ensemble_adjoint(ca_ensemble *e, const float *Y0, const float *YbN,
                               int32_t every, float *Yb0, float *D0b, float *awb, void *stream) {
     if (!e || !Y0 || !YbN || !Yb0 || !D0b || !awb || nsteps < 1 || every < 1 || !(dt > 0)) return CA_ERR_ARG;
     if (e->ck_nsteps != nsteps || e->ck_every != every) {
-        for (float **p : {&e->ckpt, &e->segb})
+        for (float **p : {&e->ckpt, &e->segb, &e->recb})
             if (*p) {
                 (void)hipFree(*p);
                 *p = nullptr;
             }
         e->ck_nsteps = e->ck_every = -1;
-        const int64_t nseg = (nsteps + every - 1) / every;
-        EHIPCHK(e, hipMalloc(&e->ckpt, (size_t)((nseg + 1) * e->S) * sizeof(float)));
-        EHIPCHK(e, hipMalloc(&e->segb, (size_t)(every * e->S) * sizeof(float)));
+        // three launches over kept stage states where these take at most 1 GiB
+        // (and that is free); otherwise checkpoints and segments
+        const int64_t state = e->S * (int64_t)sizeof(float);
+        if (7 * nsteps * state <= (int64_t{1} << 30) && nsteps <= 65535) {
+            if (hipMalloc(&e->recb, (size_t)(6 * nsteps * state)) != hipSuccess ||
+                hipMalloc(&e->segb, (size_t)(nsteps * state)) != hipSuccess) {
+                (void)hipGetLastError();
+                if (e->recb) (void)hipFree(e->recb);
+                e->recb = e->segb = nullptr;
+            }
+        }
+        if (!e->recb) {
+            const int64_t nseg = (nsteps + every - 1) / every;
+            EHIPCHK(e, hipMalloc(&e->ckpt, (size_t)((nseg + 1) * state)));
+            EHIPCHK(e, hipMalloc(&e->segb, (size_t)(every * state)));
+        }
         e->ck_nsteps = nsteps;
         e->ck_every = every;
     }
+    if (e->recb)
+        return ens_adjoint_split(e, Y0, YbN, dt, nsteps, Yb0, D0b, awb, e->segb, e->recb, (hipStream_t)stream);
     return ens_adjoint_launch(e, Y0, YbN, dt, nsteps, every, Yb0, D0b, awb, e->ckpt, e->segb, (hipStream_t)stream);
 }
 

@@ -333,15 +333,17 @@ ca_status ca_ensemble_autotune(ca_ensemble *e, const float *Y, double dt, int32_
 /* new per-member alpha_w and / or D0 (host arrays of nmembers; NULL keeps) */
 ca_status ca_ensemble_set_params(ca_ensemble *e, const double *alpha_w, const double *D0);
 /* Reverse mode of nsteps ensemble steps (the vector-Jacobian product of the
- * solution operator), with step checkpointing every `every` steps.  No
+ * solution operator).  No
  * reference counterpart: the reference differentiates only its Jacobians, in
  * forward mode (implicit/autodiff_utils.jl), and calibrates without gradients.
  * Given the initial states Y0 and the cotangent YbN of the states after
  * nsteps steps, writes the cotangent of Y0 to Yb0 (ragged, like Y0) and of
  * each member's D0 and alpha_w to D0b, awb (device arrays of nmembers).
- * Recomputes the forward trajectory itself; runs with 64 lanes per member
- * when every member has at most 32 levels or CA_ENS_LANES was set to 64, else
- * 128. */
+ * Recomputes the forward trajectory itself, in scratch that the ensemble
+ * keeps: 7 states per step, where that is at most 1 GiB and free, and
+ * otherwise a checkpoint every `every` steps and the states of one such
+ * segment.  Runs with 64 lanes per member when every member has at most 32
+ * levels or CA_ENS_LANES was set to 64, else 128. */
 ca_status ca_ensemble_adjoint(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int32_t nsteps,
                               int32_t every, float *Yb0, float *D0b, float *awb, void *stream);
 /* ca_ensemble_adjoint without any device allocation.  No counterpart in the
@@ -353,7 +355,7 @@ ca_status ca_ensemble_adjoint(ca_ensemble *e, const float *Y0, const float *YbN,
  * ca_ensemble_state_size(e) floats, and a larger request returns CA_ERR_ARG
  * before any launch.  Every call on one GPU shares that array: calls that
  * overlap on one GPU (on different streams, or from different ensembles or
- * threads) race.  Same kernels and results as ca_ensemble_adjoint. */
+ * threads) race.  Same results as ca_ensemble_adjoint. */
 ca_status ca_ensemble_adjoint_noalloc(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int32_t nsteps,
                                       int32_t every, float *Yb0, float *D0b, float *awb, void *stream);
 
