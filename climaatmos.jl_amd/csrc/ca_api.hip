@@ -809,11 +809,15 @@ ca_status create_impl(const ca_geometry *geom, const ca_params *par, const ca_co
         HIPCHK(h, hipMemset(h->FI[i], 0xff, (size_t)h->fi_size * sizeof(float)));
     ars343(h);
     h->newton_variant = (nl + 1 <= 64) ? 1 : 0;
-    // level chunks sized so that small grids still fill the chip: about
-    // 1024 wavefronts for the per-node sweeps, 1024 workgroups for the DSS
+    // level chunks sized so that small grids still fill the chip: the largest
+    // that leaves about 7000 wavefronts of k_laplacians and 1500 workgroups of
+    // the DSS.  A level more per work item costs the latency of a level, one
+    // less the loads its set-up shares: a step takes 134 us with chunks of 1 and
+    // 1 (the rule) at h_elem 8, 30 levels against 141 with 3 and 2, 211 with 1
+    // and 2 at h_elem 10, 45 levels against 219 with 4 and 3; at h_elem 16, 63
+    // levels all from 2 to 8 are within 1%.
     {
         const int64_t layer_waves = (nc + 63) / 64;
-        const int64_t want = (1024 + layer_waves - 1) / layer_waves;
         // wavefronts of k_explicit a SIMD holds: 3 with vertical diffusion (147
         // VGPRs), 4 without (105, 124 with the final combination)
         h->explicit_chunk = h->final_chunk = explicit_chunk(layer_waves, nl, n.vdiff && !n.idiff ? 3 : 4);
@@ -825,12 +829,11 @@ ca_status create_impl(const ca_geometry *geom, const ca_params *par, const ca_co
         // 3.93 ms per gradient of 8 steps with chunks of 4 at h_elem 8, 30 levels,
         // 1.77 against 2.04 at h_elem 4, 16 levels (6 steps)
         h->adj_chunk = explicit_chunk(layer_waves, nl, 2);
-        h->lap_chunk = (int)std::min<int64_t>(4, std::max<int64_t>(2, (nl + want - 1) / want));
+        h->lap_chunk = (int)std::min<int64_t>(4, (layer_waves * nl + 6999) / 7000);
         if (g.ncl > 0) {
-            const int64_t wantd = (1024 + g.ncl - 1) / g.ncl;
             // 6 levels per workgroup measured best at h_elem 30, 63 levels (the
             // staged DSS's three launches 2-3% faster than with 8)
-            h->dss_chunk = (int)std::min<int64_t>(6, std::max<int64_t>(2, (nl + wantd - 1) / wantd));
+            h->dss_chunk = (int)std::min<int64_t>(6, ((int64_t)g.ncl * nl + 1499) / 1500);
         }
     }
     return CA_OK;
