@@ -228,19 +228,57 @@ struct AdjSharedT {
     };
 };
 
-// The part of AdjSharedT one implicit stage's reverse uses (newton_vjp alone)
+// The part of AdjSharedT one implicit stage's reverse uses (newton_vjp alone).
+// The wavefronts a CU holds are bounded by these bytes, so the local reverse
+// passes' scratch shares the Schur system's: they run before its rows are built
+// and after it is solved.  9.6 KB per column of 32 levels, 16 columns per CU;
+// 12.3 KB and 12 with every array on its own (37.3 -> 34.5 us per stage at
+// h_elem 8, 30 levels).
 template <int NF>
 struct NewtonAdjShared {
     static constexpr int NFv = NF;
-    ens::StageShared<NF> S;
+    struct {
+        float U[5][NF];
+        struct {
+            float c[11][NF];
+            double cd[3][NF];
+            float row[6][NF];
+            union {
+                double sys[2][4][NF];
+                float W[24][NF];
+            };
+            float x[NF], hr[NF], rJ[NF], ve[NF];
+        } nw;  // as ens::NwT
+    } S;
     float Ut[1][5][NF];
     float Ub[5][NF];
     float Utb[5][NF];
-    float W[24][NF];
     double lam[NF];
 };
 
+// the scratch planes of the local reverse passes
+template <int NF>
+__device__ __forceinline__ float (*scratch(AdjSharedT<NF> &A))[NF] {
+    return A.W;
+}
+template <int NF>
+__device__ __forceinline__ float (*scratch(NewtonAdjShared<NF> &A))[NF] {
+    return A.S.nw.W;
+}
+
 __device__ __forceinline__ void sync() { __syncthreads(); }
+// between the lanes of one column: up to 64 of them are one wavefront's, whose
+// LDS accesses are carried out in order
+template <int LPM>
+__device__ __forceinline__ void sync_column() {
+    if constexpr (LPM <= 64) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+        __syncthreads();
+    }
+}
 
 // Reverse of ens::explicit_tendency at Y: given the tendency cotangent Tb,
 // adds the state cotangent to Yb and returns this thread's D0 cotangent.
@@ -554,9 +592,9 @@ __device__ void newton_replay(SH &S, const DevGeom &g, const DevNum &n, float dt
     const int nl = g.nlev;
     ens::stage_thermo<LPM>(S, g, n, tid);
     for (int f = tid; f <= nl; f += LPM) S.nw.x[f] = (f >= 1 && f <= nl - 1) ? S.U[4][f] - u3N[f] : 0.0f;
-    sync();
+    sync_column<LPM>();
     ens::stage_rows<LPM>(S, g, dtg, tid);
-    sync();
+    sync_column<LPM>();
     for (int k = tid; k < nl; k += LPM) {
         const float de = S.nw.row[2][k] * S.nw.x[k] + S.nw.row[3][k] * S.nw.x[k + 1] - S.nw.row[5][k];
         S.U[0][k] = rhoN[k];
@@ -564,10 +602,10 @@ __device__ void newton_replay(SH &S, const DevGeom &g, const DevNum &n, float dt
         S.nw.ve[k] = S.U[3][k];
     }
     for (int f = tid; f <= nl; f += LPM) S.U[4][f] = (f >= 1 && f <= nl - 1) ? u3N[f] : 0.0f;
-    sync();
+    sync_column<LPM>();
     if (n.upw != 0) {
         ens::stage_enthalpy<LPM>(S, g, n, tid);
-        sync();
+        sync_column<LPM>();
     }
 }
 
@@ -581,7 +619,7 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
     constexpr int NF = AS::NFv;
     auto &S = A.S;
     const int nl = g.nlev;
-    float (*W)[NF] = A.W;
+    float (*W)[NF] = scratch(A);
     newton_replay<LPM>(S, g, n, dtg, rhoN, u3N, tid);  // S.U = U_i, S.nw = internals; V_i (rho e) in S.nw.ve
     double awbar = 0.0;
     // ---- upwind correction: U_e = V_e + dtg corr(V); V = U except rho e
@@ -595,7 +633,7 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
             }
             W[0][f] = dFb;
         }
-        sync();
+        sync_column<LPM>();
         // faces: dF = rJf (upw - cen), rJf = (rJ_f-1 + rJ_f)/2, v = u3 g33
         // contributions: W[1..4] h of centres f-2..f+1, W[5] rJ below, W[6] rJ above; u3 direct
         for (int f = tid; f <= nl; f += LPM) {
@@ -630,7 +668,7 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
             W[5][f] = rJa;
             W[6][f] = rJbv;
         }
-        sync();
+        sync_column<LPM>();
         // centres: gather h and rJ cotangents of centre k: from faces k+2 (as
         // f-2), k+1 (as f-1), k (as f), k-1 (as f+1); rJ from faces k+1, k
         for (int k = tid; k < nl; k += LPM) {
@@ -650,10 +688,10 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
             W[7][k] = out[4];  // to face k
             W[8][k] = out[5];  // to face k + 1
         }
-        sync();
+        sync_column<LPM>();
         for (int f = tid; f <= nl; f += LPM)
             if (f >= 1 && f <= nl - 1) A.Ub[4][f] += W[7][f] + W[8][f - 1];
-        sync();
+        sync_column<LPM>();
     }
     // ---- Newton update: V = U~ - delta; A.Ub now holds the V cotangent.
     // delta: dr_k = a0 x_k + a1 x_k+1 - Rr, de_k = e0 x_k + e1 x_k+1 - Re,
@@ -692,7 +730,7 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
         S.nw.sys[1][2][f] = U;
         S.nw.sys[1][3][f] = xb;
     }
-    sync();
+    sync_column<LPM>();
     // transposed rows: L'_f = U_{f-1}, D'_f = D_f, U'_f = L_{f+1}
     for (int f = tid; f < nl; f += LPM) {
         S.nw.sys[0][0][f] = f >= 1 ? S.nw.sys[1][2][f - 1] : 0.0;
@@ -700,7 +738,7 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
         S.nw.sys[0][2][f] = f + 1 < nl ? S.nw.sys[1][0][f + 1] : 0.0;
         S.nw.sys[0][3][f] = S.nw.sys[1][3][f];
     }
-    sync();
+    sync_column<LPM>();
     int src = 0;
     for (int s = 1; s < nl; s <<= 1) {
         for (int f = tid; f < nl; f += LPM) {
@@ -724,11 +762,11 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
             S.nw.sys[src ^ 1][2][f] = nU;
             S.nw.sys[src ^ 1][3][f] = nr;
         }
-        sync();
+        sync_column<LPM>();
         src ^= 1;
     }
     for (int f = tid; f <= nl; f += LPM) A.lam[f] = f < nl ? S.nw.sys[src][3][f] * ca_drcp(S.nw.sys[src][1][f]) : 0.0;
-    sync();
+    sync_column<LPM>();
     // faces 1 .. nl - 1: cotangents of the Schur row entries and rhs, then
     // of the 11 values the face row reads (face_vjp); W[0..3] centre
     // below, W[4..7] centre above, W[8..10] u_3 of faces f-1, f, f+1;
@@ -779,7 +817,7 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
         W[13][f] = r1v;
         W[14][f] = e1v;
     }
-    sync();
+    sync_column<LPM>();
     // centres: cotangents of the centre rows (a0, a1, e0, e1, Rr, Re) from
     // the Schur rows of faces k and k+1 and from dr, de; then the rows'
     // reverse onto rJ and h of centres k-1, k, k+1 (W[15..20]) and the u_3 of
@@ -862,7 +900,7 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
         W[21][k] = u3k;
         W[22][k] = u3k1;
     }
-    sync();
+    sync_column<LPM>();
     // centres: gather rJ, h cotangents; chain through rJ = rho J and h(U~);
     // add the face rows' centre cotangents (face k: above, face k+1: below)
     for (int k = tid; k < nl; k += LPM) {
@@ -888,7 +926,7 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
         W[21][k] += out[4];
         W[22][k] += out[5];
     }
-    sync();
+    sync_column<LPM>();
     for (int f = tid; f <= nl; f += LPM) {
         if (f >= 1 && f <= nl - 1) {
             float v = W[21][f] + W[22][f - 1] + W[9][f];
@@ -897,7 +935,7 @@ __device__ double newton_vjp(AS &A, const DevGeom &g, const DevNum &n, float dtg
             A.Utb[4][f] += v;
         }
     }
-    sync();
+    sync_column<LPM>();
     return awbar;
 }
 

@@ -199,11 +199,11 @@ ca_status newton_vjp(ca_handle *h, const float *Ut, const float *Un, const float
     const DevGeom &g = h->g;
     if (g.nlev > kMaxAdjLevels) return fail(h, CA_ERR_ARG, "newton_vjp: nlev > 128");
     if (g.nlev <= 32)
-        sadj::k_newton_vjp<32, 33, 2><<<dim3(cdiv(g.ncol, 2)), 64, 0, st>>>(h->cgeo, h->n, g.nC, g.ncol, Ut, Un, Ub,
-                                                                            dtg, Utb, fib, cfi, fa, fb);
+        sadj::k_newton_vjp<32, 33, 8><<<dim3(cdiv(g.ncol, 8)), 256, 0, st>>>(h->cgeo, h->n, g.nC, g.ncol, Ut, Un, Ub,
+                                                                             dtg, Utb, fib, cfi, fa, fb);
     else if (g.nlev <= 64)
-        sadj::k_newton_vjp<64, 65, 1><<<dim3(g.ncol), 64, 0, st>>>(h->cgeo, h->n, g.nC, g.ncol, Ut, Un, Ub, dtg, Utb,
-                                                                   fib, cfi, fa, fb);
+        sadj::k_newton_vjp<64, 65, 4><<<dim3(cdiv(g.ncol, 4)), 256, 0, st>>>(h->cgeo, h->n, g.nC, g.ncol, Ut, Un, Ub,
+                                                                             dtg, Utb, fib, cfi, fa, fb);
     else
         sadj::k_newton_vjp<128, 129, 1><<<dim3(g.ncol), 128, 0, st>>>(h->cgeo, h->n, g.nC, g.ncol, Ut, Un, Ub, dtg,
                                                                       Utb, fib, cfi, fa, fb);
