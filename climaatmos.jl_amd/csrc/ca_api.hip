@@ -424,9 +424,11 @@ void launch_newton_rows(const ca_handle *h, const StageSrc &src, float dtg, int 
     const int nl = g.nlev;
     const bool v4 = stage_al16(h, src, i, U, nullptr);
     float *FI = keep_fi ? h->FI[i] : nullptr;
-    if (nl >= 64) launch_rows<2, 64, 16, 256>(h, v4, src, dtg, U, FI, st);
-    else if (h->newton_variant == 2) launch_rows<1, 64, 32, 256>(h, v4, src, dtg, U, FI, st);  // 32-column tiles
-    else if (!h->n.sphere || (nl > 56 && g.ncol >= 16 * 4096)) launch_rows<1, 64, 16, 256>(h, v4, src, dtg, U, FI, st);
+    const bool sph = h->n.sphere;
+    if (nl > 96 || (nl >= 64 && !sph)) launch_rows<2, 64, 16, 256>(h, v4, src, dtg, U, FI, st);
+    else if (nl > 64) launch_rows<3, 32, 16, 256>(h, v4, src, dtg, U, FI, st);
+    else if (h->newton_variant == 2 && nl < 64) launch_rows<1, 64, 32, 256>(h, v4, src, dtg, U, FI, st);  // 32-column tiles
+    else if (!sph || (nl > 56 && g.ncol >= 16 * 4096)) launch_rows<1, 64, 16, 256>(h, v4, src, dtg, U, FI, st);
     else if (nl > 32) launch_rows<2, 32, 16, 256>(h, v4, src, dtg, U, FI, st);
     else launch_rows<1, 32, 16, 512>(h, v4, src, dtg, U, FI, st);
 }

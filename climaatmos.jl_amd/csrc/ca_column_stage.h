@@ -1,7 +1,7 @@
 // ca_column_stage.h -- the implicit ARS343 stage and the explicit tendency of
 // one column held in a wavefront's registers: lane l owns the R consecutive
-// rows R l .. R l + R - 1 (row k = centre k and face k), so R = 1 holds
-// columns of up to 64 levels and R = 2 of up to 128.  Face nlev carries
+// rows R l .. R l + R - 1 (row k = centre k and face k) of its column's W lanes, so
+// a column has up to R W levels.  Face nlev carries
 // u_3 = 0 and needs no row of its own.
 //
 // Vertical neighbours are lane exchanges (DPP wave shifts, ca_newton_pcr.hip)
@@ -105,31 +105,39 @@ __device__ __forceinline__ double temperature(const DevNum &n, double et, float 
 }
 
 // The tridiagonal Schur system in float64 (the acoustic system is stiff:
-// dtg c / dz >> 1).  Two rows per lane: the odd row is eliminated into its
-// even neighbours first, which leaves one row per lane for parallel cyclic
-// reduction over the column's W lanes, and is substituted back.  With W = 32 the
-// exchanges across lanes 31 / 32 fetch the other column's finite values, which
-// meet exactly zero couplings.
+// dtg c / dz >> 1).  With two or three rows per lane the lane's upper rows are
+// eliminated first, as x_j = p_j - q_j x_0 - s_j x_0' of the lane's first row and
+// that of the lane above; one row per lane is left for parallel cyclic
+// reduction over the column's W lanes, and the others are substituted back.  With
+// W = 32 the exchanges across lanes 31 / 32 fetch the other column's finite
+// values, which meet exactly zero couplings.
 template <int R, int W>
 __device__ __forceinline__ void solve(const double (&L)[R], const double (&D)[R], const double (&U)[R],
                                       const double (&b)[R], float (&x)[R]) {
-    double Ld, Dd, Ud, rd, Lo = 0.0, Uo = 0.0, ro = 0.0;
-    if constexpr (R == 1) {
-        Ld = L[0];
-        Dd = D[0];
-        Ud = U[0];
-        rd = b[0];
-    } else {
-        static_assert(R == 2, "one or two rows per lane");
+    static_assert(R >= 1 && R <= 3, "one to three rows per lane");
+    double Ld = L[0], Dd = D[0], Ud = U[0], rd = b[0];
+    double p1 = 0.0, q1 = 0.0, s1 = 0.0, p2 = 0.0, q2 = 0.0, s2 = 0.0;
+    if constexpr (R >= 2) {
         const double i = ca_drcp(D[1]);
-        Lo = L[1] * i;
-        Uo = U[1] * i;
-        ro = b[1] * i;
-        const double Lp = pcr::up1(Lo), Up = pcr::up1(Uo), rp = pcr::up1(ro);  // odd row of the lane below
-        Dd = D[0] - L[0] * Up - U[0] * Lo;
-        rd = b[0] - L[0] * rp - U[0] * ro;
-        Ld = -L[0] * Lp;
-        Ud = -U[0] * Uo;
+        if constexpr (R == 2) {
+            q1 = L[1] * i;
+            s1 = U[1] * i;
+            p1 = b[1] * i;
+        } else {
+            const double f = L[2] * i, j = ca_drcp(D[2] - f * U[1]);
+            q2 = -(f * L[1]) * j;
+            s2 = U[2] * j;
+            p2 = (b[2] - f * b[1]) * j;
+            q1 = (L[1] - U[1] * q2) * i;
+            s1 = -(U[1] * s2) * i;
+            p1 = (b[1] - U[1] * p2) * i;
+        }
+        // the last row of the lane below
+        const double qb = pcr::up1(R == 2 ? q1 : q2), sb = pcr::up1(R == 2 ? s1 : s2), pb = pcr::up1(R == 2 ? p1 : p2);
+        Dd = D[0] - L[0] * sb - U[0] * q1;
+        rd = b[0] - L[0] * pb - U[0] * p1;
+        Ld = -L[0] * qb;
+        Ud = -U[0] * s1;
     }
 #pragma unroll
     for (int s = 1; s < W; s <<= 1) {
@@ -148,7 +156,11 @@ __device__ __forceinline__ void solve(const double (&L)[R], const double (&D)[R]
     }
     const double xe = rd * ca_drcp(Dd);
     x[0] = (float)xe;
-    if constexpr (R == 2) x[1] = (float)(ro - Lo * xe - Uo * pcr::dn1(xe));
+    if constexpr (R >= 2) {
+        const double xn = pcr::dn1(xe);
+        x[1] = (float)(p1 - q1 * xe - s1 * xn);
+        if constexpr (R == 3) x[2] = (float)(p2 - q2 * xe - s2 * xn);
+    }
 }
 
 // correct_implicit_advection_tendency! (implicit_tendency.jl:322-339): the rho e_tot

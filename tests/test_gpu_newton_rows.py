@@ -36,7 +36,7 @@ def _step_vs_oracle(g, num, Y32, tuning=None, T_sfc_col=None):
     return field_errors(got, ref, g), ref
 
 
-@pytest.mark.parametrize("nlev", [3, 31, 32, 33, 63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("nlev", [3, 31, 32, 33, 63, 64, 65, 94, 95, 96, 97, 127, 128, 129])
 def test_sphere_step_at_the_edges_of_the_level_ranges(nlev):
     g = G.cubed_sphere(2, G.tanh_stretched_faces(nlev, 30000.0, 200.0), PAR.planet_radius, PAR.Omega)
     num = P.Numerics(dt=100.0)
