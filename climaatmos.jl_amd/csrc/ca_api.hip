@@ -574,8 +574,8 @@ void point_level_tables(DevGeom &g, int nl, const float *dlc, const float *dlf, 
 // 107 at 9; h_elem 22, 63 levels 50.9 at 6 against 48.3 at 13 and 53.6 at 5;
 // h_elem 16, 63 levels 31.0 at 7 against 29.6 at 6 and 34.2 at 3; h_elem 8, 30
 // levels 12.5 at 1 against 15.1 at 4; with vertical diffusion h_elem 13, 45
-// levels 29.2 at 4 against 33.3 at 2, h_elem 30, 50 levels 97.1 at 9 against
-// 106 at 7.
+// levels 27.7 at 3 against 29.4 at 2 and 32.7 at 8, h_elem 30, 50 levels 85.9 at
+// 9 against 92.8 at 4 and 99.4 at 3.
 int explicit_chunk(int64_t layer_waves, int nl, int waves_per_simd) {
     const double slots = 1024.0 * waves_per_simd;
     int best = 1;
@@ -820,9 +820,10 @@ ca_status create_impl(const ca_geometry *geom, const ca_params *par, const ca_co
     // levels all from 2 to 8 are within 1%.
     {
         const int64_t layer_waves = (nc + 63) / 64;
-        // wavefronts of k_explicit a SIMD holds: 3 with vertical diffusion (147
-        // VGPRs), 4 without (105, 124 with the final combination)
-        h->explicit_chunk = h->final_chunk = explicit_chunk(layer_waves, nl, n.vdiff && !n.idiff ? 3 : 4);
+        // wavefronts of k_explicit a SIMD holds: 4 (105 VGPRs, 121 with vertical
+        // diffusion); with the final combination 3 if it also diffuses (138)
+        h->explicit_chunk = explicit_chunk(layer_waves, nl, 4);
+        h->final_chunk = explicit_chunk(layer_waves, nl, n.vdiff && !n.idiff ? 3 : 4);
         // the hook kernels' sweeps: 4 levels measured best at h_elem 16, 63 levels
         // (17.6, 19.8 and 20.3 us per implicit tendency with 4, 2 and 8), fewer
         // while that leaves less than 4 wavefronts per SIMD

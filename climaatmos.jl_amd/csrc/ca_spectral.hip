@@ -64,7 +64,7 @@ struct ColState {
     float l4;                  // C3 of nabla^4 u (hyperdiffusion)
     float dr, d1, d2, de;      // partial centre tendencies
     float sd;                  // dry static energy (vertical diffusion)
-    float uc0, uc1, uc2;       // velocity in the diffusion basis
+    float uc0, uc1, uc2;       // velocity as the diffusion takes it (uc2: REV)
     float Kd;                  // eddy diffusivity K_h of the centre
     float rhoe;                // rho e_tot (the final combination's U_4 value)
 };
@@ -87,6 +87,10 @@ struct ColState {
 // flight it is compiled for 3 wavefronts per SIMD: 148 us at the same size
 // against 169 us for 4 (124 VGPRs) and 163 us for 4 without the level
 // prefetch.
+// VDIFF diffuses u_i / s: the Cartesian basis of the covariant components is
+// the same at every level of a column up to that factor, so the components
+// diffuse on their own.  121 VGPRs, 4 wavefronts per SIMD; through the three
+// Cartesian components (REV) 147 and 3: 105 -> 86 us at h_elem 30, 50 levels.
 // REV: see ca_dPhiref.
 template <bool SPH, bool HYPER, bool VDIFF, bool FIN, bool REV>
 __global__ void __launch_bounds__(256)
@@ -280,16 +284,16 @@ k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int c
             if (VDIFF) {
                 cur.sd = n.cp_d * (T - n.T_0) + g.Phic[k];
                 cur.Kd = ca_Kc(g, n, col, k, p, spd0);
-                if (sph) {
+                if (sph && REV) {
                     const float *B = g.basis;
                     float is = ca_rcp(s);
                     cur.uc0 = (u1 * B[0 * nc + col] + u2 * B[3 * nc + col]) * is;
                     cur.uc1 = (u1 * B[1 * nc + col] + u2 * B[4 * nc + col]) * is;
                     cur.uc2 = (u1 * B[2 * nc + col] + u2 * B[5 * nc + col]) * is;
                 } else {
-                    cur.uc0 = u1;
-                    cur.uc1 = u2;
-                    cur.uc2 = 0.0f;
+                    const float is = sph ? ca_rcp(s) : 1.0f;
+                    cur.uc0 = u1 * is;
+                    cur.uc1 = u2 * is;
                 }
             }
         }
@@ -330,7 +334,7 @@ k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int c
                     float fac = Jf * iJv * (-2.0f * rK) * 0.5f;
                     Fu0 = fac * (cur.uc0 - prev.uc0) * iJv;
                     Fu1 = fac * (cur.uc1 - prev.uc1) * iJv;
-                    Fu2 = fac * (cur.uc2 - prev.uc2) * iJv;
+                    if (REV) Fu2 = fac * (cur.uc2 - prev.uc2) * iJv;
                 }
             }
             if ((k >= k0 && k < k1) || (k == nl && k1 == nl)) {
@@ -355,15 +359,16 @@ k_explicit(DevGeom g, DevNum n, const float *Y, const float *L, float *Yt, int c
                 float s = g.sc[kk];
                 const float iJc = iJh * g.isJc[kk];
                 de -= (Fs - Fs_prev) * iJc;
-                float e0 = (Fu0 - Fu0_prev) * iJc, e1 = (Fu1 - Fu1_prev) * iJc, e2 = (Fu2 - Fu2_prev) * iJc;
+                float e0 = (Fu0 - Fu0_prev) * iJc, e1 = (Fu1 - Fu1_prev) * iJc;
                 float c1, c2;
-                if (sph) {
+                if (sph && REV) {
                     const float *B = g.basis;
+                    const float e2 = (Fu2 - Fu2_prev) * iJc;
                     c1 = s * (e0 * B[6 * nc + col] + e1 * B[7 * nc + col] + e2 * B[8 * nc + col]);
                     c2 = s * (e0 * B[9 * nc + col] + e1 * B[10 * nc + col] + e2 * B[11 * nc + col]);
                 } else {
-                    c1 = e0;
-                    c2 = e1;
+                    c1 = sph ? s * e0 : e0;
+                    c2 = sph ? s * e1 : e1;
                 }
                 const float irho = ca_rcp(prev.rho);
                 d1 -= c1 * irho;
