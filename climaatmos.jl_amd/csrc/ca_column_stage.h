@@ -16,7 +16,7 @@
 namespace cst {
 
 // value of the row below / above every row (row 0 / the last row receive some
-// lane's finite value; every use selects by the row index)
+// lane's value, maybe another column's: every use selects by the row index)
 template <int R, class T>
 __device__ __forceinline__ void prev(const T (&v)[R], T (&o)[R]) {
     const T e = pcr::up1(v[R - 1]);
@@ -108,9 +108,7 @@ __device__ __forceinline__ double temperature(const DevNum &n, double et, float 
 // dtg c / dz >> 1).  With two or three rows per lane the lane's upper rows are
 // eliminated first, as x_j = p_j - q_j x_0 - s_j x_0' of the lane's first row and
 // that of the lane above; one row per lane is left for parallel cyclic
-// reduction over the column's W lanes, and the others are substituted back.  With
-// W = 32 the exchanges across lanes 31 / 32 fetch the other column's finite
-// values, which meet exactly zero couplings.
+// reduction over the column's W lanes, and the others are substituted back.
 template <int R, int W>
 __device__ __forceinline__ void solve(const double (&L)[R], const double (&D)[R], const double (&U)[R],
                                       const double (&b)[R], float (&x)[R]) {
@@ -133,7 +131,8 @@ __device__ __forceinline__ void solve(const double (&L)[R], const double (&D)[R]
             p1 = (b[1] - U[1] * p2) * i;
         }
         // the last row of the lane below
-        const double qb = pcr::up1(R == 2 ? q1 : q2), sb = pcr::up1(R == 2 ? s1 : s2), pb = pcr::up1(R == 2 ? p1 : p2);
+        const double qb = pcr::below<W>(R == 2 ? q1 : q2), sb = pcr::below<W>(R == 2 ? s1 : s2);
+        const double pb = pcr::below<W>(R == 2 ? p1 : p2);
         Dd = D[0] - L[0] * sb - U[0] * q1;
         rd = b[0] - L[0] * pb - U[0] * p1;
         Ld = -L[0] * qb;
@@ -144,9 +143,9 @@ __device__ __forceinline__ void solve(const double (&L)[R], const double (&D)[R]
         const double iD = ca_drcp(Dd);
         const double Ln = Ld * iD, Un = Ud * iD, rn = rd * iD;
         double La, Ua, ra, Lb, Ub, rb;
-        pcr::pcr_nbrs(Ln, s, La, Lb);
-        pcr::pcr_nbrs(Un, s, Ua, Ub);
-        pcr::pcr_nbrs(rn, s, ra, rb);
+        pcr::pcr_nbrs<W>(Ln, s, La, Lb);
+        pcr::pcr_nbrs<W>(Un, s, Ua, Ub);
+        pcr::pcr_nbrs<W>(rn, s, ra, rb);
         const double nD = Dd - Ld * Ua - Ud * Lb;
         const double nr = rd - Ld * ra - Ud * rb;
         Ld = -Ld * La;
@@ -157,7 +156,7 @@ __device__ __forceinline__ void solve(const double (&L)[R], const double (&D)[R]
     const double xe = rd * ca_drcp(Dd);
     x[0] = (float)xe;
     if constexpr (R >= 2) {
-        const double xn = pcr::dn1(xe);
+        const double xn = pcr::above<W>(xe);
         x[1] = (float)(p1 - q1 * xe - s1 * xn);
         if constexpr (R == 3) x[2] = (float)(p2 - q2 * xe - s2 * xn);
     }
@@ -344,14 +343,14 @@ __device__ __forceinline__ void tri32(const float (&L)[R], const float (&D)[R], 
         const float iD = rcp_nr(D[1]);
         Lo = L[1] * iD;
         Uo = U[1] * iD;
-        const float Lp = pcr::up1(Lo), Up = pcr::up1(Uo);
+        const float Lp = pcr::below<W>(Lo), Up = pcr::below<W>(Uo);
         Ds = D[0] - L[0] * Up - U[0] * Lo;
         Ls = -L[0] * Lp;
         Us = -U[0] * Uo;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             ro[i] = b[i][1] * iD;
-            r[i] = b[i][0] - L[0] * pcr::up1(ro[i]) - U[0] * ro[i];
+            r[i] = b[i][0] - L[0] * pcr::below<W>(ro[i]) - U[0] * ro[i];
         }
     }
 #pragma unroll
@@ -359,12 +358,12 @@ __device__ __forceinline__ void tri32(const float (&L)[R], const float (&D)[R], 
         const float iD = rcp_nr(Ds);
         const float Ln = Ls * iD, Un = Us * iD;
         float La, Ua, Lb, Ub;
-        pcr::pcr_nbrs(Ln, s, La, Lb);
-        pcr::pcr_nbrs(Un, s, Ua, Ub);
+        pcr::pcr_nbrs<W>(Ln, s, La, Lb);
+        pcr::pcr_nbrs<W>(Un, s, Ua, Ub);
 #pragma unroll
         for (int i = 0; i < N; ++i) {
             float ra, rb;
-            pcr::pcr_nbrs(r[i] * iD, s, ra, rb);
+            pcr::pcr_nbrs<W>(r[i] * iD, s, ra, rb);
             r[i] = r[i] - Ls * ra - Us * rb;
         }
         Ds = Ds - Ls * Ua - Us * Lb;
@@ -376,7 +375,7 @@ __device__ __forceinline__ void tri32(const float (&L)[R], const float (&D)[R], 
     for (int i = 0; i < N; ++i) {
         const float x = r[i] * iD;
         b[i][0] = x;
-        if constexpr (R == 2) b[i][1] = ro[i] - Lo * x - Uo * pcr::dn1(x);
+        if constexpr (R == 2) b[i][1] = ro[i] - Lo * x - Uo * pcr::above<W>(x);
     }
 }
 

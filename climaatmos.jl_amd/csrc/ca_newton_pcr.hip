@@ -66,25 +66,45 @@ __device__ __forceinline__ void swap32(float v, float &u, float &d) {
     d = __uint_as_float(r[1]);
 }
 
-// The rows k - s (u) and k + s (d) of a parallel-cyclic-reduction step, s a
-// power of two below 64 that is a constant once the step loop is unrolled.
-// s = 1: DPP wave shifts; s = 2: two of them; s = 32: one lane swap per
-// dword; otherwise LDS-crossbar permutes.  Out-of-range lanes receive some
-// lane's finite value (with s = 2 lane 1 receives lane 0's, not its own):
-// PCR multiplies every such value by an exactly zero coupling.
-template <class T>
+// The row S = 1 or 2 below / above across the lanes of a column that has W lanes,
+// as DPP wave shifts.  With W = 32 two columns share the wavefront, and an edge
+// lane, whose source would be the other column, receives 0: the rows' couplings
+// are exactly 0 there, but 0 times a value that is not finite is not 0.  (32
+// selects per solve of two columns: 0.0 to 0.4% of a step.)
+template <int W, int S = 1, class T>
+__device__ __forceinline__ T below(T v) {
+    const T e = S == 1 ? up1(v) : up1(up1(v));
+    if constexpr (W == 64) return e;
+    return (int)(threadIdx.x & (W - 1)) < S ? T(0) : e;
+}
+template <int W, int S = 1, class T>
+__device__ __forceinline__ T above(T v) {
+    const T e = S == 1 ? dn1(v) : dn1(dn1(v));
+    if constexpr (W == 64) return e;
+    return (int)(threadIdx.x & (W - 1)) >= W - S ? T(0) : e;
+}
+
+// The rows k - s (u) and k + s (d) of a parallel-cyclic-reduction step in a
+// column of W lanes, s a power of two below W that is a constant once the step
+// loop is unrolled.  s = 1: DPP wave shifts; s = 2: two of them; s = 32: one lane
+// swap per dword; otherwise LDS-crossbar permutes.  An out-of-range lane
+// receives 0 or some lane's value of its own column (with s = 2 and W = 64 lane
+// 1 receives lane 0's, not its own), never another column's: PCR multiplies
+// every such value by an exactly zero coupling, and a column that is not finite
+// leaves the other one as it is.
+template <int W = 64, class T>
 __device__ __forceinline__ void pcr_nbrs(T v, int s, T &u, T &d) {
     if (s == 1) {
-        u = up1(v);
-        d = dn1(v);
+        u = below<W>(v);
+        d = above<W>(v);
     } else if (s == 2) {
-        u = up1(up1(v));
-        d = dn1(dn1(v));
+        u = below<W, 2>(v);
+        d = above<W, 2>(v);
     } else if (s == 32) {
         swap32(v, u, d);
     } else {
-        u = up(v, s);
-        d = dn(v, s);
+        u = __shfl_up(v, s, W);
+        d = __shfl_down(v, s, W);
     }
 }
 
