@@ -160,43 +160,54 @@ __device__ __forceinline__ float ca_Tref(const DevNum &n, float Pi) { return n.T
 // 7 kex is 2 up to 7 kex_r (|7 kex_r| <= 7e-6, checked at create), so the last
 // factor is x (2 + x) + (1 + x)^2 7 kex_r log1p(x) to below 1e-9 of its size.
 // The neighbours of one element's level differ by a few per cent in pressure:
-// log1p and expm1 take short series for |x| <= 1/4 and a longer form otherwise,
-// chosen per wavefront (a NaN takes the longer form and stays one).  The library
+// log1p and expm1 take short series for |x| <= 1/4 and a reduced argument
+// otherwise.  The line is drawn per lane, so that a node's value does not depend
+// on what else its wavefront holds; a wavefront without a large difference skips
+// the longer form (a NaN takes it and stays one).  The library
 // functions they replace were a third of k_laplacians' VALU instructions
 // (327 -> 212 per level; 52 -> 42.5 us per launch at h_elem 30, 63 levels) and a fifth of k_explicit's, and both kernels are bound by VALU
 // issue (85% and 66% busy).
-__device__ __forceinline__ bool ca_small(float x) { return __all(fabsf(x) <= 0.25f); }
-// log1p(x).  Small: 2 atanh(s), s = x / (2 + x), by its odd series to s^9 (|s| <=
-// 1/7: truncated below 1e-9).  Otherwise log(u) + (x - (u - 1)) / u with u the
-// rounded 1 + x: |log(u)| > 0.2, where the hardware log2's error is one unit.
-__device__ __forceinline__ float ca_log1p(float x, bool small) {
-    if (small) {
-        const float s = x * ca_rcp(2.0f + x), s2 = s * s;
-        const float z = fmaf(s2, fmaf(s2, fmaf(s2, fmaf(s2, 1.0f / 9.0f, 1.0f / 7.0f), 0.2f), 1.0f / 3.0f), 1.0f);
-        return 2.0f * s * z;
-    }
+__device__ __forceinline__ bool ca_small(float x) { return fabsf(x) <= 0.25f; }
+// 2 atanh(s), s = x / (2 + x), by its odd series to s^9 (|s| <= 0.172: truncated
+// below 1e-9 of the value)
+__device__ __forceinline__ float ca_log1p_series(float x) {
+    const float s = x * ca_rcp(2.0f + x), s2 = s * s;
+    const float z = fmaf(s2, fmaf(s2, fmaf(s2, fmaf(s2, 1.0f / 9.0f, 1.0f / 7.0f), 0.2f), 1.0f / 3.0f), 1.0f);
+    return 2.0f * s * z;
+}
+// log1p(x).  Large: u = 1 + x = 2^e m with m in [0.7071, 1.4142], as e ln 2 +
+// log1p(m - 1) + (x - (u - 1)) / u, the last term the rounding of u; m - 1 is
+// exact.  u <= 0 is not a number.
+__device__ __forceinline__ float ca_log1p(float x) {
+    const bool small = ca_small(x);
+    if (__all(small)) return ca_log1p_series(x);
     const float u = 1.0f + x;
-    return fmaf(__builtin_amdgcn_logf(u), 0.693147182f, (x - (u - 1.0f)) * ca_rcp(u));
+    const int e = __builtin_amdgcn_frexp_expf(0.70710677f * u);
+    const float m1 = u > 0.0f ? ldexpf(u, -e) - 1.0f : __builtin_nanf("");
+    const float v = ca_log1p_series(small ? x : m1), fe = (float)e;
+    const float lo = fmaf(fe, -1.90465421e-9f, (x - (u - 1.0f)) * ca_rcp(u));
+    return small ? v : fmaf(fe, 0.693147182f, v + lo);
 }
 // expm1(r), r = kex log1p(x).  Small (|r| <= 0.083): Taylor to r^6, truncated below
-// 1e-10.  Otherwise (1 + t)^4 - 1 with t = expm1(r / 4) by Taylor to its eighth
-// power for |r| <= 1.4, and exp(r) - 1 beyond, where it loses no digits.
+// 1e-10.  Large: r = k ln 2 + q with |q| <= 0.347, Taylor to q^8 (below 1e-9), and
+// 2^k expm1(q) + (2^k - 1).
 __device__ __forceinline__ float ca_expm1(float r, bool small) {
-    if (small)
-        return r * fmaf(r, fmaf(r, fmaf(r, fmaf(r, fmaf(r, 1.0f / 720.0f, 1.0f / 120.0f), 1.0f / 24.0f), 1.0f / 6.0f),
-                                0.5f),
-                        1.0f);
-    const float q = 0.25f * r;
-    float t = 1.0f / 40320.0f;
-    t = fmaf(t, q, 1.0f / 5040.0f);
-    t = fmaf(t, q, 1.0f / 720.0f);
-    t = fmaf(t, q, 1.0f / 120.0f);
-    t = fmaf(t, q, 1.0f / 24.0f);
-    t = fmaf(t, q, 1.0f / 6.0f);
-    t = fmaf(t, q, 0.5f);
-    t = q * fmaf(t, q, 1.0f);
-    const float e = t * fmaf(t, fmaf(t, 4.0f + t, 6.0f), 4.0f);
-    return fabsf(r) <= 1.4f ? e : __builtin_amdgcn_exp2f(1.44269504f * r) - 1.0f;
+    const float t = r * fmaf(r, fmaf(r, fmaf(r, fmaf(r, fmaf(r, 1.0f / 720.0f, 1.0f / 120.0f), 1.0f / 24.0f), 1.0f / 6.0f),
+                                     0.5f),
+                             1.0f);
+    if (__all(small)) return t;
+    const float k = rintf(1.44269504f * r);
+    const float q = fmaf(k, 1.90465421e-9f, fmaf(k, -0.693147182f, r));
+    float p = 1.0f / 40320.0f;
+    p = fmaf(p, q, 1.0f / 5040.0f);
+    p = fmaf(p, q, 1.0f / 720.0f);
+    p = fmaf(p, q, 1.0f / 120.0f);
+    p = fmaf(p, q, 1.0f / 24.0f);
+    p = fmaf(p, q, 1.0f / 6.0f);
+    p = fmaf(p, q, 0.5f);
+    p = fmaf(q * q, p, q);
+    const float sc = ldexpf(1.0f, (int)k);
+    return small ? t : fmaf(sc, p, sc - 1.0f);
 }
 // (1 + x)^(7 kex) - 1, l = log1p(x)
 __device__ __forceinline__ float ca_pow2m1(const DevNum &n, float x, float l) {
@@ -217,7 +228,7 @@ __device__ __forceinline__ float ca_dPhiref(const DevNum &n, float pa, float ipa
         const float lr = n.kex * log1pf(x);
         return -n.cp_d * (n.Tmr * lr + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * expm1f(7.0f * lr));
     }
-    const float l = ca_log1p(x, ca_small(x));
+    const float l = ca_log1p(x);
     return -n.cp_d * (n.Tmr * (n.kex * l) + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * ca_pow2m1(n, x, l));
 }
 // the same and Pi_b - Pi_a = Pi_a expm1(kex log1p(x)); with REV,
@@ -234,9 +245,8 @@ __device__ __forceinline__ void ca_dref(const DevNum &n, float pa, float ipa, fl
         dPhr = -n.cp_d * (n.Tmr * lr + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * e7);
         return;
     }
-    const bool small = ca_small(x);
-    const float l = ca_log1p(x, small);
-    dPi = Pia * ca_expm1(n.kex * l, small);
+    const float l = ca_log1p(x);
+    dPi = Pia * ca_expm1(n.kex * l, ca_small(x));
     dPhr = -n.cp_d * (n.Tmr * (n.kex * l) + (n.Tsr - n.Tmr) * (1.0f / 7.0f) * ca_pow7(Pia) * ca_pow2m1(n, x, l));
 }
 
