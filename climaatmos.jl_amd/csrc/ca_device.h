@@ -169,11 +169,13 @@ __device__ __forceinline__ float ca_Tref(const DevNum &n, float Pi) { return n.T
 // issue (85% and 66% busy).
 __device__ __forceinline__ bool ca_small(float x) { return fabsf(x) <= 0.25f; }
 // 2 atanh(s), s = x / (2 + x), by its odd series to s^9 (|s| <= 0.172: truncated
-// below 1e-9 of the value)
+// below 1e-9 of the value).  As x - s (x - z), whose last subtraction is exact to
+// half a unit however s is rounded: 2.6e-8 relative (rms), as the library's log1pf;
+// 2 s (1 + ...) had 9.7e-8.
 __device__ __forceinline__ float ca_log1p_series(float x) {
     const float s = x * ca_rcp(2.0f + x), s2 = s * s;
-    const float z = fmaf(s2, fmaf(s2, fmaf(s2, fmaf(s2, 1.0f / 9.0f, 1.0f / 7.0f), 0.2f), 1.0f / 3.0f), 1.0f);
-    return 2.0f * s * z;
+    const float z = s2 * fmaf(s2, fmaf(s2, fmaf(s2, 2.0f / 9.0f, 2.0f / 7.0f), 0.4f), 2.0f / 3.0f);
+    return fmaf(-s, x - z, x);
 }
 // log1p(x).  Large: u = 1 + x = 2^e m with m in [0.7071, 1.4142], as e ln 2 +
 // log1p(m - 1) + (x - (u - 1)) / u, the last term the rounding of u; m - 1 is
@@ -192,9 +194,8 @@ __device__ __forceinline__ float ca_log1p(float x) {
 // 1e-10.  Large: r = k ln 2 + q with |q| <= 0.347, Taylor to q^8 (below 1e-9), and
 // 2^k expm1(q) + (2^k - 1).
 __device__ __forceinline__ float ca_expm1(float r, bool small) {
-    const float t = r * fmaf(r, fmaf(r, fmaf(r, fmaf(r, fmaf(r, 1.0f / 720.0f, 1.0f / 120.0f), 1.0f / 24.0f), 1.0f / 6.0f),
-                                     0.5f),
-                             1.0f);
+    const float t = fmaf(
+        r * r, fmaf(r, fmaf(r, fmaf(r, fmaf(r, 1.0f / 720.0f, 1.0f / 120.0f), 1.0f / 24.0f), 1.0f / 6.0f), 0.5f), r);
     if (__all(small)) return t;
     const float k = rintf(1.44269504f * r);
     const float q = fmaf(k, 1.90465421e-9f, fmaf(k, -0.693147182f, r));
