@@ -209,7 +209,7 @@ __global__ void __launch_bounds__(64) k_column_steps(DevGeom gr, ColumnSet cs, D
                 ve[r] = fmaf(dt, se, rhoe[r]);
                 vw[r] = t.intF[r] ? fmaf(dt, sw, u3[r]) : 0.0f;
             }
-            cst::newton<R, 64>(t, mt, n, nl, dtg, 1.0f / dtg, vr, v1, v2, ve, vw, fr, fe, fu);
+            cst::newton<R, 64, false>(t, mt, n, nl, dtg, 1.0f / dtg, vr, v1, v2, ve, vw, fr, fe, fu);
             float d1[R], d2[R], de[R], dw[R];
             cst::explicit_column<R>(t, e, mt, f, n, vr, v1, v2, ve, vw, d1, d2, de, dw);
 #pragma unroll

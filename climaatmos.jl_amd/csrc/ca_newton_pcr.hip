@@ -531,7 +531,7 @@ __global__ void __launch_bounds__(NT) k_newton_rows(DevGeom g, DevNum n, StageSr
                 rhoe[r] = tU[3][kc][c];
                 u3[r] = t.intF[r] ? tU[4][kc][c] : 0.0f;
             }
-            cst::newton<R, W>(t, m, n, nl, dtg, idtg, rho, u1, u2, rhoe, u3, fr, fe, fu);
+            cst::newton<R, W, true>(t, m, n, nl, dtg, idtg, rho, u1, u2, rhoe, u3, fr, fe, fu);
 #pragma unroll
             for (int r = 0; r < R; ++r)
                 if (t.hasC[r]) {
