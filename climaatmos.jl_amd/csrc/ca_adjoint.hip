@@ -4,7 +4,7 @@
 // No reference counterpart: the reference has forward-mode AD for its
 // Jacobians (src/prognostic_equations/implicit/autodiff_utils.jl) and
 // gradient-free calibration (calibration/).  Given the cotangent of the
-// state after nsteps steps, k_ensemble_adjoint returns the cotangent of the
+// state after nsteps steps, the k_ens_adj_* launches return the cotangent of the
 // initial state and of each member's vertical diffusivity D0 and Rayleigh
 // coefficient alpha_w, for the same step ca_ensemble_step takes:
 //
@@ -19,11 +19,10 @@
 //             Jacobian entries, which are taken in forward mode over the 11
 //             values a face row reads (dual numbers, float64).
 //
-// Forward states: where every step's stage states fit in memory they are kept
-// (k_ens_adj_forward / record / reverse).  Otherwise the forward pass stores the
-// state every `every` steps and the reverse pass recomputes each segment's step
-// states from its checkpoint and each step's stage states from its start state
-// (k_ensemble_adjoint).  Both run the same functions.  The non-smooth points
+// Forward states: the forward pass stores the state every `every` steps; the
+// reverse pass re-runs each segment from its checkpoint, keeping the start of
+// every step, and forms the stage states of as many of its steps as the scratch
+// holds before it reverses them.  The non-smooth points
 // (the T_min clamp, the van Leer limiter branches) take the derivative of the
 // branch the forward pass took.
 #include "ca_kernels.h"
@@ -224,7 +223,7 @@ struct AdjSharedT {
     double lam[NF];           // transposed Schur solution
     union {
         float W[24][NF];      // scratch of the local reverse passes
-        double red[2][128];   // block reduction of the parameter cotangents (LPM <= 128)
+        double red[2];        // block reduction of the parameter cotangents
     };
 };
 
@@ -999,6 +998,28 @@ __device__ void reverse_step(AdjSharedT<NF> &A, const DevGeom &g, const DevNum &
     sync();
 }
 
+// kb, ab summed over the workgroup, in lane 0 (fixed order: deterministic).  Called
+// after reverse_step, whose last barrier ends the use of A.W.
+template <int LPM, int NF>
+__device__ __forceinline__ void block_sum(AdjSharedT<NF> &A, double &kb, double &ab, int tid) {
+    for (int s = 32; s >= 1; s >>= 1) {
+        kb += __shfl_down(kb, s, 64);
+        ab += __shfl_down(ab, s, 64);
+    }
+    if constexpr (LPM > 64) {
+        if (tid == 64) {
+            A.red[0] = kb;
+            A.red[1] = ab;
+        }
+        sync();
+        if (tid == 0) {
+            kb += A.red[0];
+            ab += A.red[1];
+        }
+        sync();
+    }
+}
+
 // The level tables of one member in LDS: a step reads them in every phase, and
 // a phase between two barriers cannot hide a load from the L2 (128 members,
 // 16 steps: forward 435 -> 408 us, reverse 1107 -> 1041 us).
@@ -1069,198 +1090,123 @@ __device__ __forceinline__ void state_store(const SH &S, int nl, float *dst, int
 
 }  // namespace adj
 
-// Adjoint of nsteps ensemble steps: workgroup b reverses member order[b].
-// Y0: initial states; YbN: cotangents of the states after nsteps steps.
-// Outputs: Yb0 (cotangent of Y0), D0b and awb per member.  ckpt / seg:
-// scratch of (ceil(nsteps / every) + 1) and `every` ensemble states; member
-// m's part starts at that multiple of its state offset off[m] (the offsets
-// are the prefix sums of the member state sizes, so the parts are disjoint).
-template <int LPM, int NF>
-__global__ void __launch_bounds__(LPM) k_ensemble_adjoint(const DevGeom *__restrict__ mg, DevNum n,
-                                                          const int *__restrict__ order, const int64_t *__restrict__ off,
-                                                          const float *__restrict__ Y0, const float *__restrict__ YbN,
-                                                          float *__restrict__ Yb0, float *__restrict__ D0b,
-                                                          float *__restrict__ awb, float *__restrict__ ckpt,
-                                                          float *__restrict__ seg, EnsTab tab, float dt, int nsteps,
-                                                          int every) {
-    using namespace adj;
-    static_assert(LPM <= 128, "the adjoint runs at most 128 lanes per member");
-    __shared__ AdjSharedT<NF> A;
-    auto &S = A.S;
-    const int m = order[blockIdx.x];
-    const DevGeom &g = mg[m];
-    const int nl = g.nlev;
-    const int tid = threadIdx.x;
-    const int64_t Sm = 5 * (int64_t)nl + 1;
-    const int nseg = (nsteps + every - 1) / every;
-    float *ck = ckpt + (int64_t)(nseg + 1) * off[m];
-    float *sg = seg + (int64_t)every * off[m];
-    auto load = [&](const float *src) { state_load<LPM>(S, nl, src, tid); };
-    auto store = [&](float *dst) { state_store<LPM>(S, nl, dst, tid); };
-    // forward, storing a checkpoint every `every` steps
-    load(Y0 + off[m]);
-    store(ck);
-    for (int st = 0; st < nsteps; ++st) {
-        ens::step_once<LPM>(S, g, n, tab, dt, tid);
-        if ((st + 1) % every == 0 && st + 1 < nsteps) store(ck + ((st + 1) / every) * Sm);
-    }
-    // seed
-    const float *ybn = YbN + off[m];
-    for (int k = tid; k < nl; k += LPM)
-        for (int p = 0; p < 4; ++p) A.ub[p][k] = ybn[p * nl + k];
-    for (int f = tid; f <= nl; f += LPM) A.ub[4][f] = (f == 0 || f == nl) ? 0.0f : ybn[4 * nl + f];
-    sync();
-    double kb = 0.0, ab = 0.0;
-    for (int sgi = nseg - 1; sgi >= 0; --sgi) {
-        const int len = min(every, nsteps - sgi * every);
-        load(ck + sgi * Sm);
-        for (int j = 0; j < len; ++j) {
-            store(sg + j * Sm);
-            if (j + 1 < len) ens::step_once<LPM>(S, g, n, tab, dt, tid);
-        }
-        sync();
-        for (int j = len - 1; j >= 0; --j) {
-            load(sg + j * Sm);
-            ens::step_once<LPM>(S, g, n, tab, dt, tid, A.Ut, A.Us);
-            load(sg + j * Sm);
-            reverse_step<LPM>(A, g, n, tab, dt, tid, kb, ab);
-        }
-    }
-    float *yb0 = Yb0 + off[m];
-    for (int k = tid; k < nl; k += LPM)
-        for (int p = 0; p < 4; ++p) yb0[p * nl + k] = A.ub[p][k];
-    for (int f = tid; f <= nl; f += LPM) yb0[4 * nl + f] = A.ub[4][f];
-    // parameter cotangents: block sum (fixed order: deterministic)
-    A.red[0][tid] = kb;
-    A.red[1][tid] = ab;
-    sync();
-    if (tid == 0) {
-        double s0 = 0.0, s1 = 0.0;
-        for (int t = 0; t < LPM; ++t) {
-            s0 += A.red[0][t];
-            s1 += A.red[1][t];
-        }
-        D0b[m] = (float)s0;
-        awb[m] = (float)s1;
-    }
-}
+// The scratch of a run over some of the members: one ensemble state after the
+// other, `stride` floats apart, member m's part off[m] - off0 into each.
+struct AdjScratch {
+    int64_t off0, stride;
+};
 
-#define CA_ADJ_INST(LPM, NF)                                                                                   \
-    template __global__ void k_ensemble_adjoint<LPM, NF>(const DevGeom *, DevNum, const int *, const int64_t *,         \
-                                                         const float *, const float *, float *, float *, float *,     \
-                                                         float *, float *, EnsTab, float, int, int);
-CA_ADJ_INST(64, 33)
-CA_ADJ_INST(64, 65)
-CA_ADJ_INST(128, 65)
-CA_ADJ_INST(64, 129)
-CA_ADJ_INST(128, 129)
-#undef CA_ADJ_INST
-
-// The adjoint in three launches, for runs whose step and stage states are
-// kept: the forward steps (serial per member), the stage states of all steps
-// (a workgroup per member and step: every step starts from its kept state),
-// and the reverse (serial per member).  Member m's part of seg starts at
-// nsteps off[m], of rec at 6 nsteps off[m].
+// The adjoint is composed of three launches (ens_adjoint_run): forward steps
+// (serial per member), the stage states of several steps side by side (a
+// workgroup per member and step: every step starts from its kept state), and the
+// reverse of those steps (serial per member).  A step and its reverse are the
+// same code whatever the segments are, and what a later launch needs passes
+// through memory unrounded (float states and cotangents, float64 sums), so the
+// result does not depend on `every` or on the scratch.
 //
 // What bounds it is the serial chain: one step of one member after the other,
-// two wavefronts per member, most of whose time is waits between barriers.
-// k_ensemble_adjoint's chain is the forward, nearly as many steps again for the
-// segments' states, and one more per reversed step; here the chain is the
-// forward and the reverse, and the recorded steps run side by side.  128
-// members of 30 to 128 levels, 16 steps: 2628 us there, here 408 + 134 + 1041.
+// two wavefronts per member, most of whose time is waits between barriers.  As
+// one launch that also re-ran every step it reversed, 128 members of 30 to 128
+// levels took 2628 us for 16 steps; with all stage states kept 408 + 134 + 1041.
+
+// nsteps steps from src (an ensemble state, or scratch with src_off0 = off0); the
+// start of every `every`-th step into states, the last state into end (optional)
 template <int LPM, int NF>
 __global__ void __launch_bounds__(LPM) k_ens_adj_forward(const DevGeom *__restrict__ mg, DevNum n,
                                                          const int *__restrict__ order,
-                                                         const int64_t *__restrict__ off,
-                                                         const float *__restrict__ Y0, float *__restrict__ seg,
-                                                         EnsTab tab, float dt, int nsteps) {
+                                                         const int64_t *__restrict__ off, AdjScratch sc,
+                                                         const float *src, int64_t src_off0, float *states, int every,
+                                                         float *end, EnsTab tab, float dt, int nsteps) {
     __shared__ ens::SharedT<NF> S;
     __shared__ adj::LevelsLds<NF> L;
     const int m = order[blockIdx.x];
     const int tid = threadIdx.x;
     const DevGeom g = adj::stage_levels<LPM>(L, mg[m], tid);
     const int nl = g.nlev;
-    const int64_t Sm = 5 * (int64_t)nl + 1;
-    float *sg = seg + nsteps * off[m];
-    adj::state_load<LPM>(S, nl, Y0 + off[m], tid);
-    adj::state_store<LPM>(S, nl, sg, tid);
-    for (int st = 1; st < nsteps; ++st) {
-        ens::step_once<LPM>(S, g, n, tab, dt, tid);
-        adj::state_store<LPM>(S, nl, sg + st * Sm, tid);
+    const int64_t at = off[m] - sc.off0;
+    adj::state_load<LPM>(S, nl, src + (off[m] - src_off0), tid);
+    for (int st = 0; st < nsteps; ++st) {
+        if (st % every == 0) adj::state_store<LPM>(S, nl, states + (int64_t)(st / every) * sc.stride + at, tid);
+        if (st + 1 < nsteps || end) ens::step_once<LPM>(S, g, n, tab, dt, tid);
     }
+    if (end) adj::state_store<LPM>(S, nl, end + at, tid);
 }
 
+// stage states U~_1..3, U_1..3 of the step from states[blockIdx.y] into rec
 template <int LPM, int NF>
 __global__ void __launch_bounds__(LPM) k_ens_adj_record(const DevGeom *__restrict__ mg, DevNum n,
                                                         const int *__restrict__ order,
-                                                        const int64_t *__restrict__ off,
-                                                        const float *__restrict__ seg, float *__restrict__ rec,
-                                                        EnsTab tab, float dt, int nsteps) {
+                                                        const int64_t *__restrict__ off, AdjScratch sc,
+                                                        const float *states, float *rec, EnsTab tab, float dt) {
     __shared__ ens::SharedT<NF> S;
     __shared__ adj::LevelsLds<NF> L;
-    __shared__ float R[6][5][NF];  // U~_1..3, U_1..3
+    __shared__ float R[6][5][NF];
     const int m = order[blockIdx.x];
     const int tid = threadIdx.x;
     const DevGeom g = adj::stage_levels<LPM>(L, mg[m], tid);
     const int nl = g.nlev;
-    const int64_t Sm = 5 * (int64_t)nl + 1;
-    adj::state_load<LPM>(S, nl, seg + nsteps * off[m] + blockIdx.y * Sm, tid);
+    const int64_t at = off[m] - sc.off0;
+    adj::state_load<LPM>(S, nl, states + blockIdx.y * sc.stride + at, tid);
     ens::step_once<LPM>(S, g, n, tab, dt, tid, &R[0], &R[3]);
-    float *dst = rec + 6 * (nsteps * off[m] + blockIdx.y * Sm);
-    for (int s = 0; s < 6; ++s, dst += Sm) {
+    float *dst = rec + 6 * blockIdx.y * sc.stride + at;
+    for (int s = 0; s < 6; ++s, dst += sc.stride) {
         for (int k = tid; k < nl; k += LPM)
             for (int p = 0; p < 4; ++p) dst[p * nl + k] = R[s][p][k];
         for (int f = tid; f <= nl; f += LPM) dst[4 * nl + f] = R[s][4][f];
     }
 }
 
+// Reverses nsteps steps, the last first: the cotangent of the state after them
+// from yb_in, that of the state before them into yb_out (full ensemble states,
+// maybe the same one).  psum: per member the sums of the D0 and alpha_w
+// cotangents, carried from launch to launch; `first` starts them at 0, and with D0b
+// the launch is the last and writes them out.
 template <int LPM, int NF>
 __global__ void __launch_bounds__(LPM) k_ens_adj_reverse(const DevGeom *__restrict__ mg, DevNum n,
                                                          const int *__restrict__ order,
-                                                         const int64_t *__restrict__ off,
-                                                         const float *__restrict__ YbN, float *__restrict__ Yb0,
-                                                         float *__restrict__ D0b, float *__restrict__ awb,
-                                                         const float *__restrict__ seg,
-                                                         const float *__restrict__ rec, EnsTab tab, float dt,
-                                                         int nsteps) {
+                                                         const int64_t *__restrict__ off, AdjScratch sc,
+                                                         const float *states, const float *rec, const float *yb_in,
+                                                         float *yb_out, double *psum, int first, float *D0b,
+                                                         float *awb, EnsTab tab, float dt, int nsteps) {
     using namespace adj;
+    static_assert(LPM <= 128, "the adjoint runs at most 128 lanes per member");
     __shared__ AdjSharedT<NF> A;
     __shared__ LevelsLds<NF> L;
     const int m = order[blockIdx.x];
     const int tid = threadIdx.x;
     const DevGeom g = adj::stage_levels<LPM>(L, mg[m], tid);
     const int nl = g.nlev;
-    const int64_t Sm = 5 * (int64_t)nl + 1;
-    const float *ybn = YbN + off[m];
+    const int64_t at = off[m] - sc.off0;
+    const float *ybn = yb_in + off[m];
     for (int k = tid; k < nl; k += LPM)
         for (int p = 0; p < 4; ++p) A.ub[p][k] = ybn[p * nl + k];
     for (int f = tid; f <= nl; f += LPM) A.ub[4][f] = (f == 0 || f == nl) ? 0.0f : ybn[4 * nl + f];
-    double kb = 0.0, ab = 0.0;
+    double s0 = first ? 0.0 : psum[2 * m], s1 = first ? 0.0 : psum[2 * m + 1];
     for (int j = nsteps - 1; j >= 0; --j) {
-        const float *src = rec + 6 * (nsteps * off[m] + j * Sm);
-        for (int s = 0; s < 6; ++s, src += Sm) {
+        const float *src = rec + 6 * j * sc.stride + at;
+        for (int s = 0; s < 6; ++s, src += sc.stride) {
             float (*R)[NF] = s < 3 ? A.Ut[s] : A.Us[s - 3];
             for (int k = tid; k < nl; k += LPM)
                 for (int p = 0; p < 4; ++p) R[p][k] = src[p * nl + k];
             for (int f = tid; f <= nl; f += LPM) R[4][f] = src[4 * nl + f];
         }
-        state_load<LPM>(A.S, nl, seg + nsteps * off[m] + j * Sm, tid);
+        state_load<LPM>(A.S, nl, states + j * sc.stride + at, tid);
+        double kb = 0.0, ab = 0.0;
         reverse_step<LPM>(A, g, n, tab, dt, tid, kb, ab);
+        block_sum<LPM>(A, kb, ab, tid);
+        s0 += kb;
+        s1 += ab;
     }
-    float *yb0 = Yb0 + off[m];
+    float *yb0 = yb_out + off[m];
     for (int k = tid; k < nl; k += LPM)
         for (int p = 0; p < 4; ++p) yb0[p * nl + k] = A.ub[p][k];
     for (int f = tid; f <= nl; f += LPM) yb0[4 * nl + f] = A.ub[4][f];
-    A.red[0][tid] = kb;
-    A.red[1][tid] = ab;
-    sync();
     if (tid == 0) {
-        double s0 = 0.0, s1 = 0.0;
-        for (int t = 0; t < LPM; ++t) {
-            s0 += A.red[0][t];
-            s1 += A.red[1][t];
+        psum[2 * m] = s0;
+        psum[2 * m + 1] = s1;
+        if (D0b) {
+            D0b[m] = (float)s0;
+            awb[m] = (float)s1;
         }
-        D0b[m] = (float)s0;
-        awb[m] = (float)s1;
     }
 }

@@ -5,8 +5,10 @@
 
 #include "ca_kernels.h"
 
-// ca_ensemble_adjoint_noalloc's scratch: 16 Mi floats (64 MiB) per GPU
+// ca_ensemble_adjoint_noalloc's scratch: 16 Mi floats (64 MiB) per GPU, and the
+// five states more that one member of 128 levels at the limit needs
 #define CA_NOALLOC_SCRATCH_FLOATS (int64_t(1) << 24)
+#define CA_NOALLOC_EXTRA_FLOATS (5 * (5 * CA_ENS_MAXL + 1))
 #define CA_MAX_DEVICES 64
 
 struct ca_ensemble {
@@ -22,7 +24,7 @@ struct ca_ensemble {
     int *order[2] = {nullptr, nullptr};  // 0: as given, 1: longest first
     int64_t *doff = nullptr;
     int lanes = 64;           // the lanes knob: of the adjoint's workgroups
-    bool lanes_set = false;   // set by the caller; otherwise ens_adjoint_launch chooses
+    bool lanes_set = false;   // set by the caller; otherwise ens_adjoint_part chooses
     int order_kind = 1;
     int nf = CA_ENS_NF;  // LDS face rows per member: 33, 65 or 129, from the tallest member
     std::string err;
@@ -36,9 +38,11 @@ struct ca_ensemble {
     // per-member column constants (13 floats each) and their host copy
     float *cols = nullptr;
     std::vector<float> hcols;
-    // adjoint scratch: checkpoints and segment states
-    float *ckpt = nullptr, *segb = nullptr, *recb = nullptr;
-    int ck_nsteps = -1, ck_every = -1;
+    // adjoint scratch (ens_adjoint_run), its size, and the size last asked for; the
+    // members' parameter sums
+    float *adj = nullptr;
+    int64_t adj_floats = 0, adj_asked = 0;
+    double *psum = nullptr;
     // this device's copy of the file-scope scratch array (ca_ensemble_adjoint_noalloc)
     float *noalloc_scratch = nullptr;
 };
@@ -212,6 +216,7 @@ ca_status ens_create_impl(ca_ensemble *e, const ca_params *par, const ca_config 
     if ((s = eupload(e, &e->order[0], ord0))) return s;
     if ((s = eupload(e, &e->order[1], ord1))) return s;
     if ((s = eupload(e, &e->doff, e->off))) return s;
+    if ((s = eupload(e, &e->psum, std::vector<double>(2 * (size_t)M)))) return s;
     return CA_OK;
 }
 
@@ -220,7 +225,7 @@ ca_status ens_create_impl(ca_ensemble *e, const ca_params *par, const ca_config 
 // name to a kernel (on the host the name is a stand-in, not a device
 // address): ca_ensemble_create resolves this device's address once with
 // hipGetSymbolAddress and every use goes through that pointer.
-static __device__ __align__(256) float scratch[CA_NOALLOC_SCRATCH_FLOATS];
+static __device__ __align__(256) float scratch[CA_NOALLOC_SCRATCH_FLOATS + CA_NOALLOC_EXTRA_FLOATS];
 
 std::mutex g_scratch_mu;
 float *g_scratch_ptr[CA_MAX_DEVICES] = {};
@@ -242,18 +247,57 @@ ca_status resolve_noalloc_scratch(ca_ensemble *e) {
     return CA_OK;
 }
 
-// the reverse launch shared by ca_ensemble_adjoint and its no-allocation
-// variant: ck holds (ceil(nsteps / every) + 1) * S floats, sg every * S
-ca_status ens_adjoint_launch(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int nsteps, int every,
-                             float *Yb0, float *D0b, float *awb, float *ck, float *sg, hipStream_t st) {
-    const int *ord = e->order[e->order_kind];
-    const dim3 grid(e->M);
+// States of an adjoint run besides the stage records: a checkpoint per segment and
+// the start of each step of one segment (every <= nsteps)
+int64_t adj_states(int nsteps, int every) { return ((int64_t)nsteps + every - 1) / every + every; }
+constexpr int kStageStates = 6;  // U~_1..3, U_1..3 of one step
+
+// The adjoint of members ord[0 .. count), whose states hold `stride` floats from
+// off0 on.  ck, sg, rc: ceil(nsteps / every), every and 6 * rsteps such states.
+template <int LPM, int NF>
+void ens_adjoint_launch(ca_ensemble *e, const int *ord, int count, int64_t off0, int64_t stride, const float *Y0,
+                        const float *YbN, double dt, int nsteps, int every, float *Yb0, float *D0b, float *awb,
+                        float *ck, float *sg, float *rc, int rsteps, hipStream_t st) {
+    const AdjScratch sc{off0, stride};
+    const int nseg = (int)(((int64_t)nsteps + every - 1) / every);
+    const float fdt = (float)dt;
+    if (nseg > 1)
+        k_ens_adj_forward<LPM, NF><<<count, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sc, Y0, 0, ck, every,
+                                                          ck + (nseg - 1) * stride, e->tab, fdt, (nseg - 1) * every);
+    bool first = true;  // Yb0 may be YbN
+    for (int seg = nseg - 1; seg >= 0; --seg) {
+        const int len = std::min(every, nsteps - seg * every);
+        const float *src = nseg > 1 ? ck + seg * stride : Y0;
+        k_ens_adj_forward<LPM, NF><<<count, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sc, src, nseg > 1 ? off0 : 0, sg,
+                                                          1, nullptr, e->tab, fdt, len);
+        for (int hi = len; hi > 0; hi -= std::min(rsteps, hi)) {
+            const int nr = std::min(rsteps, hi);
+            const float *s0 = sg + (hi - nr) * stride;
+            k_ens_adj_record<LPM, NF><<<dim3(count, nr), LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sc, s0, rc, e->tab,
+                                                                      fdt);
+            const bool end = seg == 0 && hi == nr;
+            k_ens_adj_reverse<LPM, NF><<<count, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sc, s0, rc,
+                                                              first ? YbN : Yb0, Yb0, e->psum, first ? 1 : 0,
+                                                              end ? D0b : nullptr, awb, e->tab, fdt, nr);
+            first = false;
+        }
+    }
+}
+
+ca_status ens_adjoint_part(ca_ensemble *e, const int *ord, int count, int64_t off0, int64_t stride, const float *Y0,
+                           const float *YbN, double dt, int nsteps, int every, float *Yb0, float *D0b, float *awb,
+                           float *scratch, int64_t floats, hipStream_t st) {
+    const int64_t nst = adj_states(nsteps, every);
+    const int rsteps = (int)std::min<int64_t>({floats / stride - nst, (int64_t)65535 * kStageStates,
+                                               (int64_t)kStageStates * every}) /
+                       kStageStates;
+    float *ck = scratch, *sg = ck + (nst - every) * stride, *rc = scratch + nst * stride;
     // lanes: 64 for members of at most 32 levels; otherwise 128 unless the caller
     // asked for 64
     const bool l64 = e->lanes_set && e->lanes == 64;
-#define CA_ADJ_GO(LPM, NF)                                                                                       \
-    k_ensemble_adjoint<LPM, NF><<<grid, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, Y0, YbN, Yb0, D0b, awb, ck, sg, \
-                                                      e->tab, (float)dt, nsteps, every)
+#define CA_ADJ_GO(LPM, NF)                                                                                         \
+    ens_adjoint_launch<LPM, NF>(e, ord, count, off0, stride, Y0, YbN, dt, nsteps, every, Yb0, D0b, awb, ck, sg, rc, \
+                                rsteps, st)
     if (e->nf == 33) CA_ADJ_GO(64, 33);
     else if (e->nf == 65 && l64) CA_ADJ_GO(64, 65);
     else if (e->nf == 65) CA_ADJ_GO(128, 65);
@@ -264,29 +308,56 @@ ca_status ens_adjoint_launch(ca_ensemble *e, const float *Y0, const float *YbN, 
     return CA_OK;
 }
 
-// the same in three launches (k_ens_adj_*): sg holds nsteps * S floats, rc 6 nsteps * S
-ca_status ens_adjoint_split(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int nsteps, float *Yb0,
-                            float *D0b, float *awb, float *sg, float *rc, hipStream_t st) {
-    const int *ord = e->order[e->order_kind];
-    const dim3 grid(e->M);
-    const bool l64 = e->lanes_set && e->lanes == 64;
-#define CA_ADJ_GO(LPM, NF)                                                                                      \
-    do {                                                                                                        \
-        k_ens_adj_forward<LPM, NF><<<grid, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, Y0, sg, e->tab, (float)dt, \
-                                                         nsteps);                                               \
-        k_ens_adj_record<LPM, NF><<<dim3(e->M, nsteps), LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sg, rc, e->tab, \
-                                                                      (float)dt, nsteps);                       \
-        k_ens_adj_reverse<LPM, NF><<<grid, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, YbN, Yb0, D0b, awb, sg, rc, \
-                                                         e->tab, (float)dt, nsteps);                            \
-    } while (0)
-    if (e->nf == 33) CA_ADJ_GO(64, 33);
-    else if (e->nf == 65 && l64) CA_ADJ_GO(64, 65);
-    else if (e->nf == 65) CA_ADJ_GO(128, 65);
-    else if (l64) CA_ADJ_GO(64, 129);
-    else CA_ADJ_GO(128, 129);
-#undef CA_ADJ_GO
-    EHIPCHK(e, hipGetLastError());
+// The adjoint in `floats` floats of scratch: all members at once where one step's
+// stage records fit beside the states, otherwise as many members at a time (in
+// the order given) as do.  The scratch must hold one member's.
+ca_status ens_adjoint_run(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int nsteps, int every,
+                          float *Yb0, float *D0b, float *awb, float *scratch, int64_t floats, hipStream_t st) {
+    const int64_t need = adj_states(nsteps, every) + kStageStates;
+    if (need * e->S <= floats)
+        return ens_adjoint_part(e, e->order[e->order_kind], e->M, 0, e->S, Y0, YbN, dt, nsteps, every, Yb0, D0b, awb,
+                                scratch, floats, st);
+    for (int m0 = 0, m1; m0 < e->M; m0 = m1) {
+        int64_t size = 0;
+        for (m1 = m0; m1 < e->M; ++m1) {
+            const int64_t sm = 5 * (int64_t)e->nlev[m1] + 1;
+            if (need * (size + sm) > floats) break;
+            size += sm;
+        }
+        if (m1 == m0) return efail(e, CA_ERR_ARG, "ensemble adjoint: the scratch does not hold one member");
+        const ca_status s = ens_adjoint_part(e, e->order[0] + m0, m1 - m0, e->off[m0], size, Y0, YbN, dt, nsteps, every,
+                                             Yb0, D0b, awb, scratch, floats, st);
+        if (s != CA_OK) return s;
+    }
     return CA_OK;
+}
+
+// The handle's scratch: room for the records of a whole segment, of fewer steps
+// where they would take more than 1 GiB, and if that is not free what the
+// checkpoints and one segment's states take (and five states of one member)
+ca_status ens_adjoint_scratch(ca_ensemble *e, int nsteps, int every) {
+    const int64_t nst = adj_states(nsteps, every);
+    const int64_t fit = (int64_t{1} << 28) / (kStageStates * e->S);
+    const int64_t rsteps = std::min<int64_t>(every, std::max<int64_t>(1, fit));
+    const int64_t want = (nst + kStageStates * rsteps) * e->S;
+    const int64_t least = (nst + 1) * e->S + CA_NOALLOC_EXTRA_FLOATS;
+    if (e->adj_floats >= want || (e->adj_asked == want && e->adj_floats >= least)) return CA_OK;
+    if (e->adj) (void)hipFree(e->adj);
+    e->adj = nullptr;
+    e->adj_floats = e->adj_asked = 0;
+    for (const int64_t f : {want, (nst + kStageStates) * e->S, least}) {
+        if (f > want) continue;
+        const hipError_t err = hipMalloc(&e->adj, (size_t)f * sizeof(float));
+        if (err == hipSuccess) {
+            e->adj_floats = f;
+            e->adj_asked = want;
+            return CA_OK;
+        }
+        (void)hipGetLastError();
+        e->adj = nullptr;
+    }
+    return efail(e, CA_ERR_DEVICE, "ca_ensemble_adjoint: no memory for " + std::to_string((long long)least) +
+                                       " floats of scratch");
 }
 
 }  // namespace
@@ -326,8 +397,7 @@ ca_status ca_ensemble_create(const ca_params *params, const ca_config *config, i
 ca_status ca_ensemble_destroy(ca_ensemble *e) {
     if (!e) return CA_ERR_ARG;
     ens_drop_graph(e);
-    for (void *p : {(void *)e->ckpt, (void *)e->segb, (void *)e->recb})
-        if (p) (void)hipFree(p);
+    if (e->adj) (void)hipFree(e->adj);
     for (void *p : e->allocs) (void)hipFree(p);
     delete e;
     return CA_OK;
@@ -458,35 +528,10 @@ ca_status ca_ensemble_set_params(ca_ensemble *e, const double *alpha_w, const do
 ca_status ca_ensemble_adjoint(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int32_t nsteps,
                               int32_t every, float *Yb0, float *D0b, float *awb, void *stream) {
     if (!e || !Y0 || !YbN || !Yb0 || !D0b || !awb || nsteps < 1 || every < 1 || !(dt > 0)) return CA_ERR_ARG;
-    if (e->ck_nsteps != nsteps || e->ck_every != every) {
-        for (float **p : {&e->ckpt, &e->segb, &e->recb})
-            if (*p) {
-                (void)hipFree(*p);
-                *p = nullptr;
-            }
-        e->ck_nsteps = e->ck_every = -1;
-        // three launches over kept stage states where these take at most 1 GiB
-        // (and that is free); otherwise checkpoints and segments
-        const int64_t state = e->S * (int64_t)sizeof(float);
-        if (7 * nsteps * state <= (int64_t{1} << 30) && nsteps <= 65535) {
-            if (hipMalloc(&e->recb, (size_t)(6 * nsteps * state)) != hipSuccess ||
-                hipMalloc(&e->segb, (size_t)(nsteps * state)) != hipSuccess) {
-                (void)hipGetLastError();
-                if (e->recb) (void)hipFree(e->recb);
-                e->recb = e->segb = nullptr;
-            }
-        }
-        if (!e->recb) {
-            const int64_t nseg = (nsteps + every - 1) / every;
-            EHIPCHK(e, hipMalloc(&e->ckpt, (size_t)((nseg + 1) * state)));
-            EHIPCHK(e, hipMalloc(&e->segb, (size_t)(every * state)));
-        }
-        e->ck_nsteps = nsteps;
-        e->ck_every = every;
-    }
-    if (e->recb)
-        return ens_adjoint_split(e, Y0, YbN, dt, nsteps, Yb0, D0b, awb, e->segb, e->recb, (hipStream_t)stream);
-    return ens_adjoint_launch(e, Y0, YbN, dt, nsteps, every, Yb0, D0b, awb, e->ckpt, e->segb, (hipStream_t)stream);
+    every = std::min(every, nsteps);
+    const ca_status s = ens_adjoint_scratch(e, nsteps, every);
+    if (s != CA_OK) return s;
+    return ens_adjoint_run(e, Y0, YbN, dt, nsteps, every, Yb0, D0b, awb, e->adj, e->adj_floats, (hipStream_t)stream);
 }
 
 ca_status ca_ensemble_adjoint_noalloc(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int32_t nsteps,
@@ -494,7 +539,7 @@ ca_status ca_ensemble_adjoint_noalloc(ca_ensemble *e, const float *Y0, const flo
     if (!e || !Y0 || !YbN || !Yb0 || !D0b || !awb || nsteps < 1 || every < 1 || !(dt > 0)) return CA_ERR_ARG;
     if (!e->noalloc_scratch)
         return efail(e, CA_ERR_DEVICE, "ca_ensemble_adjoint_noalloc: the scratch array of this device is not resolved");
-    const int64_t nseg = (nsteps + every - 1) / every;
+    const int64_t nseg = ((int64_t)nsteps + every - 1) / every;
     const int64_t need = (nseg + 1 + every) * e->S;
     if (need > CA_NOALLOC_SCRATCH_FLOATS)
         return efail(e, CA_ERR_ARG,
@@ -502,9 +547,8 @@ ca_status ca_ensemble_adjoint_noalloc(ca_ensemble *e, const float *Y0, const flo
                          std::to_string(need) + " floats of scratch, above the maximum of " +
                          std::to_string((long long)CA_NOALLOC_SCRATCH_FLOATS) +
                          " (use ca_ensemble_adjoint, or change every)");
-    float *ck = e->noalloc_scratch;
-    float *sg = ck + (nseg + 1) * e->S;
-    return ens_adjoint_launch(e, Y0, YbN, dt, nsteps, every, Yb0, D0b, awb, ck, sg, (hipStream_t)stream);
+    return ens_adjoint_run(e, Y0, YbN, dt, nsteps, std::min(every, nsteps), Yb0, D0b, awb, e->noalloc_scratch,
+                           CA_NOALLOC_SCRATCH_FLOATS + CA_NOALLOC_EXTRA_FLOATS, (hipStream_t)stream);
 }
 
 }  // extern "C"

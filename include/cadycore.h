@@ -340,22 +340,25 @@ ca_status ca_ensemble_set_params(ca_ensemble *e, const double *alpha_w, const do
  * nsteps steps, writes the cotangent of Y0 to Yb0 (ragged, like Y0) and of
  * each member's D0 and alpha_w to D0b, awb (device arrays of nmembers).
  * Recomputes the forward trajectory itself, in scratch that the ensemble
- * keeps: 7 states per step, where that is at most 1 GiB and free, and
- * otherwise a checkpoint every `every` steps and the states of one such
- * segment.  Runs with 64 lanes per member when every member has at most 32
- * levels or CA_ENS_LANES was set to 64, else 128. */
+ * keeps (the largest so far): a checkpoint every `every` steps, the states of
+ * one such segment, and their stage records, 6 states per step, of a whole
+ * segment or of as many steps as take 1 GiB; where that is not free, of fewer
+ * steps or of some of the members at a time.  The result depends on neither
+ * `every` nor the scratch, to the bit.  Runs with 64 lanes per member when every
+ * member has at most 32 levels or CA_ENS_LANES was set to 64, else 128. */
 ca_status ca_ensemble_adjoint(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int32_t nsteps,
                               int32_t every, float *Yb0, float *D0b, float *awb, void *stream);
 /* ca_ensemble_adjoint without any device allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under
  * hipGraph capture, tight serving loops, harnesses that forbid hipMalloc).
- * The checkpoints and segment states live in a file-scope device array of
- * 2^24 floats (64 MiB) per GPU, held from the library's first use on that GPU
- * until the process ends; it needs (ceil(nsteps / every) + 1 + every) *
- * ca_ensemble_state_size(e) floats, and a larger request returns CA_ERR_ARG
+ * Checkpoints, segment states and stage records live in a file-scope device
+ * array of 2^24 floats (64 MiB) per GPU, held from the library's first use on
+ * that GPU until the process ends; it takes requests of up to (ceil(nsteps /
+ * every) + 1 + every) * ca_ensemble_state_size(e) = 2^24 floats, near that
+ * some of the members at a time, and a larger request returns CA_ERR_ARG
  * before any launch.  Every call on one GPU shares that array: calls that
  * overlap on one GPU (on different streams, or from different ensembles or
- * threads) race.  Same results as ca_ensemble_adjoint. */
+ * threads) race.  Bitwise the results of ca_ensemble_adjoint. */
 ca_status ca_ensemble_adjoint_noalloc(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int32_t nsteps,
                                       int32_t every, float *Yb0, float *D0b, float *awb, void *stream);
 
