@@ -2,8 +2,10 @@
 native reverse mode:
 
 * ``EnsembleSolve``: column ensembles, ``Y_N = step^nsteps(Y_0; D0, alpha_w)``
-  (``ca_ensemble_adjoint``: checkpointing every ``every`` steps, transposed
-  Schur solve, reverse ARS343 stage sweep);
+  (forward ``ca_ensemble_step_record`` on a tape with a checkpoint every
+  ``every`` steps, backward ``ca_ensemble_pullback``: transposed Schur solve,
+  reverse ARS343 stage sweep; the value and the gradient belong to the same
+  trajectory, ``ca_ensemble_step``'s up to float32 rounding);
 * ``StepSolve``: the sphere, ``Y_N = step^nsteps(Y_0; D0)`` (forward
   ``ca_step_record`` keeps checkpoints, backward ``ca_step_pullback``).
 
@@ -45,16 +47,22 @@ class EnsembleSolve:
                     ens.set_params(alpha_w=alpha_w.detach().cpu().double().numpy(),
                                    D0=D0.detach().cpu().double().numpy())
                     Y = Y0.detach().clone().contiguous()
-                    ens.step(Y, dt, nsteps)
-                    ctx.save_for_backward(Y0.detach().clone())
+                    # what has no pullback (no steps, no spacing) still steps; its backward raises
+                    ctx.recorded = nsteps >= 1 and every >= 1
+                    if ctx.recorded:
+                        ctx.save_for_backward(ens.step_record(Y, dt, nsteps, every))
+                    else:
+                        ens.step(Y, dt, nsteps)
+                        ctx.save_for_backward(Y0.detach().clone())
                     ctx.ens, ctx.dt, ctx.nsteps, ctx.every = ens, dt, nsteps, every
                     ctx.pdtype = (D0.dtype, D0.device, alpha_w.dtype, alpha_w.device)
                     return Y
 
                 @staticmethod
                 def backward(ctx, Ybar):
-                    (Y0,) = ctx.saved_tensors
-                    Yb0, D0b, awb = ctx.ens.adjoint(Y0, Ybar.contiguous().float(), ctx.dt, ctx.nsteps, ctx.every)
+                    (tape,) = ctx.saved_tensors
+                    pull = ctx.ens.pullback if ctx.recorded else ctx.ens.adjoint
+                    Yb0, D0b, awb = pull(tape, Ybar.contiguous().float(), ctx.dt, ctx.nsteps, ctx.every)
                     dd, ddev, ad, adev = ctx.pdtype
                     return Yb0, D0b.to(dtype=dd, device=ddev), awb.to(dtype=ad, device=adev), None, None, None, None
 

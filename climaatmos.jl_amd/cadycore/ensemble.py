@@ -195,6 +195,35 @@ class ColumnEnsemble:
                        self._stream()), fn.__name__)
         return Yb0, D0b, awb
 
+    def step_record(self, Y, dt, nsteps, every=8):
+        """``nsteps`` steps of Y in place, on the trajectory that the reverse mode
+        linearises (``step``'s up to float32 rounding); returns the tape that
+        ``pullback`` takes (a device tensor of ``ca_ensemble_tape_size``
+        floats)."""
+        t = self.torch
+        n = int(self.lib.ca_ensemble_tape_size(self.h, int(nsteps), int(every)))
+        tape = t.empty(n, dtype=t.float32, device=self.device)
+        self._check(self.lib.ca_ensemble_step_record(self.h, self._ptr(Y), float(dt), int(nsteps), int(every),
+                                                     C.c_void_p(tape.data_ptr()), self._stream()),
+                    "ca_ensemble_step_record")
+        return tape
+
+    def pullback(self, tape, YbN, dt, nsteps, every=8):
+        """``adjoint`` from the tape of a ``step_record`` of the same ``dt``,
+        ``nsteps`` and ``every``."""
+        t = self.torch
+        n = int(self.lib.ca_ensemble_tape_size(self.h, int(nsteps), int(every)))
+        assert tape.is_cuda and tape.dtype == t.float32 and tape.is_contiguous() and tape.numel() == n
+        Yb0 = t.empty_like(YbN)
+        M = len(self.members)
+        D0b = t.empty(M, dtype=t.float32, device=self.device)
+        awb = t.empty(M, dtype=t.float32, device=self.device)
+        self._check(self.lib.ca_ensemble_pullback(self.h, C.c_void_p(tape.data_ptr()), self._ptr(YbN), float(dt),
+                                                  int(nsteps), int(every), self._ptr(Yb0),
+                                                  C.c_void_p(D0b.data_ptr()), C.c_void_p(awb.data_ptr()),
+                                                  self._stream()), "ca_ensemble_pullback")
+        return Yb0, D0b, awb
+
     def autotune(self, Y, dt, nsteps):
         """Times every schedule on a copy of Y and keeps the fastest; returns
         {(lanes, order): ms}."""

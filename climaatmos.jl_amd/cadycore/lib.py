@@ -83,7 +83,7 @@ EXPORTED = (
     "ca_ensemble_create", "ca_ensemble_destroy", "ca_ensemble_state_size", "ca_ensemble_member_offset",
     "ca_ensemble_last_error", "ca_ensemble_step", "ca_ensemble_step_graph", "ca_ensemble_set_tuning",
     "ca_ensemble_get_tuning", "ca_ensemble_autotune", "ca_ensemble_set_params", "ca_ensemble_adjoint",
-    "ca_ensemble_adjoint_noalloc",
+    "ca_ensemble_adjoint_noalloc", "ca_ensemble_tape_size", "ca_ensemble_step_record", "ca_ensemble_pullback",
     "ca_dss_vjp", "ca_remaining_tendency_vjp", "ca_step_adjoint", "ca_step_record", "ca_step_pullback",
     "ca_set_column_params", "ca_set_debug_poison",
     "ca_fieldvector_native", "ca_fieldvector_vijfh", "ca_set_precomputed_quantities_fv",
@@ -93,7 +93,7 @@ EXPORTED = (
 CA_TUNE_NEWTON, CA_TUNE_EXPLICIT_CHUNK, CA_TUNE_DSS_CHUNK, CA_TUNE_DSS_KIND, CA_TUNE_ADJ_CHUNK, CA_TUNE_LAP_CHUNK = 0, 1, 2, 3, 4, 5
 CA_ENS_LANES, CA_ENS_ORDER = 0, 1
 _NOT_STATUS = ("ca_state_size", "ca_last_error", "ca_profile_count", "ca_ensemble_state_size",
-               "ca_ensemble_member_offset", "ca_ensemble_last_error")
+               "ca_ensemble_member_offset", "ca_ensemble_last_error", "ca_ensemble_tape_size")
 
 
 def load_library(path: str = LIB_PATH):
@@ -153,6 +153,10 @@ def load_library(path: str = LIB_PATH):
     lib.ca_ensemble_set_params.argtypes = [vp, dpp, dpp]
     lib.ca_ensemble_adjoint.argtypes = [vp, vp, vp, C.c_double, C.c_int32, C.c_int32, vp, vp, vp, vp]
     lib.ca_ensemble_adjoint_noalloc.argtypes = [vp, vp, vp, C.c_double, C.c_int32, C.c_int32, vp, vp, vp, vp]
+    lib.ca_ensemble_tape_size.restype = C.c_int64
+    lib.ca_ensemble_tape_size.argtypes = [vp, C.c_int32, C.c_int32]
+    lib.ca_ensemble_step_record.argtypes = [vp, vp, C.c_double, C.c_int32, C.c_int32, vp, vp]
+    lib.ca_ensemble_pullback.argtypes = [vp, vp, vp, C.c_double, C.c_int32, C.c_int32, vp, vp, vp, vp]
     lib.ca_dss_vjp.argtypes = [vp, vp, vp]
     lib.ca_remaining_tendency_vjp.argtypes = [vp, vp, vp, vp, vp, vp]
     lib.ca_step_adjoint.argtypes = [vp, vp, vp, C.c_double, C.c_int32, C.c_int32, vp, vp, vp]

@@ -19,10 +19,11 @@
 //             Jacobian entries, which are taken in forward mode over the 11
 //             values a face row reads (dual numbers, float64).
 //
-// Forward states: the forward pass stores the state every `every` steps; the
-// reverse pass re-runs each segment from its checkpoint, keeping the start of
-// every step, and forms the stage states of as many of its steps as the scratch
-// holds before it reverses them.  The non-smooth points
+// Forward states: the forward pass stores the state every `every` steps and the
+// start of every step of the last segment (the tape); the reverse pass re-runs the
+// other segments from their checkpoints, keeping the start of every step, and
+// forms the stage states of as many steps as the scratch holds before it
+// reverses them.  The non-smooth points
 // (the T_min clamp, the van Leer limiter branches) take the derivative of the
 // branch the forward pass took.
 #include "ca_kernels.h"
@@ -1096,8 +1097,8 @@ struct AdjScratch {
     int64_t off0, stride;
 };
 
-// The adjoint is composed of three launches (ens_adjoint_run): forward steps
-// (serial per member), the stage states of several steps side by side (a
+// The adjoint is composed of three launches (ens_record, ens_pullback): forward
+// steps (serial per member), the stage states of several steps side by side (a
 // workgroup per member and step: every step starts from its kept state), and the
 // reverse of those steps (serial per member).  A step and its reverse are the
 // same code whatever the segments are, and what a later launch needs passes
@@ -1109,27 +1110,32 @@ struct AdjScratch {
 // one launch that also re-ran every step it reversed, 128 members of 30 to 128
 // levels took 2628 us for 16 steps; with all stage states kept 408 + 134 + 1041.
 
-// nsteps steps from src (an ensemble state, or scratch with src_off0 = off0); the
-// start of every `every`-th step into states, the last state into end (optional)
+// nsteps steps from src (an ensemble state, or scratch with src_off0 = off0).  Kept
+// in states, one after the other: the start of every `every`-th step before step
+// `tail` and of each step from there on (tail: a multiple of `every`); the last
+// state goes into end (an ensemble state; may be src, or null).
 template <int LPM, int NF>
 __global__ void __launch_bounds__(LPM) k_ens_adj_forward(const DevGeom *__restrict__ mg, DevNum n,
                                                          const int *__restrict__ order,
                                                          const int64_t *__restrict__ off, AdjScratch sc,
                                                          const float *src, int64_t src_off0, float *states, int every,
-                                                         float *end, EnsTab tab, float dt, int nsteps) {
+                                                         int tail, float *end, EnsTab tab, float dt, int nsteps) {
     __shared__ ens::SharedT<NF> S;
     __shared__ adj::LevelsLds<NF> L;
     const int m = order[blockIdx.x];
     const int tid = threadIdx.x;
     const DevGeom g = adj::stage_levels<LPM>(L, mg[m], tid);
     const int nl = g.nlev;
-    const int64_t at = off[m] - sc.off0;
+    float *keep = states + (off[m] - sc.off0);
     adj::state_load<LPM>(S, nl, src + (off[m] - src_off0), tid);
     for (int st = 0; st < nsteps; ++st) {
-        if (st % every == 0) adj::state_store<LPM>(S, nl, states + (int64_t)(st / every) * sc.stride + at, tid);
+        if (st >= tail || st % every == 0) {
+            adj::state_store<LPM>(S, nl, keep, tid);
+            keep += sc.stride;
+        }
         if (st + 1 < nsteps || end) ens::step_once<LPM>(S, g, n, tab, dt, tid);
     }
-    if (end) adj::state_store<LPM>(S, nl, end + at, tid);
+    if (end) adj::state_store<LPM>(S, nl, end + off[m], tid);
 }
 
 // stage states U~_1..3, U_1..3 of the step from states[blockIdx.y] into rec

@@ -6,9 +6,9 @@
 #include "ca_kernels.h"
 
 // ca_ensemble_adjoint_noalloc's scratch: 16 Mi floats (64 MiB) per GPU, and the
-// five states more that one member of 128 levels at the limit needs
+// four states more that one member of 128 levels at the limit needs
 #define CA_NOALLOC_SCRATCH_FLOATS (int64_t(1) << 24)
-#define CA_NOALLOC_EXTRA_FLOATS (5 * (5 * CA_ENS_MAXL + 1))
+#define CA_NOALLOC_EXTRA_FLOATS (4 * (5 * CA_ENS_MAXL + 1))
 #define CA_MAX_DEVICES 64
 
 struct ca_ensemble {
@@ -24,7 +24,7 @@ struct ca_ensemble {
     int *order[2] = {nullptr, nullptr};  // 0: as given, 1: longest first
     int64_t *doff = nullptr;
     int lanes = 64;           // the lanes knob: of the adjoint's workgroups
-    bool lanes_set = false;   // set by the caller; otherwise ens_adjoint_part chooses
+    bool lanes_set = false;   // set by the caller; otherwise ens_lanes chooses
     int order_kind = 1;
     int nf = CA_ENS_NF;  // LDS face rows per member: 33, 65 or 129, from the tallest member
     std::string err;
@@ -38,8 +38,8 @@ struct ca_ensemble {
     // per-member column constants (13 floats each) and their host copy
     float *cols = nullptr;
     std::vector<float> hcols;
-    // adjoint scratch (ens_adjoint_run), its size, and the size last asked for; the
-    // members' parameter sums
+    // adjoint scratch, its size, and the size last asked for; the members' parameter
+    // sums
     float *adj = nullptr;
     int64_t adj_floats = 0, adj_asked = 0;
     double *psum = nullptr;
@@ -247,105 +247,134 @@ ca_status resolve_noalloc_scratch(ca_ensemble *e) {
     return CA_OK;
 }
 
-// States of an adjoint run besides the stage records: a checkpoint per segment and
-// the start of each step of one segment (every <= nsteps)
-int64_t adj_states(int nsteps, int every) { return ((int64_t)nsteps + every - 1) / every + every; }
+// The reverse mode of the ensemble's steps.  A run's tape is a checkpoint for every
+// segment of `every` steps but the last, and the start of each step of the last
+// one (1 <= every <= nsteps throughout).
+int64_t tape_states(int nsteps, int every) { return ((int64_t)nsteps + every - 1) / every - 1 + every; }
 constexpr int kStageStates = 6;  // U~_1..3, U_1..3 of one step
+// A spacing asks for the states of its tape and of the records of one segment.
+// Where these also hold the start of every step beside one step's records, no
+// segment is run again: that is the tape's spacing then (every = 8: up to 57
+// steps; 128 members of 30 to 128 levels, 16 steps, value and gradient 1980 ->
+// 1774 us).
+int64_t run_states(int nsteps, int every) { return tape_states(nsteps, every) + (int64_t)kStageStates * every; }
+int tape_spacing(int nsteps, int every) {
+    every = std::min(every, nsteps);
+    return nsteps + (int64_t)kStageStates <= run_states(nsteps, every) ? nsteps : every;
+}
 
-// The adjoint of members ord[0 .. count), whose states hold `stride` floats from
-// off0 on.  ck, sg, rc: ceil(nsteps / every), every and 6 * rsteps such states.
+// some of the members, ord[0 .. count), whose states hold `stride` floats from off0 on
+struct EnsPart {
+    const int *ord;
+    int count;
+    AdjScratch sc;
+};
+EnsPart all_members(const ca_ensemble *e) { return {e->order[e->order_kind], e->M, {0, e->S}}; }
+
+// lanes: 64 for members of at most 32 levels; otherwise 128 unless the caller
+// asked for 64
+#define CA_ENS_LANES_GO(GO)                        \
+    do {                                           \
+        const bool l64 = e->lanes_set && e->lanes == 64; \
+        if (e->nf == 33) GO(64, 33);               \
+        else if (e->nf == 65 && l64) GO(64, 65);   \
+        else if (e->nf == 65) GO(128, 65);         \
+        else if (l64) GO(64, 129);                 \
+        else GO(128, 129);                         \
+    } while (0)
+
+// nsteps steps of the members from src with the tape kept (src_off0, end: see the
+// kernel).  every >= nsteps keeps the start of every step.
+void ens_record(const ca_ensemble *e, const EnsPart &p, const float *src, int64_t src_off0, double dt, int nsteps,
+                int every, float *tape, float *end, hipStream_t st) {
+    const int tail = every < nsteps ? (nsteps - 1) / every * every : 0;
+#define CA_GO(LPM, NF)                                                                                          \
+    k_ens_adj_forward<LPM, NF><<<p.count, LPM, 0, st>>>(e->geoms, e->n, p.ord, e->doff, p.sc, src, src_off0, tape, every, \
+                                                        tail, end, e->tab, (float)dt, nsteps)
+    CA_ENS_LANES_GO(CA_GO);
+#undef CA_GO
+}
+
+// The pullback over a tape.  sg: room for the states of one segment (may be the
+// tape's tail, whose contents are used first); rc: for the stage records of rsteps
+// steps.
 template <int LPM, int NF>
-void ens_adjoint_launch(ca_ensemble *e, const int *ord, int count, int64_t off0, int64_t stride, const float *Y0,
-                        const float *YbN, double dt, int nsteps, int every, float *Yb0, float *D0b, float *awb,
-                        float *ck, float *sg, float *rc, int rsteps, hipStream_t st) {
-    const AdjScratch sc{off0, stride};
+void ens_pullback_launch(const ca_ensemble *e, const EnsPart &p, const float *tape, const float *YbN, double dt,
+                         int nsteps, int every, float *Yb0, float *D0b, float *awb, float *sg, float *rc, int rsteps,
+                         hipStream_t st) {
     const int nseg = (int)(((int64_t)nsteps + every - 1) / every);
+    const int64_t stride = p.sc.stride;
     const float fdt = (float)dt;
-    if (nseg > 1)
-        k_ens_adj_forward<LPM, NF><<<count, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sc, Y0, 0, ck, every,
-                                                          ck + (nseg - 1) * stride, e->tab, fdt, (nseg - 1) * every);
     bool first = true;  // Yb0 may be YbN
     for (int seg = nseg - 1; seg >= 0; --seg) {
         const int len = std::min(every, nsteps - seg * every);
-        const float *src = nseg > 1 ? ck + seg * stride : Y0;
-        k_ens_adj_forward<LPM, NF><<<count, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sc, src, nseg > 1 ? off0 : 0, sg,
-                                                          1, nullptr, e->tab, fdt, len);
+        const float *states = seg == nseg - 1 ? tape + seg * stride : sg;
+        if (seg < nseg - 1) ens_record(e, p, tape + seg * stride, p.sc.off0, dt, len, len, sg, nullptr, st);
         for (int hi = len; hi > 0; hi -= std::min(rsteps, hi)) {
             const int nr = std::min(rsteps, hi);
-            const float *s0 = sg + (hi - nr) * stride;
-            k_ens_adj_record<LPM, NF><<<dim3(count, nr), LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sc, s0, rc, e->tab,
-                                                                      fdt);
+            const float *s0 = states + (hi - nr) * stride;
+            k_ens_adj_record<LPM, NF><<<dim3(p.count, nr), LPM, 0, st>>>(e->geoms, e->n, p.ord, e->doff, p.sc, s0, rc,
+                                                                        e->tab, fdt);
             const bool end = seg == 0 && hi == nr;
-            k_ens_adj_reverse<LPM, NF><<<count, LPM, 0, st>>>(e->geoms, e->n, ord, e->doff, sc, s0, rc,
-                                                              first ? YbN : Yb0, Yb0, e->psum, first ? 1 : 0,
-                                                              end ? D0b : nullptr, awb, e->tab, fdt, nr);
+            k_ens_adj_reverse<LPM, NF><<<p.count, LPM, 0, st>>>(e->geoms, e->n, p.ord, e->doff, p.sc, s0, rc,
+                                                                first ? YbN : Yb0, Yb0, e->psum, first ? 1 : 0,
+                                                                end ? D0b : nullptr, awb, e->tab, fdt, nr);
             first = false;
         }
     }
 }
+// with the stage records in `floats` floats at rc (at least one step's)
+void ens_pullback(const ca_ensemble *e, const EnsPart &p, const float *tape, const float *YbN, double dt, int nsteps,
+                  int every, float *Yb0, float *D0b, float *awb, float *sg, float *rc, int64_t floats,
+                  hipStream_t st) {
+    const int rsteps = (int)std::min<int64_t>({floats / (kStageStates * p.sc.stride), 65535, every});
+#define CA_GO(LPM, NF) \
+    ens_pullback_launch<LPM, NF>(e, p, tape, YbN, dt, nsteps, every, Yb0, D0b, awb, sg, rc, rsteps, st)
+    CA_ENS_LANES_GO(CA_GO);
+#undef CA_GO
+}
 
-ca_status ens_adjoint_part(ca_ensemble *e, const int *ord, int count, int64_t off0, int64_t stride, const float *Y0,
-                           const float *YbN, double dt, int nsteps, int every, float *Yb0, float *D0b, float *awb,
-                           float *scratch, int64_t floats, hipStream_t st) {
-    const int64_t nst = adj_states(nsteps, every);
-    const int rsteps = (int)std::min<int64_t>({floats / stride - nst, (int64_t)65535 * kStageStates,
-                                               (int64_t)kStageStates * every}) /
-                       kStageStates;
-    float *ck = scratch, *sg = ck + (nst - every) * stride, *rc = scratch + nst * stride;
-    // lanes: 64 for members of at most 32 levels; otherwise 128 unless the caller
-    // asked for 64
-    const bool l64 = e->lanes_set && e->lanes == 64;
-#define CA_ADJ_GO(LPM, NF)                                                                                         \
-    ens_adjoint_launch<LPM, NF>(e, ord, count, off0, stride, Y0, YbN, dt, nsteps, every, Yb0, D0b, awb, ck, sg, rc, \
-                                rsteps, st)
-    if (e->nf == 33) CA_ADJ_GO(64, 33);
-    else if (e->nf == 65 && l64) CA_ADJ_GO(64, 65);
-    else if (e->nf == 65) CA_ADJ_GO(128, 65);
-    else if (l64) CA_ADJ_GO(64, 129);
-    else CA_ADJ_GO(128, 129);
-#undef CA_ADJ_GO
+// Tape, pullback and nothing kept, in `floats` floats of scratch: all members at
+// once where one step's stage records fit beside the tape, otherwise as many
+// members at a time (in the order given) as do.  The scratch must hold one
+// member's.
+ca_status ens_adjoint_run(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int nsteps, int every,
+                          float *Yb0, float *D0b, float *awb, float *scratch, int64_t floats, hipStream_t st) {
+    if ((nsteps + (int64_t)kStageStates) * e->S <= floats) every = nsteps;  // no segment run again
+    const int64_t nst = tape_states(nsteps, every), need = nst + kStageStates;
+    const bool all = need * e->S <= floats;
+    for (int m0 = 0, m1 = e->M; m0 < e->M; m0 = m1, m1 = e->M) {
+        EnsPart p = all_members(e);
+        if (!all) {
+            int64_t size = 0;
+            for (m1 = m0; m1 < e->M; ++m1) {
+                const int64_t sm = 5 * (int64_t)e->nlev[m1] + 1;
+                if (need * (size + sm) > floats) break;
+                size += sm;
+            }
+            if (m1 == m0) return efail(e, CA_ERR_ARG, "ensemble adjoint: the scratch does not hold one member");
+            p = {e->order[0] + m0, m1 - m0, {e->off[m0], size}};
+        }
+        float *tail = scratch + (nst - every) * p.sc.stride, *rc = scratch + nst * p.sc.stride;
+        ens_record(e, p, Y0, 0, dt, nsteps, every, scratch, nullptr, st);
+        ens_pullback(e, p, scratch, YbN, dt, nsteps, every, Yb0, D0b, awb, tail, rc, floats - nst * p.sc.stride, st);
+    }
     EHIPCHK(e, hipGetLastError());
     return CA_OK;
 }
 
-// The adjoint in `floats` floats of scratch: all members at once where one step's
-// stage records fit beside the states, otherwise as many members at a time (in
-// the order given) as do.  The scratch must hold one member's.
-ca_status ens_adjoint_run(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int nsteps, int every,
-                          float *Yb0, float *D0b, float *awb, float *scratch, int64_t floats, hipStream_t st) {
-    const int64_t need = adj_states(nsteps, every) + kStageStates;
-    if (need * e->S <= floats)
-        return ens_adjoint_part(e, e->order[e->order_kind], e->M, 0, e->S, Y0, YbN, dt, nsteps, every, Yb0, D0b, awb,
-                                scratch, floats, st);
-    for (int m0 = 0, m1; m0 < e->M; m0 = m1) {
-        int64_t size = 0;
-        for (m1 = m0; m1 < e->M; ++m1) {
-            const int64_t sm = 5 * (int64_t)e->nlev[m1] + 1;
-            if (need * (size + sm) > floats) break;
-            size += sm;
-        }
-        if (m1 == m0) return efail(e, CA_ERR_ARG, "ensemble adjoint: the scratch does not hold one member");
-        const ca_status s = ens_adjoint_part(e, e->order[0] + m0, m1 - m0, e->off[m0], size, Y0, YbN, dt, nsteps, every,
-                                             Yb0, D0b, awb, scratch, floats, st);
-        if (s != CA_OK) return s;
-    }
-    return CA_OK;
-}
-
-// The handle's scratch: room for the records of a whole segment, of fewer steps
-// where they would take more than 1 GiB, and if that is not free what the
-// checkpoints and one segment's states take (and five states of one member)
-ca_status ens_adjoint_scratch(ca_ensemble *e, int nsteps, int every) {
-    const int64_t nst = adj_states(nsteps, every);
+// The handle's scratch: `states` states and the records of rsteps steps, of fewer
+// where they would take more than 1 GiB or that is not free; at least `least`
+// floats
+ca_status ens_scratch(ca_ensemble *e, int64_t states, int64_t rsteps, int64_t least) {
     const int64_t fit = (int64_t{1} << 28) / (kStageStates * e->S);
-    const int64_t rsteps = std::min<int64_t>(every, std::max<int64_t>(1, fit));
-    const int64_t want = (nst + kStageStates * rsteps) * e->S;
-    const int64_t least = (nst + 1) * e->S + CA_NOALLOC_EXTRA_FLOATS;
+    rsteps = std::min<int64_t>(rsteps, std::max<int64_t>(1, fit));
+    const int64_t want = (states + kStageStates * rsteps) * e->S;
     if (e->adj_floats >= want || (e->adj_asked == want && e->adj_floats >= least)) return CA_OK;
     if (e->adj) (void)hipFree(e->adj);
     e->adj = nullptr;
     e->adj_floats = e->adj_asked = 0;
-    for (const int64_t f : {want, (nst + kStageStates) * e->S, least}) {
+    for (const int64_t f : {want, (states + kStageStates) * e->S, least}) {
         if (f > want) continue;
         const hipError_t err = hipMalloc(&e->adj, (size_t)f * sizeof(float));
         if (err == hipSuccess) {
@@ -356,7 +385,7 @@ ca_status ens_adjoint_scratch(ca_ensemble *e, int nsteps, int every) {
         (void)hipGetLastError();
         e->adj = nullptr;
     }
-    return efail(e, CA_ERR_DEVICE, "ca_ensemble_adjoint: no memory for " + std::to_string((long long)least) +
+    return efail(e, CA_ERR_DEVICE, "ensemble reverse mode: no memory for " + std::to_string((long long)least) +
                                        " floats of scratch");
 }
 
@@ -529,9 +558,39 @@ ca_status ca_ensemble_adjoint(ca_ensemble *e, const float *Y0, const float *YbN,
                               int32_t every, float *Yb0, float *D0b, float *awb, void *stream) {
     if (!e || !Y0 || !YbN || !Yb0 || !D0b || !awb || nsteps < 1 || every < 1 || !(dt > 0)) return CA_ERR_ARG;
     every = std::min(every, nsteps);
-    const ca_status s = ens_adjoint_scratch(e, nsteps, every);
+    // least: what the checkpoints and one segment's states take, and what one member
+    // needs beside them, which ens_adjoint_run can do with
+    const int64_t nst = tape_states(nsteps, every);
+    const ca_status s = ens_scratch(e, nst, every, (nst + 2) * e->S + CA_NOALLOC_EXTRA_FLOATS);
     if (s != CA_OK) return s;
     return ens_adjoint_run(e, Y0, YbN, dt, nsteps, every, Yb0, D0b, awb, e->adj, e->adj_floats, (hipStream_t)stream);
+}
+
+int64_t ca_ensemble_tape_size(const ca_ensemble *e, int32_t nsteps, int32_t every) {
+    if (!e || nsteps < 1 || every < 1) return 0;
+    return tape_states(nsteps, tape_spacing(nsteps, every)) * e->S;
+}
+
+ca_status ca_ensemble_step_record(ca_ensemble *e, float *Y, double dt, int32_t nsteps, int32_t every, float *tape,
+                                  void *stream) {
+    if (!e || !Y || !tape || nsteps < 1 || every < 1 || !(dt > 0)) return CA_ERR_ARG;
+    ens_record(e, all_members(e), Y, 0, dt, nsteps, tape_spacing(nsteps, every), tape, Y, (hipStream_t)stream);
+    EHIPCHK(e, hipGetLastError());
+    return CA_OK;
+}
+
+ca_status ca_ensemble_pullback(ca_ensemble *e, const float *tape, const float *YbN, double dt, int32_t nsteps,
+                               int32_t every, float *Yb0, float *D0b, float *awb, void *stream) {
+    if (!e || !tape || !YbN || !Yb0 || !D0b || !awb || nsteps < 1 || every < 1 || !(dt > 0)) return CA_ERR_ARG;
+    const int64_t total = run_states(nsteps, std::min(every, nsteps));
+    every = tape_spacing(nsteps, every);
+    const int64_t seg = every < nsteps ? every : 0;  // one segment's states besides the tape's
+    const ca_status s = ens_scratch(e, seg, (total - tape_states(nsteps, every)) / kStageStates, (seg + kStageStates) * e->S);
+    if (s != CA_OK) return s;
+    ens_pullback(e, all_members(e), tape, YbN, dt, nsteps, every, Yb0, D0b, awb, e->adj, e->adj + seg * e->S,
+                 e->adj_floats - seg * e->S, (hipStream_t)stream);
+    EHIPCHK(e, hipGetLastError());
+    return CA_OK;
 }
 
 ca_status ca_ensemble_adjoint_noalloc(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int32_t nsteps,

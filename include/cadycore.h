@@ -340,14 +340,32 @@ ca_status ca_ensemble_set_params(ca_ensemble *e, const double *alpha_w, const do
  * nsteps steps, writes the cotangent of Y0 to Yb0 (ragged, like Y0) and of
  * each member's D0 and alpha_w to D0b, awb (device arrays of nmembers).
  * Recomputes the forward trajectory itself, in scratch that the ensemble
- * keeps (the largest so far): a checkpoint every `every` steps, the states of
- * one such segment, and their stage records, 6 states per step, of a whole
- * segment or of as many steps as take 1 GiB; where that is not free, of fewer
- * steps or of some of the members at a time.  The result depends on neither
- * `every` nor the scratch, to the bit.  Runs with 64 lanes per member when every
- * member has at most 32 levels or CA_ENS_LANES was set to 64, else 128. */
+ * keeps (the largest so far): room for a checkpoint every `every` steps, the
+ * states of one such segment, and their stage records, 6 states per step, of a
+ * whole segment or of as many steps as take 1 GiB; where that is not free, of
+ * fewer steps or of some of the members at a time.  The result depends on neither
+ * `every` nor the scratch, to the bit.  The trajectory is ca_ensemble_step's up
+ * to float32 rounding (a last bit can decide a limiter branch); for a value and
+ * its gradient on one trajectory, see ca_ensemble_step_record.  Runs with 64
+ * lanes per member when every member has at most 32 levels or CA_ENS_LANES was
+ * set to 64, else 128. */
 ca_status ca_ensemble_adjoint(ca_ensemble *e, const float *Y0, const float *YbN, double dt, int32_t nsteps,
                               int32_t every, float *Yb0, float *D0b, float *awb, void *stream);
+/* The two halves of ca_ensemble_adjoint, for a caller that also wants the
+ * states.  ca_ensemble_step_record runs nsteps steps of Y in place, to the bit
+ * those that ca_ensemble_adjoint linearises (as ca_ensemble_step up to float32
+ * rounding), and writes what the pullback needs to tape, a device array of
+ * ca_ensemble_tape_size(e, nsteps, every) floats that the caller owns: ceil(nsteps
+ * / every) - 1 + every states, or nsteps where these and the records of a step
+ * fit ceil(nsteps / every) - 1 + 7 every (every <= nsteps).  ca_ensemble_pullback is
+ * ca_ensemble_adjoint from a tape, which it only reads; dt, nsteps, every and
+ * the ensemble's parameters must be the recorded run's.  It keeps scratch in
+ * the ensemble as ca_ensemble_adjoint does. */
+int64_t ca_ensemble_tape_size(const ca_ensemble *e, int32_t nsteps, int32_t every);
+ca_status ca_ensemble_step_record(ca_ensemble *e, float *Y, double dt, int32_t nsteps, int32_t every, float *tape,
+                                  void *stream);
+ca_status ca_ensemble_pullback(ca_ensemble *e, const float *tape, const float *YbN, double dt, int32_t nsteps,
+                               int32_t every, float *Yb0, float *D0b, float *awb, void *stream);
 /* ca_ensemble_adjoint without any device allocation.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under
  * hipGraph capture, tight serving loops, harnesses that forbid hipMalloc).

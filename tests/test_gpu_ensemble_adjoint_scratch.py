@@ -29,13 +29,13 @@ def _make(nlevs):
 
 
 @pytest.mark.parametrize("nlevs,nsteps", [([3], 1), ([32, 5, 17], 5), ([33, 64, 8], 7), ([128, 65, 30, 3], 9),
-                                          ([30] * 300, 2)], ids=lambda v: str(v)[:16])
+                                          ([30] * 300, 2), ([33, 64, 8], 40)], ids=lambda v: str(v)[:16])
 def test_gradient_does_not_depend_on_the_scratch(nlevs, nsteps):
     torch = _torch()
     e, Y0, w = _make(nlevs)
     ref = e.adjoint(Y0, w, 10.0, nsteps, nsteps)
     assert all(torch.isfinite(x).all() for x in ref)
-    for every in (1, 2, 4, nsteps + 5):
+    for every in (1, 2, 4, nsteps + 5):  # 40 steps with 2 or 4 run their segments again
         for noalloc in (False, True):
             got = e.adjoint(Y0, w, 10.0, nsteps, every, noalloc=noalloc)
             for name, a, b in zip(("Y0", "D0", "alpha_w"), ref, got):
@@ -45,11 +45,11 @@ def test_gradient_does_not_depend_on_the_scratch(nlevs, nsteps):
 
 @pytest.mark.parametrize("nsteps,every", [(1, 1), (2, 2), (2, 1)])
 def test_fixed_array_takes_the_members_in_parts(nsteps, every):
-    """4000 members of 128 levels: 3 or 4 states fit the array of 2^24 floats, the 8
-    to 9 that also hold one step's stage records do not."""
+    """4000 members of 128 levels: 3 or 4 states fit the array of 2^24 floats, the 7
+    to 8 that also hold one step's stage records do not."""
     torch = _torch()
     e, Y0, w = _make([128] * 4000)
-    assert 4 * e.S <= 1 << 24 < 8 * e.S
+    assert 4 * e.S <= 1 << 24 < 7 * e.S
     ref = e.adjoint(Y0, w, 10.0, nsteps, every)
     got = e.adjoint(Y0, w, 10.0, nsteps, every, noalloc=True)
     for name, a, b in zip(("Y0", "D0", "alpha_w"), ref, got):
@@ -58,8 +58,8 @@ def test_fixed_array_takes_the_members_in_parts(nsteps, every):
 
 
 def test_every_bounds_the_memory():
-    """512 steps with a checkpoint every 16: 32 checkpoints and the 7 states of 16
-    steps are 144 states, 7 states of every step would be 3584."""
+    """512 steps with a checkpoint every 16: 31 checkpoints and the 7 states of 16
+    steps are 143 states, 7 states of every step would be 3584."""
     torch = _torch()
     e, Y0, w = _make([128] * 64)
     e.adjoint(Y0, w, 10.0, 1, 1)  # the kernels are loaded
@@ -68,5 +68,5 @@ def test_every_bounds_the_memory():
     e.adjoint(Y0, w, 10.0, 512, 16)
     torch.cuda.synchronize()
     taken = free - torch.cuda.mem_get_info()[0]
-    assert taken <= 2 * 144 * 4 * e.S, taken  # twice: the allocators' granularity
+    assert taken <= 2 * 143 * 4 * e.S, taken  # twice: the allocators' granularity
     e.close()
