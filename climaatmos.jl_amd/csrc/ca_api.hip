@@ -132,6 +132,7 @@ template <class T>
 ca_status dalloc(ca_handle *h, T **p, size_t count) {
     void *q = nullptr;
     hipError_t e = hipMalloc(&q, count * sizeof(T) + 16);
+    if (e != hipSuccess) (void)hipGetLastError();  // reported here, not by the next launch
     if (e != hipSuccess) return fail(h, CA_ERR_DEVICE, std::string("hipMalloc: ") + hipGetErrorString(e));
     h->allocs.push_back(q);
     *p = (T *)q;

@@ -51,7 +51,9 @@ ca_status adj_ensure(ca_handle *h, int64_t rec_steps, int64_t nck) {
         if ((s = upload(h, &h->cgeo, v))) return s;
     }
     // the records and checkpoints grow with the call's `every` and step
-    // count; a larger request replaces the smaller buffer
+    // count; a larger request replaces the smaller buffer, and with it the
+    // recorded trajectory (also where the larger one is not to be had)
+    if (rec_steps > h->aw_rec_steps || nck > h->aw_ck_n) h->rec_valid = false;
     if (rec_steps > h->aw_rec_steps) {
         if ((s = dfree(h, h->aw_rec))) return s;
         h->aw_rec = nullptr;
