@@ -81,6 +81,7 @@ struct ca_handle {
     DevGeom gT{};                 // g with the transposed DSS tables
     DevGeom *cgeo = nullptr;      // per-column one-column views of g (Newton stage reverse)
     int adj_chunk = 8;            // levels per work item of k_explicit_vjp
+    int adj_chunk_min = 8;        // the smallest that the reverse-mode workspace takes
     float *aw_buf = nullptr;      // 13 S-sized cotangent / scratch planes
     float *aw_L = nullptr;        // 4 Laplacian-shaped planes: Lb, Lb2, fa | fb
     double *aw_d0 = nullptr;      // D0 cotangent partials [chunks x ncol]
@@ -833,6 +834,10 @@ ca_status create_impl(const ca_geometry *geom, const ca_params *par, const ca_co
         // 3.93 ms per gradient of 8 steps with chunks of 4 at h_elem 8, 30 levels,
         // 1.77 against 2.04 at h_elem 4, 16 levels (6 steps)
         h->adj_chunk = explicit_chunk(layer_waves, nl, 2);
+        // the workspace takes chunks from 8 levels (4 to 8 on small grids) on,
+        // whatever the model chose
+        const int64_t want = (1024 + layer_waves - 1) / layer_waves;
+        h->adj_chunk_min = (int)std::min<int64_t>({h->adj_chunk, 8, std::max<int64_t>(4, (nl + want - 1) / want)});
         h->lap_chunk = (int)std::min<int64_t>(4, (layer_waves * nl + 6999) / 7000);
         if (g.ncl > 0) {
             // 6 levels per workgroup measured best at h_elem 30, 63 levels (the
@@ -1415,9 +1420,9 @@ ca_status ca_set_tuning(ca_handle *h, int32_t knob, int32_t value) {
     }
     if (knob == CA_TUNE_ADJ_CHUNK) {
         if (value < 1 || value > h->g.nlev) return fail(h, CA_ERR_ARG, "adjoint chunk must be in [1, nlev]");
-        if (h->aw_d0 && value < h->adj_chunk)
+        if (h->aw_d0 && value < h->adj_chunk_min)
             return fail(h, CA_ERR_ARG, "adjoint chunk cannot shrink once the reverse-mode workspace exists");
-        h->adj_chunk = value;
+        h->adj_chunk = h->adj_chunk_min = value;
         return CA_OK;
     }
     return fail(h, CA_ERR_ARG, "unknown tuning knob");

@@ -24,7 +24,7 @@ ca_status adj_ensure(ca_handle *h, int64_t rec_steps, int64_t nck) {
         if ((s = dalloc(h, &h->aw_L, 16 * (size_t)g.nC))) return s;
         HIPCHK(h, hipMemset(h->aw_buf, 0xff, (size_t)AB_COUNT * h->S * sizeof(float)));
         HIPCHK(h, hipMemset(h->aw_L, 0xff, 16 * (size_t)g.nC * sizeof(float)));
-        const int nch = (int)cdiv(g.nlev, h->adj_chunk);
+        const int nch = (int)cdiv(g.nlev, h->adj_chunk_min);
         if ((s = dalloc(h, &h->aw_d0, (size_t)nch * g.ncol))) return s;
         // per-column one-column views of the geometry (the Newton stage reverse)
         std::vector<DevGeom> v(g.ncol);
