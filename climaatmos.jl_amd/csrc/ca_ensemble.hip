@@ -60,15 +60,6 @@ struct SharedT {
     };
 };
 
-// The part of SharedT one implicit stage uses (newton_stage alone)
-template <int NF>
-struct StageShared {
-    static constexpr int NFv = NF;
-    float fi[1][3][NF];
-    float U[5][NF];
-    NwT<NF> nw;
-};
-
 enum { EC_RHOJ, EC_KH, EC_KV, EC_U1, EC_U2, EC_RHO, EC_SD, EC_IRHOJ, EC_D1, EC_D2 };
 enum { NC_RHO, NC_K, NC_T, NC_P, NC_PI, NC_CT1, NC_CT2, NC_H, NC_J, NC_IJ, NC_RJ };
 

@@ -18,8 +18,6 @@ namespace pcr {
 
 template <class T>
 __device__ __forceinline__ T up(T v, int d) { return __shfl_up(v, d, 64); }
-template <class T>
-__device__ __forceinline__ T dn(T v, int d) { return __shfl_down(v, d, 64); }
 
 // Shifts by one lane across the whole wavefront as DPP wave shifts
 // (wave_shr:1, lane i <- lane i - 1; wave_shl:1, lane i <- lane i + 1) in the
@@ -114,7 +112,7 @@ __device__ __forceinline__ void pcr_nbrs(T v, int s, T &u, T &d) {
 
 // NF / NI: compile-time numbers of full-state and implicit-tendency sources
 // (the three ARS343 implicit stages have (2, 0), (3, 1), (4, 2)); -1 reads
-// the counts from src.
+// the counts from src (the recorded stage states of thread-per-column runs).
 template <int NF, int NI>
 __device__ __forceinline__ void assemble(const StageSrc &src, int64_t nC, int64_t q, bool okc, bool cen,
                                          bool face, float out[5]) {
@@ -161,20 +159,16 @@ __device__ __forceinline__ void ca_fma4(float a, const float4 &x, float4 &s) {
 template <int NF, int NI>
 __device__ __forceinline__ void assemble4(const StageSrc &src, int64_t nC, int64_t q, bool okc, bool cen,
                                           bool face, float4 out[5]) {
-    const int nf = NF >= 0 ? NF : src.nfull;
-    const int ni = NI >= 0 ? NI : src.nfi;
 #pragma unroll
     for (int comp = 0; comp < 4; ++comp) {
         float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (okc && cen) {
 #pragma unroll
-            for (int t = 0; t < (NF >= 0 ? NF : CA_MAX_SRC); ++t)
-                if (t < nf) ca_fma4(src.cf[t], ca_ld4(src.full[t] + comp * nC + q), s);
+            for (int t = 0; t < NF; ++t) ca_fma4(src.cf[t], ca_ld4(src.full[t] + comp * nC + q), s);
             if (comp == 0 || comp == 3) {
                 const int ci = comp == 0 ? 0 : 1;
 #pragma unroll
-                for (int t = 0; t < (NI >= 0 ? NI : CA_MAX_SRC); ++t)
-                    if (t < ni) ca_fma4(src.ci[t], ca_ld4(src.fi[t] + ci * nC + q), s);
+                for (int t = 0; t < NI; ++t) ca_fma4(src.ci[t], ca_ld4(src.fi[t] + ci * nC + q), s);
             }
         }
         out[comp] = s;
@@ -182,11 +176,9 @@ __device__ __forceinline__ void assemble4(const StageSrc &src, int64_t nC, int64
     float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if (okc && face) {
 #pragma unroll
-        for (int t = 0; t < (NF >= 0 ? NF : CA_MAX_SRC); ++t)
-            if (t < nf) ca_fma4(src.cf[t], ca_ld4(src.full[t] + 4 * nC + q), s);
+        for (int t = 0; t < NF; ++t) ca_fma4(src.cf[t], ca_ld4(src.full[t] + 4 * nC + q), s);
 #pragma unroll
-        for (int t = 0; t < (NI >= 0 ? NI : CA_MAX_SRC); ++t)
-            if (t < ni) ca_fma4(src.ci[t], ca_ld4(src.fi[t] + 2 * nC + q), s);
+        for (int t = 0; t < NI; ++t) ca_fma4(src.ci[t], ca_ld4(src.fi[t] + 2 * nC + q), s);
     }
     out[4] = s;
 }
