@@ -225,8 +225,9 @@ class ColumnEnsemble:
         return Yb0, D0b, awb
 
     def autotune(self, Y, dt, nsteps):
-        """Times every schedule on a copy of Y and keeps the fastest; returns
-        {(lanes, order): ms}."""
+        """Times both member orders on a copy of Y and keeps the faster; returns
+        {(lanes, order): ms} (the steps do not depend on the lanes: one time per
+        order, entered for each)."""
         t = (C.c_double * 6)()
         self._check(self.lib.ca_ensemble_autotune(self.h, self._ptr(Y), float(dt), int(nsteps), self._stream(), t),
                     "ca_ensemble_autotune")

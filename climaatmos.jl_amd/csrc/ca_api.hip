@@ -822,8 +822,8 @@ ca_status create_impl(const ca_geometry *geom, const ca_params *par, const ca_co
     // levels all from 2 to 8 are within 1%.
     {
         const int64_t layer_waves = (nc + 63) / 64;
-        // wavefronts of k_explicit a SIMD holds: 4 (105 VGPRs, 121 with vertical
-        // diffusion); with the final combination 3 if it also diffuses (138)
+        // wavefronts of k_explicit a SIMD holds: 4 (108 VGPRs, 124 with vertical
+        // diffusion, 127 with the final combination); 3 with both (141)
         h->explicit_chunk = explicit_chunk(layer_waves, nl, 4);
         h->final_chunk = explicit_chunk(layer_waves, nl, n.vdiff && !n.idiff ? 3 : 4);
         // the hook kernels' sweeps: 4 levels measured best at h_elem 16, 63 levels

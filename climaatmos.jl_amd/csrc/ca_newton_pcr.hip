@@ -446,14 +446,14 @@ CA_INST_PCR(4, 2, true)
 // Shapes (launch_newton_rows chooses):
 //   96 < nlev <= 128   R = 2, W = 64 (independent columns from 64 levels on)
 //   64 < nlev <= 96    R = 3, W = 32: of 64 lanes with two rows each a column of 90
-//       levels uses 45, of 32 lanes with three it uses 30; 189 VGPRs, 2
-//       wavefronts per SIMD, which R = 2, W = 64 has too (151 VGPRs, 64 KB of
+//       levels uses 45, of 32 lanes with three it uses 30; 192 VGPRs, 2
+//       wavefronts per SIMD, which R = 2, W = 64 has too (154 VGPRs, 64 KB of
 //       LDS).  75 us per stage at h_elem 16, 90 levels against 84 for R = 2, W =
 //       64 and 927 for the thread-per-column stage, whose 384 wavefronts walk
 //       their columns four times on 1024 SIMDs; 227 against 240 at h_elem 30, 66
 //       levels, 257 against 271 at 96
 //   32 < nlev <= 64    R = 2, W = 32: the tridiagonal solve of two columns costs
-//       one local elimination and five exchanges instead of twice six; 149
+//       one local elimination and five exchanges instead of twice six; 155
 //       VGPRs, 3 wavefronts per SIMD.  23.2 us at h_elem 10, 45 levels against
 //       25.6 for R = 1, W = 64 (28 for k_newton_pcr); 97.6 against 98.9 at
 //       h_elem 26, 45 levels

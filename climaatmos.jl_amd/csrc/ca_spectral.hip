@@ -78,18 +78,20 @@ struct ColState {
 // Level k + 1 (and the face above it) is loaded while level k is computed: the
 // kernel issues about 300 VALU instructions per level, and with the loads at
 // their use it waited 63% of its wavefront cycles, mostly for them.  The nine
-// values in flight fit 105 VGPRs, 4 wavefronts per SIMD.  At h_elem 30, 63
+// values in flight fit 108 VGPRs, 4 wavefronts per SIMD.  At h_elem 30, 63
 // levels: 96 us with them and chunks of 11; without, 111 us at 5 wavefronts per
 // SIMD and 120 us at 6 (80 VGPRs, a 36-byte spill).
 // FIN (the step's last explicit tendency, which also forms the final
 // combination) also loads three earlier tendencies at the top of each level so
-// that they arrive during the level's arithmetic.  With these 24 values in
-// flight it is compiled for 3 wavefronts per SIMD: 148 us at the same size
-// against 169 us for 4 (124 VGPRs) and 163 us for 4 without the level
-// prefetch.
+// that they arrive during the level's arithmetic: 24 values in flight, 127 VGPRs,
+// 4 wavefronts per SIMD, 148 us at the same size (163 us without the level
+// prefetch).  Its attribute asks for 3 wavefronts all the same: asked for 4, the
+// compiler reaches the same registers but moves the loads of the level tables (five
+// per centre and five per face, issued together otherwise) down to their uses,
+// where they are waited for one after the other: 168 us.
 // VDIFF diffuses u_i / s: the Cartesian basis of the covariant components is
 // the same at every level of a column up to that factor, so the components
-// diffuse on their own.  121 VGPRs, 4 wavefronts per SIMD; through the three
+// diffuse on their own.  124 VGPRs, 4 wavefronts per SIMD; through the three
 // Cartesian components (REV) 147 and 3: 105 -> 86 us at h_elem 30, 50 levels.
 // REV: see ca_dPhiref.
 template <bool SPH, bool HYPER, bool VDIFF, bool FIN, bool REV>

@@ -399,9 +399,10 @@ ca_status ca_remaining_tendency_vjp(ca_handle *h, float *Yb, const float *Ytb, c
  * supports nlev <= 128, no surface fluxes and explicit diffusion only, and
  * returns CA_ERR_ARG otherwise, before any launch.
  * ca_step that also keeps what its pullback needs: runs nsteps steps of Y in
- * place (as ca_step, up to float32 rounding) and stores the state at every `every`-th step in the
- * handle (ceil(nsteps / every) states; ca_step_pullback adds `every` steps of
- * stage records, 7 states + 4 Laplacian sets each).  every = 0 keeps the
+ * place (as ca_step, up to float32 rounding) and stores in the handle the state
+ * at every `every`-th step (ceil(nsteps / every) states) and the stage records
+ * of the last such segment, with room for `every` steps of 7 states + 4
+ * Laplacian sets each.  every = 0 keeps the
  * stage records of all nsteps steps instead (nsteps x (7 states + 4 Laplacian
  * sets) of device memory): the pullback then only reverses, with no
  * recomputation, and gives bitwise the same cotangents. */
@@ -409,9 +410,9 @@ ca_status ca_step_record(ca_handle *h, float *Y, double dt, int32_t nsteps, int3
 /* The pullback of the last ca_step_record: given the cotangent YbN of its
  * result, writes the cotangent of its input to Yb0 and, with vertical
  * diffusion and D0b != NULL, each column's D0 cotangent to D0b [ncol].  The
- * last checkpoint segment's stage states were kept by the forward where memory
- * allowed; each other segment is re-run once with its stage states recorded,
- * then reversed.  The column parameters must be those of the recorded run. */
+ * last checkpoint segment's stage states were kept by the forward; each other
+ * segment is re-run once with its stage states recorded, then reversed (and the
+ * last one too in a second pullback of a run of several segments).  The column parameters must be those of the recorded run. */
 ca_status ca_step_pullback(ca_handle *h, const float *YbN, float *Yb0, float *D0b, void *stream);
 /* ca_step_record on a copy of Y0 followed by ca_step_pullback (every as
  * there, 0 included).
