@@ -1108,7 +1108,7 @@ struct AdjScratch {
 // What bounds it is the serial chain: one step of one member after the other,
 // two wavefronts per member, most of whose time is waits between barriers.  As
 // one launch that also re-ran every step it reversed, 128 members of 30 to 128
-// levels took 2628 us for 16 steps; with all stage states kept 408 + 134 + 1041.
+// levels took 2628 us for 16 steps; here 421 + 168 + 1071, 6 steps' records at a time.
 
 // nsteps steps from src (an ensemble state, or scratch with src_off0 = off0).  Kept
 // in states, one after the other: the start of every `every`-th step before step
